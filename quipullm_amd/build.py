@@ -1,6 +1,6 @@
 """Builds the native parts in-tree (quipullm_amd/lib/):
 
-* quipu_kernels.hsaco -- the gfx950 kernels (hipcc --genco), loaded at run time with hipModuleLoad;
+* quipu_kernels.hsaco, quipu_small.hsaco -- the gfx950 kernels (hipcc --genco), loaded with hipModuleLoad;
 * libquipu.so         -- the C ABI of include/quipu.h (HIP runtime, op table);
 * quipu_napi.node     -- the Node.js (N-API) addon over libquipu.so, for the JavaScript host.
 
@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -22,6 +23,7 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 NODE_INC = "/usr/include/node"
 
 HSACO = os.path.join(LIB, "quipu_kernels.hsaco")
+HSACO2 = os.path.join(LIB, "quipu_small.hsaco")
 SO = os.path.join(LIB, "libquipu.so")
 NAPI = os.path.join(LIB, "quipu_napi.node")
 
@@ -56,10 +58,14 @@ TIMELINE_LIB = os.path.join(LIB, "timeline")
 
 
 def build_kernels(lib=LIB, defs=()):
-    src = os.path.join(CSRC, "kernels", "qp_kernels.hip")
-    out = os.path.join(lib, "quipu_kernels.hsaco")
-    _atomic(out, lambda o: _run([HIPCC, "--genco", *HIP_FLAGS, *defs, "-o", o, src], "kernels"))
-    return out
+    """The two code objects, compiled side by side."""
+    def one(name):
+        src = os.path.join(CSRC, "kernels", "qp_%s.hip" % name)
+        out = os.path.join(lib, "quipu_%s.hsaco" % name)
+        _atomic(out, lambda o: _run([HIPCC, "--genco", *HIP_FLAGS, *defs, "-o", o, src], name))
+        return out
+    with ThreadPoolExecutor(2) as ex:
+        return list(ex.map(one, ("kernels", "small")))
 
 
 def build_lib(lib=LIB, defs=()):
@@ -93,7 +99,7 @@ def build_timeline():
     """The profiling build of the kernels, library and addon into lib/timeline/ (not part of build_all)."""
     os.makedirs(TIMELINE_LIB, exist_ok=True)
     defs = ("-DQP_TIMELINE",)
-    out = [build_kernels(TIMELINE_LIB, defs), build_lib(TIMELINE_LIB, defs), build_napi(TIMELINE_LIB)]
+    out = build_kernels(TIMELINE_LIB, defs) + [build_lib(TIMELINE_LIB, defs), build_napi(TIMELINE_LIB)]
     return [o for o in out if o]
 
 
@@ -106,14 +112,14 @@ def build_all(oracle=True):
     os.makedirs(LIB, exist_ok=True)
     if not shutil.which(HIPCC) and not os.path.exists(HIPCC):
         raise RuntimeError("hipcc not found")
-    out = [build_kernels(), build_lib(), build_napi()]
+    out = build_kernels() + [build_lib(), build_napi()]
     if oracle:
         build_oracle()
     return [o for o in out if o]
 
 
 def built() -> bool:
-    return all(os.path.exists(p) for p in (HSACO, SO))
+    return all(os.path.exists(p) for p in (HSACO, HSACO2, SO))
 
 
 if __name__ == "__main__":

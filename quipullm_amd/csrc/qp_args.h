@@ -132,6 +132,17 @@ typedef struct {
     uint64_t part, cnt;
 } QpGemmArgs;
 
+// qp_sk_<fmt>: matmul of few token rows on integer weights (qp_small.hip).  xs: X as operands (qp_split_f16) of `rows`
+// rows (a multiple of 16).  kw: K slices per workgroup (1, 2 or 4).  Grid y: tpe slots (of each expert), each taking
+// every tpe-th block of 16 NT rows.  lst != 0: grouped by expert as in QpGemmArgs; xrows, yrows, nlst: rows of X's
+// operands and y and entries of lst that exist.  wrows: rows of the whole tensor.
+typedef struct {
+    uint64_t w, xs, y, paso, lst, off, wrows;
+    uint32_t n, k, acc, rows;
+    uint32_t kw, tpe, tfijo, pad;
+    uint32_t xrows, yrows, nlst, pad2;
+} QpSkArgs;
+
 // moe_group: lst[off[e] .. off[e + 1]) = the jobs i < T * n (in increasing order) with sel[i] == e, e < n_exp;
 // off[n_exp] = the number listed.  nsel: entries of sel and lst that exist.
 typedef struct {

@@ -32,7 +32,7 @@ bool g_init = false;
 std::atomic<int> g_lost{0};
 int g_device = 0;
 hipStream_t g_stream = nullptr;
-hipModule_t g_mod = nullptr;
+hipModule_t g_mod = nullptr, g_mod2 = nullptr;
 std::mutex g_mu;
 std::unordered_map<uint64_t, uint64_t> g_allocs;  // address -> bytes
 uint64_t g_bytes = 0;
@@ -77,14 +77,25 @@ int hip_fail(hipError_t e, const char* what) {
 // ------------------------------------------------------------------------------------------------ kernels
 enum Kid {
 #define K(name) K_##name,
+#define M(name) K_##name,
 #include "qp_kernel_list.inc"
 #undef K
+#undef M
     K_COUNT
 };
 const char* kNames[] = {
 #define K(name) "qp_" #name,
+#define M(name) "qp_" #name,
 #include "qp_kernel_list.inc"
 #undef K
+#undef M
+};
+const bool kSmall[] = {  // in the second code object (qp_small.hip)
+#define K(name) false,
+#define M(name) true,
+#include "qp_kernel_list.inc"
+#undef K
+#undef M
 };
 hipFunction_t g_fn[K_COUNT];
 
@@ -419,6 +430,7 @@ int workspace(uint64_t bytes, uint64_t* out) {
 struct SplitMemo {
     uint64_t x, xs, paso;
     uint32_t k, rows, mul, cap, gen;
+    bool ints;  // qp_split_f16's operands, not qp_split_bf16's planes
     bool valid;
 } g_split_memo = {};
 // While a graph is captured nothing runs, so a split recorded then proves nothing about the planes' contents now,
@@ -426,16 +438,68 @@ struct SplitMemo {
 // and graph launches invalidate it.
 // mul, cap: rows T * mul of x, at most cap (QpSplitArgs); 0: T rows.
 int split_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse,
-                uint32_t mul = 0, uint32_t cap = 0) {
+                uint32_t mul = 0, uint32_t cap = 0, bool ints = false) {
     const SplitMemo& m = g_split_memo;
     if (reuse && !g_capturing && m.valid && m.x == x && m.xs == xs && m.paso == paso && m.k == K && m.rows == rows &&
-        m.mul == mul && m.cap == cap && m.gen == g_ws_gen)
+        m.mul == mul && m.cap == cap && m.gen == g_ws_gen && m.ints == ints)
         return 0;
     QpSplitArgs sa = {x, xs, paso, K, rows, mul, cap};
-    g_split_memo = {x, xs, paso, K, rows, mul, cap, g_ws_gen, false};
-    if (int e = launch(K_split_bf16, grid_cap((uint64_t)tmax * K / 8), 1, 1, 256, 0, sa)) return e;
+    g_split_memo = {x, xs, paso, K, rows, mul, cap, g_ws_gen, ints, false};
+    if (int e = ints ? launch(K_split_f16, cdiv(K, 256), rows / 16, 1, 256, 0, sa)
+                     : launch(K_split_bf16, grid_cap((uint64_t)tmax * K / 8), 1, 1, 256, 0, sa))
+        return e;
     g_split_memo.valid = !g_capturing;
     return 0;
+}
+
+// ---- integer-weight matmul of few token rows (qp_small.hip): X as operands, 16 R weight rows per wavefront.
+// Bytes of the operands and scales of `rows` rows (a multiple of 16) of K inputs.
+uint64_t sk_bytes(uint32_t rows, uint32_t K) { return (uint64_t)(rows / 16) * cdiv(K, 256) * (17 * 1024 + 64); }
+
+Kid sk_kid(int fmt, uint32_t nt, uint32_t R) {
+#define SK_R1(F) {K_sk_##F##_t1r1, K_sk_##F##_t2r1, K_sk_##F##_t4r1}
+#define SK_R2(F) {K_sk_##F##_t1r2, K_sk_##F##_t2r2, K_sk_##F##_t4r2}
+    static const Kid r1[8][3] = {SK_R1(q4k), SK_R1(q5k), SK_R1(q6k), SK_R1(q3k),
+                                 SK_R1(q2k), SK_R1(q8), SK_R1(iq4nl), SK_R1(f32)};
+    static const Kid r2[5][3] = {SK_R2(q4k), SK_R2(q5k), SK_R2(q6k), SK_R2(q3k), SK_R2(q2k)};
+#undef SK_R1
+#undef SK_R2
+    const int t = nt == 1 ? 0 : nt == 2 ? 1 : 2;
+    if (is_kq(fmt)) return R == 2 ? r2[kq_index(fmt)][t] : r1[kq_index(fmt)][t];
+    if (fmt == QP_F32 && R == 2) return K_sk_f32_t4r2;
+    return r1[fmt == QP_Q8_0 ? 5 : fmt == QP_IQ4_NL ? 6 : 7][t];
+}
+
+// a: everything but the split of the work, in token blocks of 16 nt rows, tpe slots of them and E experts (dense: 1).
+int run_sk(int fmt, QpSkArgs& a, uint32_t nt, uint32_t tpe, uint32_t E, uint32_t R) {
+    const uint32_t nch = cdiv(a.k, 256), units = is_kq(fmt) ? cdiv(nch, 4) : nch;
+    a.kw = units >= 4 ? 4 : units >= 2 ? 2 : 1;
+    a.tpe = tpe;
+    const uint32_t gx = cdiv(a.n, 16 * R * (4 / a.kw));
+    const uint32_t lds = a.kw > 1 ? 4 * R * nt * 64 * 16 : 0;
+    return launch(sk_kid(fmt, nt, R), gx, tpe * E, 1, 256, lds, a);
+}
+
+// The dense matmuls that take this path (the others: the 128- and 256-token tiles of op_matmul_mt), by the tokens the
+// dispatch covers, measured with weights past the last-level cache, this path against the tiles in us:
+//   K-quants below 256 tokens: Q4_K 14336 x 4096 at 64 / 128 / 192 tokens 43 / 79 / 117 against 79 / 87 / 149, Q6_K
+//     4096 x 14336 66 / 100 / 180 against 105 / 119 / 173; at 256 tokens 144 against 129 (14336 x 4096);
+//   Q8_0 and IQ4_NL (whose sums are scaled every 32 inputs) up to 64 tokens, and below 256 where the product is small:
+//     Q8_0 11008 x 4096 at 64 / 128 tokens 59 / 103 against 66 / 73; 2816 x 1024 at 256 tokens 21 against 30;
+//   f32 always: 128 x 2048 (a router) at 64 / 2048 tokens 26 / 34 against 38 / 50, 4096 x 4096 49 / 689 against 71 / 738.
+// Below 64 tokens the other path is the vector-unit kernel (Q4_K 14336 x 4096 at 32 tokens 27 against 1120).
+bool sk_takes(int fmt, uint32_t tmax, uint32_t N, uint32_t K) {
+    if (fmt == QP_F32) return true;
+    if (is_kq(fmt)) return tmax < 256;
+    return tmax <= 64 || (tmax < 256 && (uint64_t)N * K * cdiv(tmax, 64) <= 12u << 20);
+}
+// 16-row tiles per wavefront: two where that leaves enough workgroups (X is read once per 16 R rows): 8192 rows times
+// 64-token blocks (Q4_K 14336 x 4096 at 32 tokens 27 against 36 us with one; 4096 x 4096 18.6 against 14.9).  Q8_0 and
+// IQ4_NL always one (2816 x 1024 at 256 tokens 21 against 25); f32 two from half of that on, in 64-token blocks.
+uint32_t sk_rows(int fmt, uint32_t nt, uint32_t yb, uint32_t N) {
+    if (planar(fmt)) return 1;
+    if (fmt == QP_F32) return nt == 4 && (uint64_t)N * yb >= 4096 ? 2 : 1;
+    return (uint64_t)N * yb >= 8192 ? 2 : 1;
 }
 
 int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z) {
@@ -460,6 +524,23 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
     if (xplanes && (!is_kq(fmt) || tmax < 256 || (g_capturing && !g_noalloc) || getenv_flag("QP_NO_MFMA")))
         return fail(QP_E_ARG, "%s: P[4] = 2 (x holds input planes) needs K-quant weights and a chunk of 256 tokens "
                               "or more on the matrix cores", name);
+    const uint32_t t1 = tmax ? tmax : 1;
+    if (!xplanes && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") && sk_takes(fmt, t1, N, K) &&
+        (!g_noalloc || sk_bytes(cdiv(t1, 16) * 16, K) <= QP_SCRATCH_BYTES)) {
+        QpSkArgs s = {};
+        s.w = a.w;
+        s.y = a.y;
+        s.paso = a.paso;
+        s.n = N;
+        s.k = K;
+        s.acc = acc;
+        s.wrows = N;
+        const uint32_t nt = t1 <= 16 ? 1 : t1 <= 32 ? 2 : 4, yb = cdiv(t1, 16 * nt);
+        s.rows = 16 * cdiv(t1, 16);
+        if (int e = workspace(sk_bytes(s.rows, K), &s.xs)) return e;
+        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, true)) return e;
+        return run_sk(fmt, s, nt, yb, 1, sk_rows(fmt, nt, yb, N));
+    }
     if (tmax >= 64 && !getenv_flag("QP_NO_MFMA")) {
         // matrix cores: 128 x 128 tiles (the kernel reads T from paso; tiles past it exit)
         const Kid k = fmt == QP_Q4_K ? K_gemm_mfma_q4k : fmt == QP_Q6_K ? K_gemm_mfma_q6k
@@ -1064,6 +1145,33 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
     // same planes: the sums are bit-equal).  P[5] = 1: the previous matmul split the same x (see split_input).  Not while capturing a graph or
     // under qp_dispatch_noalloc (the planes need the workspace): there x is split in the tiles as without P[4].
     const uint32_t m = c.U(4);
+    // Few jobs per expert: integer weights, 16 jobs per token tile (qp_small.hip).  Jobs per token: tfijo of the gate and
+    // up products, P[4] of the down product (8 where it says none).  128 experts of Q4_K 768 x 2048, 8 per token, the
+    // whole FFN in us against the 128-job tiles: 32 tokens 193 against 615, 512 983 against 1980, 1024 (64 jobs per
+    // expert) 2023 against 2118, 2048 4464 against 2371.
+    const uint32_t per_tok = tfijo > 1 ? tfijo : m ? m : 8;
+    if (!g_capturing && !g_noalloc && !getenv_flag("QP_NO_MFMA") && 32ull * tz * per_tok <= 64ull * E) {
+        // (without P[4]: every row of x that a job of y can read)
+        const uint64_t rows = m ? (uint64_t)32 * tz * m : ((uint64_t)a.yrows + tfijo - 1) / tfijo;
+        QpSkArgs s = {};
+        s.w = a.w;
+        s.y = a.y;
+        s.paso = a.paso;
+        s.lst = a.lst;
+        s.off = a.off;
+        s.n = N;
+        s.k = K;
+        s.acc = acc;
+        s.wrows = (uint64_t)E * N;
+        s.tfijo = tfijo;
+        s.yrows = a.yrows;
+        s.nlst = a.nlst;
+        s.xrows = (uint32_t)(rows < a.xrows ? rows : a.xrows);
+        s.rows = cdiv(s.xrows, 16) * 16;
+        if (int e = workspace(sk_bytes(s.rows, K), &s.xs)) return e;
+        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, s.rows, c.U(5) == 1, m ? m : s.xrows, s.xrows, true)) return e;
+        return run_sk(fmt, s, 1, a.tpe, E, is_kq(fmt) ? 2 : 1);
+    }
     if (m && !g_capturing && !g_noalloc) {
         if (K % 8) return fail(QP_E_ARG, "%s: input planes need K %% 8 == 0", name);
         const uint64_t r64 = (uint64_t)32 * tz * m;
@@ -1589,8 +1697,12 @@ int qp_init(int device) {
     if (const char* e = getenv("QP_KERNELS")) path = e;
     else path = self_dir() + "/quipu_kernels.hsaco";
     HIPCHK(hipModuleLoad(&g_mod, path.c_str()), ("hipModuleLoad " + path).c_str());
+    // the second code object lies beside the first
+    const size_t slash = path.rfind('/');
+    const std::string path2 = (slash == std::string::npos ? std::string() : path.substr(0, slash + 1)) + "quipu_small.hsaco";
+    HIPCHK(hipModuleLoad(&g_mod2, path2.c_str()), ("hipModuleLoad " + path2).c_str());
     for (int k = 0; k < K_COUNT; k++)
-        HIPCHK(hipModuleGetFunction(&g_fn[k], g_mod, kNames[k]), kNames[k]);
+        HIPCHK(hipModuleGetFunction(&g_fn[k], kSmall[k] ? g_mod2 : g_mod, kNames[k]), kNames[k]);
     g_device = device;
     g_init = true;
     return 0;

@@ -1,0 +1,116 @@
+"""The integer-weight matmuls of few token rows (qp_small.hip) against float64, at the edges of their tiles.
+
+Bound: the weights are exact and x keeps 22 bits below its largest magnitude per 256 inputs, so what is left is the
+rounding of float32 sums.  An output adds at most A = K / 16 + K / 64 terms in a row (two or three matrix instructions
+per 32 inputs, each adding to the running sum; one addition per 256 inputs and K slice), each rounding to 2^-24 of a
+partial sum of at most S = sum |x_k| (|scale * quant| + |minimum|); roundings of either sign make sqrt(A) of them count.
+The test allows 4 sqrt(A) 2^-24 S.  S is at most 3 sum |x_k| max |w| for these random blocks' rows (quants of the whole
+range, minima no larger than the largest product).
+"""
+import numpy as np
+import pytest
+
+from quipullm_amd import capi
+from test_gpu_ops import FMTS, PLANAR, dev, raw_matrix  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def weights(oracle, fmt, raw, N, K):
+    return (oracle.dequant(fmt, raw, N * K) if fmt != capi.F32 else raw.view(np.float32)).reshape(N, K).astype(np.float64)
+
+
+def bound(W, x):
+    K = W.shape[1]
+    return 4 * np.sqrt(K / 16 + K / 64) * 2.0 ** -24 * 3 * np.abs(x.astype(np.float64)).sum(1)[:, None] * np.abs(W).max(1)[None]
+
+
+def matmul(quipu, dev, fmt, raw, N, K, x, y0=None, t_op=True):
+    T = x.shape[0]
+    y = dev.buf(np.full((T + 2, N), 7.0, np.float32) if y0 is None else np.vstack([y0, np.full((2, N), 7.0, np.float32)]))
+    wb = [dev.matrix(fmt, raw, N, K)]
+    if fmt in PLANAR:
+        wb.append(capi.scale_plane(fmt, wb[0], N, K))
+    grid = ((N + 63) // 64, 1, (T + 31) // 32) if t_op else capi.dim2((N + 7) // 8) + ((T + 3) // 4,)
+    quipu.dispatch("matmul_%s_%s" % (capi.FMT_NAME[fmt], "t" if t_op else "4"),
+                   [("u", N), ("u", K), ("u", y0 is not None), ("u", 0)], [dev.paso(T, 0)] + wb + [dev.buf(x), y], grid)
+    out = dev.get(y, (T + 2, N))
+    assert np.all(out[T:] == 7.0)  # rows past T are not written
+    return out[:T]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("T,N,K", [(2, 1, 256), (15, 17, 768), (17, 200, 1280), (33, 33, 2048), (64, 130, 4352),
+                                   (65, 16, 1024), (130, 4100, 512), (255, 96, 5376)])
+def test_few_tokens(quipu, dev, oracle, fmt, T, N, K):
+    """Tile and block edges: one row, 16 and 16 + 1 rows, token tiles of 16, 32 and 64 with remainders, K of one block, of
+    part of a group of four, and of more groups than K slices."""
+    raw = raw_matrix(fmt, N, K, 71)
+    W = weights(oracle, fmt, raw, N, K)
+    rng = np.random.default_rng(72)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    y0 = rng.standard_normal((T, N)).astype(np.float32) if T % 2 else None
+    got = matmul(quipu, dev, fmt, raw, N, K, x, y0, t_op=T % 3 != 0)
+    want = x.astype(np.float64) @ W.T + (0 if y0 is None else y0)
+    assert np.all(np.abs(got - want) <= bound(W, x) + (0 if y0 is None else 2.0 ** -23 * np.abs(y0)))
+
+
+@pytest.mark.parametrize("fmt,K", [(capi.Q8_0, 32), (capi.Q8_0, 288), (capi.IQ4_NL, 96), (capi.IQ4_NL, 544),
+                                   (capi.F32, 16), (capi.F32, 272), (capi.F32, 1040)])
+def test_few_tokens_ragged_k(quipu, dev, oracle, fmt, K):
+    """K that is no multiple of 256: the last chunk's missing blocks are zeros on both sides."""
+    T, N = 19, 37
+    raw = raw_matrix(fmt, N, K, 73)
+    W = weights(oracle, fmt, raw, N, K)
+    x = np.random.default_rng(74).standard_normal((T, K)).astype(np.float32)
+    assert np.all(np.abs(matmul(quipu, dev, fmt, raw, N, K, x, t_op=False) - x.astype(np.float64) @ W.T) <= bound(W, x))
+
+
+@pytest.mark.parametrize("fmt", [capi.Q4_K, capi.Q6_K, capi.Q8_0, capi.F32])
+def test_few_tokens_magnitudes(quipu, dev, oracle, fmt):
+    """Rows of magnitude 1e-30 .. 1e30, a zero row, a row of denormals, an outlier, and rows with an infinity and a NaN,
+    which stay in their own rows."""
+    T, N, K = 40, 50, 1024
+    raw = raw_matrix(fmt, N, K, 75)
+    W = weights(oracle, fmt, raw, N, K)
+    rng = np.random.default_rng(76)
+    x = (rng.standard_normal((T, K)) * 10.0 ** rng.integers(-30, 31, size=T)[:, None]).astype(np.float32)
+    x[3] = 0.0
+    x[4] = (rng.standard_normal(K) * 1e-39).astype(np.float32)
+    x[5, 7] *= 1e6
+    x[6, 100] = np.inf
+    x[7, 300] = np.nan
+    got = matmul(quipu, dev, fmt, raw, N, K, x)
+    ok = [t for t in range(T) if t not in (6, 7)]
+    want = x[ok].astype(np.float64) @ W.T
+    assert np.all(got[3] == 0.0) and not np.isfinite(got[[6, 7]]).any()
+    assert np.all(np.abs(got[ok] - want) <= bound(W, x[ok]) + 1e-37)  # (sums below the smallest normal may be flushed)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_few_jobs_per_expert(quipu, dev, oracle, fmt):
+    """matmul_<fmt>_eg with few jobs per expert: experts without jobs, one with every token (more than a tile), gathered
+    input rows (tfijo = 3) and job rows; the two of them with and without P[4] give the same bits."""
+    E, N, K, k, T = 9, 70, 768, 3, 21
+    rng = np.random.default_rng(77)
+    sel = np.stack([np.concatenate([[4], rng.choice([0, 2, 7], 2, replace=False)]) for _ in range(T)]).astype(np.uint32).ravel()
+    raw = raw_matrix(fmt, E * N, K, 78)
+    W = weights(oracle, fmt, raw, E * N, K).reshape(E, N, K)
+    hw = dev.matrix(fmt, raw, E * N, K)
+    wb = [hw, capi.scale_plane(fmt, hw, E * N, K)] if fmt in PLANAR else [hw]
+    sb, lb, ob = dev.buf(sel), dev.zeros(4 * T * k), dev.zeros(4 * (E + 1))
+    p = dev.paso(T, 0)
+    quipu.dispatch("moe_group", [("u", E), ("u", k)], [p, sb, lb, ob])
+    for tfijo, m in ((k, 1), (1, k)):
+        x = rng.standard_normal((T * k // tfijo, K)).astype(np.float32)
+        xb, outs = dev.buf(x), []
+        for extra in ([("u", m), ("u", 0)], []):
+            y = dev.zeros(4 * T * k * N)
+            quipu.dispatch("matmul_%s_eg" % capi.FMT_NAME[fmt], [("u", N), ("u", K), ("u", 0), ("u", tfijo)] + extra,
+                           [p] + wb + [xb, y, lb, ob], ((N + 63) // 64, E, 1))
+            outs.append(dev.get(y, (T * k, N)))
+        assert np.array_equal(outs[0], outs[1])
+        for j in range(T * k):
+            e = sel[j]
+            xr = x[j // tfijo][None]
+            assert np.all(np.abs(outs[0][j] - (xr.astype(np.float64) @ W[e].T)[0]) <= bound(W[e], xr)[0]), j

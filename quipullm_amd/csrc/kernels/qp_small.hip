@@ -116,55 +116,59 @@ QP_DEV u32x4 sk_transpose(u32x4 v) {
 // The dword of lane `from` / 4.
 QP_DEV uint32_t sk_from(uint32_t v, uint32_t from) { return (uint32_t)__builtin_amdgcn_ds_bpermute((int)from, (int)v); }
 
-// Byte i of w, twice, as f16 times 2^-SH (SH = 0, 2, 4, 6 or -5) plus off * 2^-SH: the byte in the low mantissa bits
+// Two bytes of w as f16 times 2^-SH (-5 <= SH <= 6) plus off * 2^-SH: the byte in the low mantissa bits
 // of a power of two (1024 at SH = 0), which the addition takes away.
 template <int SH>
 QP_DEV h2 sk_dup(uint32_t w, uint32_t sel, float off = 0.0f) {
     constexpr uint32_t top = 0x64u - SH * 4;  // high byte of 2^(10 - SH)
-    const float c = off * (SH >= 0 ? 1.0f / (1 << (SH > 0 ? SH : 0)) : 32.0f) - (SH >= 0 ? 1024.0f / (1 << (SH > 0 ? SH : 0)) : 32768.0f);
+    constexpr float unit = SH >= 0 ? 1.0f / (1 << (SH > 0 ? SH : 0)) : (float)(1 << (SH < 0 ? -SH : 0));
+    const float c = (off - 1024.0f) * unit;
     const h2 o = {(_Float16)c, (_Float16)c};
     return as_h2(__builtin_amdgcn_perm(top * 0x01010101u, w, sel)) + o;
 }
 constexpr uint32_t sk_sel(int i, int j) { return 0x04000400u | (uint32_t)i | ((uint32_t)j << 16); }
 
 // The quants stay where they are in the low 10 bits of a half, which as f16 is a subnormal: value * 2^-24 times the
-// power of two of their position (exact; the scales take the position's power away, the block's f32 scale the 2^24).
+// power of two of their position (exact).  The scale they are multiplied by takes the position's power away and carries
+// 32 times the power of two SkK::UP, so that the products are normal f16: the matrix instructions take subnormal
+// operands, but align them as if their leading bit were set, and drop the low bits of the sum (Q2_K 4e-6 off instead of
+// 3e-7 at K = 1024).  The block's f32 scale takes all of it away.
 
 // ------------------------------------------------------------------ K-quants
 template <int FMT> struct SkK;
-template <> struct SkK<QP_Q4_K> { static constexpr int NC = 9, HDR = 0, RB = 144; static constexpr bool MIN = true, LO = false; };
-template <> struct SkK<QP_Q5_K> { static constexpr int NC = 11, HDR = 0, RB = 176; static constexpr bool MIN = true, LO = false; };
-template <> struct SkK<QP_Q6_K> { static constexpr int NC = 13, HDR = 12, RB = 208; static constexpr bool MIN = true, LO = true; };
-template <> struct SkK<QP_Q3_K> { static constexpr int NC = 7, HDR = 6, RB = 112; static constexpr bool MIN = false, LO = false; };
-template <> struct SkK<QP_Q2_K> { static constexpr int NC = 5, HDR = 0, RB = 80; static constexpr bool MIN = true, LO = false; };
+template <> struct SkK<QP_Q4_K> { static constexpr int NC = 9, HDR = 0, RB = 144, UP = 2; static constexpr bool MIN = true, LO = false; };
+template <> struct SkK<QP_Q5_K> { static constexpr int NC = 11, HDR = 0, RB = 176, UP = 2; static constexpr bool MIN = true, LO = false; };
+template <> struct SkK<QP_Q6_K> { static constexpr int NC = 13, HDR = 12, RB = 208, UP = 0; static constexpr bool MIN = true, LO = true; };
+template <> struct SkK<QP_Q3_K> { static constexpr int NC = 7, HDR = 6, RB = 112, UP = 2; static constexpr bool MIN = false, LO = false; };
+template <> struct SkK<QP_Q2_K> { static constexpr int NC = 5, HDR = 0, RB = 80, UP = 4; static constexpr bool MIN = true, LO = false; };
 
 // One block of one row, from the point of view of a lane: its dwords t[chunk] of the data chunks and the whole header.
-// The block is d * 2^24 * sum(step products) - dmin * sum(mins * sums of 16 inputs).
+// The block is d * 2^(19 - UP) * sum(step products) - dmin * sum(mins * sums of 16 inputs).
 template <int FMT>
 struct SkBlock {
     uint32_t t[SkK<FMT>::NC];
     uint32_t h[4];    // the header chunk
-    uint32_t sc[4];   // scales: Q4_K/Q5_K 6 bits of sub-blocks 0..7 in sc[0..1], minima in sc[2..3]; others 16 bytes
+    uint32_t sc[4];   // scales times 2^UP: Q4_K/Q5_K sub-blocks 0..7 in sc[0..1] (minima in sc[2..3]); others 16 bytes
     uint32_t dd;      // Q6_K: d, Q2_K: d, dmin (the arrays after the rows)
 
     QP_DEV void setup() {
         if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) {
-            sc[0] = h[1] & 0x3f3f3f3fu;
-            sc[1] = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
+            sc[0] = (h[1] << 2) & 0xfcfcfcfcu;
+            sc[1] = ((h[3] << 2) & 0x3c3c3c3cu) | (h[1] & 0xc0c0c0c0u);
             sc[2] = h[2] & 0x3f3f3f3fu;
             sc[3] = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
         } else if constexpr (FMT == QP_Q6_K) {
 #pragma unroll
             for (int i = 0; i < 4; i++) sc[i] = h[i] ^ 0x80808080u;
         } else if constexpr (FMT == QP_Q3_K) {
-            const uint32_t k1 = 0x03030303u, k2 = 0x0f0f0f0fu;
-            sc[0] = (h[0] & k2) | ((h[2] & k1) << 4);
-            sc[1] = (h[1] & k2) | (((h[2] >> 2) & k1) << 4);
-            sc[2] = ((h[0] >> 4) & k2) | (((h[2] >> 4) & k1) << 4);
-            sc[3] = ((h[1] >> 4) & k2) | (((h[2] >> 6) & k1) << 4);
+            const uint32_t k1 = 0xc0c0c0c0u, k2 = 0x3c3c3c3cu;
+            sc[0] = ((h[0] << 2) & k2) | ((h[2] << 6) & k1);
+            sc[1] = ((h[1] << 2) & k2) | ((h[2] << 4) & k1);
+            sc[2] = ((h[0] >> 2) & k2) | ((h[2] << 2) & k1);
+            sc[3] = ((h[1] >> 2) & k2) | (h[2] & k1);
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; i++) sc[i] = h[i] & 0x0f0f0f0fu;
+            for (int i = 0; i < 4; i++) sc[i] = (h[i] << 4) & 0xf0f0f0f0u;
         }
     }
     QP_DEV float d() const {
@@ -202,14 +206,14 @@ struct SkBlock {
         }
         return r;
     }
-    // scale * quant * 2^-24 of this lane's eight inputs of step j (32 inputs), as f16 (lo: what is left of Q6_K's
+    // scale * quant * 2^(UP - 19) of this lane's eight inputs of step j (32 inputs), as f16 (lo: what is left of Q6_K's
     // products, which reach 8064).
     template <int j>
     QP_DEV void step(h8& hi, h8& lo) const {
         h2 q[4], s[2];
         if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) {
             constexpr int c = (FMT == QP_Q4_K ? 1 : 3) + 2 * (j >> 1), at = (j & 1) * 4;
-            s[0] = s[1] = sk_dup<at>(sc[j >> 2], sk_sel(j & 3, j & 3));
+            s[0] = s[1] = sk_dup<at - 5>(sc[j >> 2], sk_sel(j & 3, j & 3));
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)];
@@ -226,7 +230,7 @@ struct SkBlock {
         } else if constexpr (FMT == QP_Q2_K) {
             constexpr int c = 1 + 2 * (j >> 2), at = 2 * (j & 3);
 #pragma unroll
-            for (int i = 0; i < 2; i++) s[i] = sk_dup<at>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3));
+            for (int i = 0; i < 2; i++) s[i] = sk_dup<at - 5>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3));
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)];
@@ -237,7 +241,7 @@ struct SkBlock {
             h2 o[2];
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                s[i] = sk_dup<at>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3), -32.0f);
+                s[i] = sk_dup<at - 5>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3), -128.0f);
                 const float m4 = -4.0f * (1 << at) * 0x1p-24f;
                 o[i] = s[i] * h2{(_Float16)m4, (_Float16)m4};
             }
@@ -253,7 +257,7 @@ struct SkBlock {
             constexpr int hh = j >> 2, qd = j & 3, c = 4 * hh + (qd & 1) * 2, at = (qd >> 1) * 4, up = 4 + at - 2 * qd;
 #pragma unroll
             for (int i = 0; i < 2; i++)
-                s[i] = sk_dup<at>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3), -128.0f);
+                s[i] = sk_dup<at - 5>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3), -128.0f);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)], hb = t[8 + 2 * hh + (i >> 1)];
@@ -392,7 +396,7 @@ QP_DEV void sk_kq(const SkRows (&rw)[R], uint32_t nb, uint32_t gi0, uint32_t gi1
                 step(SkInt<4>()); step(SkInt<5>()); step(SkInt<6>()); step(SkInt<7>());
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    const float d = blk[r].d() * 0x1p24f;
+                    const float d = blk[r].d() * (float)(1 << (19 - F::UP));
                     if constexpr (F::MIN) {
                         const h8 mn = blk[r].mins(g);
                         const float dm = blk[r].dmin();
@@ -503,15 +507,16 @@ QP_DEV void sk_pl(const SkRows (&rw)[R], uint32_t K, uint32_t ch0, uint32_t ch1,
                         a = iq4nl_lut4(q & 0x0f0f0f0fu) ^ 0x80808080u;
                         b = iq4nl_lut4((q >> 4) & 0x0f0f0f0fu) ^ 0x80808080u;
                     }
-                    const h2 o = {(_Float16)(-128.0f * 0x1p-24f), (_Float16)(-128.0f * 0x1p-24f)};
+                    const h2 k14 = {(_Float16)16384.0f, (_Float16)16384.0f}, o = {(_Float16)-0.125f, (_Float16)-0.125f};
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         const uint32_t w8 = i < 2 ? a : b;
-                        const h2 v = as_h2(((i & 1) ? w8 >> 8 : w8) & 0x00ff00ffu) + o;
+                        // byte * 2^-24 to (byte - 128) * 2^-10
+                        const h2 v = __builtin_elementwise_fma(as_h2(((i & 1) ? w8 >> 8 : w8) & 0x00ff00ffu), k14, o);
                         hi[2 * i] = v[0];
                         hi[2 * i + 1] = v[1];
                     }
-                    d = ds[r][j] * 0x1p24f;
+                    d = ds[r][j] * 0x1p10f;
                 }
 #pragma unroll
                 for (int t = 0; t < NT; t++) {

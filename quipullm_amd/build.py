@@ -1,6 +1,6 @@
 """Builds the native parts in-tree (quipullm_amd/lib/):
 
-* quipu_kernels.hsaco, quipu_small.hsaco -- the gfx950 kernels (hipcc --genco), loaded with hipModuleLoad;
+* quipu_kernels.hsaco, quipu_small.hsaco, quipu_attn.hsaco -- the gfx950 kernels (hipcc --genco), loaded with hipModuleLoad;
 * libquipu.so         -- the C ABI of include/quipu.h (HIP runtime, op table);
 * quipu_napi.node     -- the Node.js (N-API) addon over libquipu.so, for the JavaScript host.
 
@@ -23,7 +23,7 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 NODE_INC = "/usr/include/node"
 
 HSACO = os.path.join(LIB, "quipu_kernels.hsaco")
-HSACO2 = os.path.join(LIB, "quipu_small.hsaco")
+OBJECTS = ("kernels", "small", "attn")   # qp_<name>.hip -> quipu_<name>.hsaco
 SO = os.path.join(LIB, "libquipu.so")
 NAPI = os.path.join(LIB, "quipu_napi.node")
 
@@ -58,14 +58,14 @@ TIMELINE_LIB = os.path.join(LIB, "timeline")
 
 
 def build_kernels(lib=LIB, defs=()):
-    """The two code objects, compiled side by side."""
+    """The code objects, compiled side by side."""
     def one(name):
         src = os.path.join(CSRC, "kernels", "qp_%s.hip" % name)
         out = os.path.join(lib, "quipu_%s.hsaco" % name)
         _atomic(out, lambda o: _run([HIPCC, "--genco", *HIP_FLAGS, *defs, "-o", o, src], name))
         return out
-    with ThreadPoolExecutor(2) as ex:
-        return list(ex.map(one, ("kernels", "small")))
+    with ThreadPoolExecutor(len(OBJECTS)) as ex:
+        return list(ex.map(one, OBJECTS))
 
 
 def build_lib(lib=LIB, defs=()):
@@ -119,7 +119,7 @@ def build_all(oracle=True):
 
 
 def built() -> bool:
-    return all(os.path.exists(p) for p in (HSACO, HSACO2, SO))
+    return all(os.path.exists(p) for p in [SO] + [os.path.join(LIB, "quipu_%s.hsaco" % n) for n in OBJECTS])
 
 
 if __name__ == "__main__":

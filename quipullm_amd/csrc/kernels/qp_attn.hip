@@ -1,0 +1,349 @@
+// Causal attention over f32 caches, sliding windows and rings (the reference's atencion, gpu.js:467-539) on the matrix
+// cores, at f32 accuracy.
+//
+// A workgroup takes 16 RG (query, head) rows of one KV head and a share of the key tiles of 32 slots, dealt to its four
+// wavefronts; each keeps its own softmax state and they meet in LDS.  Scores are S^T = K Q^T and outputs O^T += V^T P^T
+// with v_mfma_f32_16x16x32_f16: a lane holds 8 scores of one row, which are its operand of the second product.  Every
+// f32 operand is an f16 high and low part (22 bits) below a power of two: of the row for Q, of the largest magnitude that
+// the wavefront has met so far for K and V (so a tile is never scaled past f16's range, and values down to 2^-12 of the
+// largest keep all 22 bits), 2^10 for P.  Three products per pair (high high, high low, low high); f16 caches need two.
+// Probabilities, their sums, the maxima and the outputs are f32.
+#include "qp_common.h"
+
+#define KERNEL extern "C" __global__
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+QP_DEV f32x4 ax_mfma(h8 a, h8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+// f16 high and low parts of eight values already below 2^10.
+QP_DEV void ax_split(const float* v, float up, h8& hi, h8& lo) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float s = v[i] * up;
+        hi[i] = (_Float16)s;
+        lo[i] = (_Float16)(s - (float)hi[i]);
+    }
+}
+// Exponent e of a magnitude, clamped so that 2^(9 - e) and 2^(e - 9) are normal; -117 for 0.
+QP_DEV int ax_exp(float m) {
+    const int e = (int)((__float_as_uint(m) >> 23) & 255) - 127;
+    return e < -117 ? -117 : e;
+}
+QP_DEV float ax_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+constexpr float AX_LOG2E = 1.4426950408889634f;
+
+template <int HD, bool F16, int RG>
+QP_DEV void attn_x_body(const QpAttnArgs& a) {
+    constexpr int KS = HD / 32, DT = HD / 16;  // steps of 32 dimensions, tiles of 16 (DT dimensions per lane of 16)
+    extern __shared__ float4 ax_lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n16 = lane & 15;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t T = min(paso_T(a.paso), a.tcov), pos0 = paso_pos(a.paso);
+    const uint32_t G = a.nh / a.nkv, kvh = blockIdx.x, kvd = a.nkv * HD, nrow = T * G;
+    const uint32_t r0 = blockIdx.y * (16 * RG);
+    if (r0 >= nrow) return;
+    const uint32_t t_lo = r0 / G, t_hi = (min(r0 + 16 * RG, nrow) - 1) / G;
+    // ---- the rows' queries
+    h8 qh[RG][KS], ql[RG][KS];
+    float qs[RG];         // score = accumulator * qs (times the keys' scale), in units of log2
+    int lim[RG], low[RG]; // keys low < key <= lim
+#pragma unroll
+    for (int r = 0; r < RG; r++) {
+        const uint32_t row = r0 + r * 16 + n16, rc = min(row, nrow - 1), t = rc / G, h = kvh * G + rc % G;
+        float v[KS][8];
+        float mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const uint64_t at = a.q + 4 * (((uint64_t)t * a.nh + h) * HD + s * 32 + g * 8);
+            const float4 x = gload<float4>(at), y = gload<float4>(at + 16);
+            const float w[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                v[s][i] = w[i];
+                mx = fmaxf(mx, fabsf(w[i]));
+            }
+        }
+        mx = fmaxf(mx, bfly_f<4>(mx, lane));
+        mx = fmaxf(mx, bfly_f<5>(mx, lane));
+        const int e = ax_exp(mx);
+#pragma unroll
+        for (int s = 0; s < KS; s++) ax_split(v[s], ax_pow2(9 - e), qh[r][s], ql[r][s]);
+        qs[r] = ax_pow2(e - 9) * a.scale * AX_LOG2E;
+        lim[r] = (int)(pos0 + t);
+        low[r] = a.swa && pos0 + t >= a.swa ? (int)(pos0 + t - a.swa) : -1;
+    }
+    // ---- the key tiles: keys kbeg .. kend in slots first .. (ring: then 0 ..), whole tiles of 32 slots
+    const uint32_t kend = a.cap ? pos0 + t_hi + 1 : min(pos0 + t_hi + 1, a.rows);
+    const uint32_t kbeg = a.swa && pos0 + t_lo + 1 > a.swa ? min(pos0 + t_lo + 1 - a.swa, kend) : 0;
+    const uint32_t first = a.cap ? kbeg % a.cap : kbeg, nkey = a.cap ? min(kend - kbeg, a.cap) : kend - kbeg;
+    const uint32_t end_a = a.cap ? min(first + nkey, a.cap) : first + nkey, end_b = first + nkey - end_a;
+    const uint32_t ta = nkey ? (end_a + 31) / 32 - first / 32 : 0, nt = ta + (end_b + 31) / 32;
+    const uint32_t per = (nt + a.nsplit - 1) / a.nsplit, i0 = blockIdx.z * per, i1 = min(nt, i0 + per);
+    constexpr uint32_t eb = F16 ? 2 : 4;
+    const uint64_t slots = F16 ? (a.rows + 31ull) / 32 * 32 : a.rows;  // (the f16 value cache holds whole tiles)
+    const __amdgpu_buffer_rsrc_t kr = kq_rsrc(a.kc, (uint64_t)a.rows * kvd * eb), vr = kq_rsrc(a.vc, slots * kvd * eb);
+
+    constexpr int KL = F16 ? KS : 2 * KS;       // 16-byte loads of one key per lane
+    constexpr int VL = F16 ? DT : 8 * (DT / 4); // 16-byte loads of a tile's values per lane
+    u32x4 kw[2][KL], vw[VL];
+    struct Tile { uint32_t slot, lo, hi; int off; };  // slots lo .. hi of it hold keys slot + off
+    auto tile = [&](uint32_t i) __attribute__((always_inline)) {
+        Tile t;
+        if (i < ta) t = {(first / 32 + i) * 32, first, end_a, (int)(kbeg - first)};
+        else t = {(i - ta) * 32, 0, end_b, (int)(kbeg + a.cap - first)};
+        return t;
+    };
+    auto load_k = [&](uint32_t i) __attribute__((always_inline)) {
+        const Tile t = tile(i);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t s = t.slot + h * 16 + n16;
+            const uint32_t o = i < i1 && s >= t.lo && s < t.hi ? (s * kvd + kvh * HD + 8 * g) * eb : QP_NOOFF;
+#pragma unroll
+            for (int c = 0; c < KL; c++)
+                kw[h][c] = __builtin_amdgcn_raw_buffer_load_b128(kr, o, F16 ? c * 64 : (c >> 1) * 128 + (c & 1) * 16, 0);
+        }
+    };
+    auto load_v = [&](uint32_t i) __attribute__((always_inline)) {
+        const Tile t = tile(i);
+        if constexpr (F16) {
+            const uint32_t o = i < i1 ? (t.slot * kvd + (kvh * HD + DT * n16) * 32) * 2 + g * 16 : QP_NOOFF;
+#pragma unroll
+            for (int c = 0; c < DT; c++) vw[c] = __builtin_amdgcn_raw_buffer_load_b128(vr, o, c * 64, 0);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t s = t.slot + (j >> 2) * 16 + 4 * g + (j & 3);
+                const uint32_t o = i < i1 && s >= t.lo && s < t.hi ? (s * kvd + kvh * HD + DT * n16) * 4 : QP_NOOFF;
+#pragma unroll
+                for (int c = 0; c < DT / 4; c++)
+                    vw[j * (DT / 4) + c] = __builtin_amdgcn_raw_buffer_load_b128(vr, o, c * 16, 0);
+            }
+        }
+    };
+
+    f32x4 o[RG][DT];
+    float m[RG], l[RG];
+    int ek = -117, ev = -117;  // exponents of the largest key and value so far
+#pragma unroll
+    for (int r = 0; r < RG; r++) {
+        m[r] = -3.0e38f;
+        l[r] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DT; d++) o[r][d] = f32x4{0, 0, 0, 0};
+    }
+    uint32_t i = i0 + wave;
+    load_k(i);
+    load_v(i);
+    for (; i < i1; i += 4) {
+        const Tile t = tile(i);
+        // ---- S^T = K Q^T
+        float upk = 1.0f, ck = 1.0f;
+        if constexpr (!F16) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int c = 0; c < KL; c++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) mx = fmaxf(mx, fabsf(__uint_as_float(kw[h][c][x])));
+            ek = max(ek, __builtin_amdgcn_readfirstlane(ax_exp(wave_max_v(mx, lane))));
+            upk = ax_pow2(9 - ek);
+            ck = ax_pow2(ek - 9);
+        }
+        f32x4 s[RG][2];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int c = 0; c < KS; c++) {
+                h8 kh, kl;
+                if constexpr (F16) {
+                    kh = __builtin_bit_cast(h8, kw[h][c]);
+                } else {
+                    float v[8];
+#pragma unroll
+                    for (int x = 0; x < 8; x++) v[x] = __uint_as_float(kw[h][2 * c + (x >> 2)][x & 3]);
+                    ax_split(v, upk, kh, kl);
+                }
+#pragma unroll
+                for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kh, qh[r][c], c ? s[r][h] : f32x4{0, 0, 0, 0});
+#pragma unroll
+                for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kh, ql[r][c], s[r][h]);
+                if constexpr (!F16) {
+#pragma unroll
+                    for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kl, qh[r][c], s[r][h]);
+                }
+            }
+        load_k(i + 4);
+        // ---- softmax of the lane's 8 keys of each of its rows
+        // all slots hold keys that every row of the block sees
+        const bool whole = t.slot >= t.lo && t.slot + 32 <= t.hi && (int)t.slot + 31 + t.off <= (int)(pos0 + t_lo) &&
+                           (!a.swa || (int)t.slot + t.off > (int)(pos0 + t_hi) - (int)a.swa);
+        h8 ph[RG], pl[RG];
+        float corr[RG];
+#pragma unroll
+        for (int r = 0; r < RG; r++) {
+            const float c = qs[r] * ck;
+            float x[8], mx = -3.0e38f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                x[j] = s[r][j >> 2][j & 3] * c;
+                if (!whole) {
+                    const uint32_t sl = t.slot + (j >> 2) * 16 + 4 * g + (j & 3);
+                    const int key = (int)sl + t.off;
+                    x[j] = sl >= t.lo && sl < t.hi && key <= lim[r] && key > low[r] ? x[j] : -__builtin_inff();
+                }
+                mx = fmaxf(mx, x[j]);
+            }
+            mx = fmaxf(mx, bfly_f<4>(mx, lane));
+            mx = fmaxf(mx, bfly_f<5>(mx, lane));
+            const float mn = fmaxf(m[r], mx);
+            corr[r] = __builtin_amdgcn_exp2f(m[r] - mn);
+            m[r] = mn;
+            float sum = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float p = __builtin_amdgcn_exp2f(x[j] - mn);
+                sum += p;
+                const float p10 = p * 1024.0f;
+                ph[r][j] = (_Float16)p10;
+                pl[r][j] = (_Float16)(p10 - (float)ph[r][j]);
+            }
+            l[r] = l[r] * corr[r] + sum;
+        }
+        // ---- O^T += V^T P^T
+        float upv = 1.0f, ratio = 1.0f;
+        if constexpr (!F16) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int c = 0; c < VL; c++)
+#pragma unroll
+                for (int x = 0; x < 4; x++) mx = fmaxf(mx, fabsf(__uint_as_float(vw[c][x])));
+            const int en = max(ev, __builtin_amdgcn_readfirstlane(ax_exp(wave_max_v(mx, lane))));
+            ratio = ev - en < -120 ? 0.0f : ax_pow2(ev - en);
+            ev = en;
+            upv = ax_pow2(9 - ev);
+        }
+        float keep = ratio;
+        bool same = true;
+#pragma unroll
+        for (int r = 0; r < RG; r++) same = same && corr[r] * ratio == 1.0f;
+        if (!__builtin_amdgcn_readfirstlane(__all(same))) {
+#pragma unroll
+            for (int r = 0; r < RG; r++) {
+                const float f = corr[r] * keep;
+#pragma unroll
+                for (int d = 0; d < DT; d++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) o[r][d][x] *= f;
+            }
+        }
+        const bool inside = t.slot >= t.lo && t.slot + 32 <= t.hi;
+#pragma unroll
+        for (int d = 0; d < DT; d++) {
+            h8 vh, vl;
+            if constexpr (F16) {
+                vh = __builtin_bit_cast(h8, vw[d]);
+                if (!inside) {  // slots without a key may hold anything
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const uint32_t sl = t.slot + (j >> 2) * 16 + 4 * g + (j & 3);
+                        vh[j] = sl >= t.lo && sl < t.hi ? vh[j] : (_Float16)0.0f;
+                    }
+                }
+            } else {
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = __uint_as_float(vw[j * (DT / 4) + (d >> 2)][d & 3]);
+                ax_split(v, upv, vh, vl);
+            }
+#pragma unroll
+            for (int r = 0; r < RG; r++) o[r][d] = ax_mfma(vh, ph[r], o[r][d]);
+#pragma unroll
+            for (int r = 0; r < RG; r++) o[r][d] = ax_mfma(vh, pl[r], o[r][d]);
+            if constexpr (!F16) {
+#pragma unroll
+                for (int r = 0; r < RG; r++) o[r][d] = ax_mfma(vl, ph[r], o[r][d]);
+            }
+        }
+        load_v(i + 4);
+    }
+    // ---- the four wavefronts' states meet: [wave][row][HD + 4], then [wave][row] (m, l)
+    constexpr int LD = HD + 4;
+    float* ol = reinterpret_cast<float*>(ax_lds);
+    float* ml = ol + 4 * RG * 16 * LD;
+    const float back = (F16 ? 1.0f : ax_pow2(ev - 9)) * 0x1p-10f;
+#pragma unroll
+    for (int r = 0; r < RG; r++) {
+        float lt = l[r];
+        lt += bfly_f<4>(lt, lane);
+        lt += bfly_f<5>(lt, lane);
+        const uint32_t at = wave * RG * 16 + r * 16 + n16;
+        if (g == 0) {
+            ml[2 * at] = m[r];
+            ml[2 * at + 1] = lt;
+        }
+        // dimensions DT * (4 g + x) + d of the row
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int d = 0; d < DT; d += 4)
+                *reinterpret_cast<float4*>(ol + at * LD + DT * (4 * g + x) + d) =
+                    make_float4(o[r][d][x] * back, o[r][d + 1][x] * back, o[r][d + 2][x] * back, o[r][d + 3][x] * back);
+    }
+    __syncthreads();
+    for (uint32_t k = tid; k < RG * 16 * (HD / 4); k += 256) {
+        const uint32_t lr = k / (HD / 4), c = k % (HD / 4), row = r0 + lr;
+        if (row >= nrow) continue;
+        float M = -3.0e38f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) M = fmaxf(M, ml[2 * (w * RG * 16 + lr)]);
+        float L = 0.0f;
+        float4 s = make_float4(0, 0, 0, 0);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const uint32_t at = w * RG * 16 + lr;
+            const float lw = ml[2 * at + 1], f = lw != 0.0f ? __builtin_amdgcn_exp2f(ml[2 * at] - M) : 0.0f;
+            const float4 v = *reinterpret_cast<const float4*>(ol + at * LD + 4 * c);
+            L += lw * f;
+            if (f != 0.0f) s = make_float4(s.x + v.x * f, s.y + v.y * f, s.z + v.z * f, s.w + v.w * f);
+        }
+        const uint32_t t = row / G, h = kvh * G + row % G;
+        const uint64_t at = (uint64_t)t * a.nh + h;
+        if (a.nsplit == 1) {
+            gstore<float4>(a.o + 4 * (at * HD + 4 * c), make_float4(s.x / L, s.y / L, s.z / L, s.w / L));
+        } else {
+            gstore<float4>(a.part_o + 4 * ((at * a.nsplit + blockIdx.z) * HD + 4 * c), s);
+            if (c == 0) gstore<float2>(a.part_ml + 8 * (at * a.nsplit + blockIdx.z), make_float2(M, L));
+        }
+    }
+}
+
+#define ATTN_X(HD, NAME, F16)                                                                                         \
+    KERNEL __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void qp_attn_x_h##HD##_##NAME##_r1(         \
+        QpAttnArgs a) { attn_x_body<HD, F16, 1>(a); }                                                                 \
+    KERNEL __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void qp_attn_x_h##HD##_##NAME##_r2(         \
+        QpAttnArgs a) { attn_x_body<HD, F16, 2>(a); }
+ATTN_X(64, f32, false) ATTN_X(128, f32, false) ATTN_X(64, f16, true) ATTN_X(128, f16, true)
+
+// The splits' partial states of each (query, head) row -> o, in split order: grid rows, hd threads.
+KERNEL __launch_bounds__(128) void qp_attn_x_comb(QpAttnArgs a) {
+    const uint32_t t = blockIdx.x / a.nh, d = threadIdx.x;
+    if (t >= paso_T(a.paso)) return;
+    const uint64_t row = blockIdx.x;
+    const uint64_t ml = a.part_ml + 8 * row * a.nsplit, po = a.part_o + 4 * (row * a.nsplit * a.hd + d);
+    float M = -3.0e38f;
+    for (uint32_t s = 0; s < a.nsplit; s++) M = fmaxf(M, gload<float>(ml + 8 * s));
+    float L = 0.0f, o = 0.0f;
+    for (uint32_t s = 0; s < a.nsplit; s++) {
+        const float lw = gload<float>(ml + 8 * s + 4), f = lw != 0.0f ? __builtin_amdgcn_exp2f(gload<float>(ml + 8 * s) - M) : 0.0f;
+        const float v = gload<float>(po + 4ull * s * a.hd);
+        L += lw * f;
+        o += f != 0.0f ? v * f : 0.0f;
+    }
+    gstore<float>(a.o + 4 * (row * a.hd + d), o / L);
+}

@@ -185,7 +185,11 @@ typedef struct {
     uint32_t rows;           // slots of the cache; keys at or past it are not read
     uint32_t orows;          // 0: o holds f32 rows; else o receives them as the next matmul's bf16 input planes
                              // (qp_split_bf16's layout, orows token rows, K = nh hd)
-    uint32_t pad[2];
+    // qp_attn_x_*: shares of the keys (grid z); above 1: each row's partial state per share, part_o [T nh][nsplit][hd]
+    // and part_ml [T nh][nsplit] (maximum in units of log2, sum), merged by qp_attn_x_comb;
+    // tcov: tokens the dispatch covers (none past them is computed)
+    uint32_t nsplit, tcov;
+    uint64_t part_o, part_ml;
 } QpAttnArgs;
 
 // Split-K decode attention with fused q/k norm + RoPE + KV append (one token).

@@ -32,7 +32,7 @@ bool g_init = false;
 std::atomic<int> g_lost{0};
 int g_device = 0;
 hipStream_t g_stream = nullptr;
-hipModule_t g_mod = nullptr, g_mod2 = nullptr;
+hipModule_t g_mod = nullptr;  // the first code object (timeline builds read its records)
 std::mutex g_mu;
 std::unordered_map<uint64_t, uint64_t> g_allocs;  // address -> bytes
 uint64_t g_bytes = 0;
@@ -78,24 +78,33 @@ int hip_fail(hipError_t e, const char* what) {
 enum Kid {
 #define K(name) K_##name,
 #define M(name) K_##name,
+#define A(name) K_##name,
 #include "qp_kernel_list.inc"
 #undef K
 #undef M
+#undef A
     K_COUNT
 };
 const char* kNames[] = {
 #define K(name) "qp_" #name,
 #define M(name) "qp_" #name,
+#define A(name) "qp_" #name,
 #include "qp_kernel_list.inc"
 #undef K
 #undef M
+#undef A
 };
-const bool kSmall[] = {  // in the second code object (qp_small.hip)
-#define K(name) false,
-#define M(name) true,
+// The code objects (beside each other; one source file each) and which of them holds a kernel.
+constexpr int kObjects = 3;
+const char* kObjectNames[kObjects] = {"quipu_kernels.hsaco", "quipu_small.hsaco", "quipu_attn.hsaco"};
+const uint8_t kObject[] = {
+#define K(name) 0,
+#define M(name) 1,
+#define A(name) 2,
 #include "qp_kernel_list.inc"
 #undef K
 #undef M
+#undef A
 };
 hipFunction_t g_fn[K_COUNT];
 
@@ -908,6 +917,33 @@ int op_atencion(const Ctx& c) {
         return launch((two ? km2 : km)[a.hd == 128][gi], a.nkv, cdiv(c.gy ? c.gy : 1, (two ? 1 : 4) * tpw), 1, 256, 0,
                       a);
     }
+    // f32 caches, windows and rings: matrix cores at f32 accuracy (qp_attn.hip), 16 or 32 (query, head) rows per
+    // workgroup, the keys shared out (grid z) while the rows alone give fewer than one workgroup per CU and every share
+    // keeps 128 keys.  A ring without a window, or a cache whose offsets pass 31 bits, stays with the general kernel.
+    const uint32_t T = c.gy ? c.gy : 1, nrow = T * G, RG = nrow > 16 ? 2 : 1, yb = cdiv(nrow, 16 * RG);
+    if ((!a.cap || a.swa) && 4ull * a.nkv * a.hd * ((a.rows + 31) / 32 * 32) < (1ull << 31) && !getenv_flag("QP_NO_MFMA")) {
+        const uint32_t cus = g_cus > 0 ? (uint32_t)g_cus : 1u;
+        const uint32_t keys = a.swa && a.swa + T < a.rows ? a.swa + T : a.rows;
+        uint32_t ns = cdiv(cus, a.nkv * yb);
+        if (ns > cdiv(keys, 128)) ns = cdiv(keys, 128);
+        if (ns > 64) ns = 64;
+        const uint64_t per = (uint64_t)T * a.nh * (4 * a.hd + 8);  // bytes of one share's partial states
+        if (g_capturing && !g_noalloc) ns = 1;                     // (they need the workspace)
+        if (g_noalloc && ns * per > QP_SCRATCH_BYTES) ns = 1;
+        a.nsplit = ns;
+        a.tcov = T;
+        if (ns > 1) {
+            if (int e = workspace(ns * per, &a.part_o)) return e;
+            a.part_ml = a.part_o + 4ull * T * a.nh * ns * a.hd;
+            if (a.part_o == g_split_memo.xs) g_split_memo.valid = false;  // (a split input kept there is overwritten)
+        }
+        static const Kid kx[2][2][2] = {{{K_attn_x_h64_f32_r1, K_attn_x_h64_f32_r2}, {K_attn_x_h64_f16_r1, K_attn_x_h64_f16_r2}},
+                                        {{K_attn_x_h128_f32_r1, K_attn_x_h128_f32_r2},
+                                         {K_attn_x_h128_f16_r1, K_attn_x_h128_f16_r2}}};
+        const uint32_t lds = 4 * RG * 16 * (a.hd + 4) * 4 + 4 * RG * 16 * 8;
+        if (int e = launch(kx[a.hd == 128][a.f16 ? 1 : 0][RG == 2], a.nkv, yb, ns, 256, lds, a)) return e;
+        return ns == 1 ? 0 : launch(K_attn_x_comb, T * a.nh, 1, 1, a.hd, 0, a);
+    }
     const uint32_t qb = 32 / G;
     a.qb = qb;
     return launch(a.hd == 64 ? K_attn_hd64 : K_attn_hd128, a.nkv, cdiv(c.gy ? c.gy : 1, qb), 1, 256, attn_lds(a.hd),
@@ -1696,13 +1732,16 @@ int qp_init(int device) {
     std::string path;
     if (const char* e = getenv("QP_KERNELS")) path = e;
     else path = self_dir() + "/quipu_kernels.hsaco";
-    HIPCHK(hipModuleLoad(&g_mod, path.c_str()), ("hipModuleLoad " + path).c_str());
-    // the second code object lies beside the first
     const size_t slash = path.rfind('/');
-    const std::string path2 = (slash == std::string::npos ? std::string() : path.substr(0, slash + 1)) + "quipu_small.hsaco";
-    HIPCHK(hipModuleLoad(&g_mod2, path2.c_str()), ("hipModuleLoad " + path2).c_str());
+    const std::string dir = slash == std::string::npos ? std::string() : path.substr(0, slash + 1);
+    hipModule_t mods[kObjects];
+    for (int i = 0; i < kObjects; i++) {
+        const std::string p = i ? dir + kObjectNames[i] : path;
+        HIPCHK(hipModuleLoad(&mods[i], p.c_str()), ("hipModuleLoad " + p).c_str());
+    }
+    g_mod = mods[0];
     for (int k = 0; k < K_COUNT; k++)
-        HIPCHK(hipModuleGetFunction(&g_fn[k], kSmall[k] ? g_mod2 : g_mod, kNames[k]), kNames[k]);
+        HIPCHK(hipModuleGetFunction(&g_fn[k], mods[kObject[k]], kNames[k]), kNames[k]);
     g_device = device;
     g_init = true;
     return 0;

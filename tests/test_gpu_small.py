@@ -114,3 +114,72 @@ def test_few_jobs_per_expert(quipu, dev, oracle, fmt):
             e = sel[j]
             xr = x[j // tfijo][None]
             assert np.all(np.abs(outs[0][j] - (xr.astype(np.float64) @ W[e].T)[0]) <= bound(W[e], xr)[0]), j
+
+
+@pytest.mark.parametrize("f16", [0, 1])
+@pytest.mark.parametrize("hd,nh,nkv,T,pos0,swa,cap", [
+    (128, 8, 8, 1, 0, 0, 0),          # one key
+    (64, 6, 2, 5, 31, 0, 0),          # a group of 3 heads, 15 rows, keys to a tile's edge
+    (128, 8, 4, 8, 1000, 0, 0),       # 16 rows, keys shared out
+    (128, 10, 2, 7, 64, 0, 0),        # 35 rows: the second block of 32 nearly empty
+    (64, 32, 1, 3, 500, 0, 0),        # 32 heads per KV head
+    (128, 4, 2, 70, 130, 33, 0),      # a window narrower than a block, no ring
+    (64, 8, 2, 24, 200, 64, 88),      # a ring of 88 slots (no multiple of 32) that the keys wrap in
+    (128, 4, 4, 1, 500, 100, 132),    # one token of a ring
+    (64, 4, 4, 40, 0, 64, 104),       # a ring that is not full yet
+])
+def test_attention_any_cache(quipu, dev, hd, nh, nkv, T, pos0, swa, cap, f16):
+    """atencion on f32 caches, windows and rings against float64: keys a row does not see (later ones, those before its
+    window, ring slots not written) are NaN or 6e4 in the cache and must not matter.
+
+    Bound: scores are exact to 2^-21 |q| |k| scale (22-bit factors, products and sums in float32), so weights to that
+    relative error e; outputs to (2 e + 2^-19) max |v| (22-bit probabilities and values, float32 sums over the keys)."""
+    kvd, n = nkv * hd, pos0 + T
+    rng = np.random.default_rng(81)
+    q = rng.standard_normal((T, nh * hd)).astype(np.float32)
+    kf, vf = (rng.standard_normal((n, kvd)).astype(np.float32) * 10.0 ** rng.uniform(-2, 1, (n, 1)).astype(np.float32)
+              for _ in range(2))
+    dt = np.float16 if f16 else np.float32
+    kf, vf = kf.astype(dt).astype(np.float32), vf.astype(dt).astype(np.float32)
+    slots = cap or n + 9
+    # (the f16 path without windows takes slots not yet written as finite: the engine zeroes its caches)
+    kc, vc = (np.full((slots, kvd), 0 if f16 and not swa and nh // nkv in (1, 2, 4, 8) else np.nan, dt) for _ in range(2))
+    for p in range(max(0, n - slots), n):
+        kc[p % slots], vc[p % slots] = kf[p], vf[p]
+    if swa and not cap:
+        kc[:max(0, pos0 + 1 - swa)] = 6e4  # before every row's window
+    if f16:
+        import refs
+        vb = dev.buf(refs.v_tiled(vc, kvd))
+    else:
+        vb = dev.buf(vc)
+    o = dev.zeros(4 * T * nh * hd)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    quipu.dispatch("atencion", [("u", hd), ("u", nh), ("u", nkv), ("u", swa), ("f", scale), ("u", cap), ("u", 0), ("u", 0),
+                                ("u", f16), ("u", slots)],
+                   [dev.paso(T, pos0), dev.buf(q), dev.buf(kc), vb, o], (nh, T))
+    got = dev.get(o, (T, nh, hd))
+    q64, k64, v64 = (a.astype(np.float64).reshape(a.shape[0], -1, hd) for a in (q, kf, vf))
+    for t in range(T):
+        a, b = max(0, pos0 + t + 1 - swa) if swa else 0, pos0 + t + 1
+        for h in range(nh):
+            k, v = k64[a:b, h * nkv // nh], v64[a:b, h * nkv // nh]
+            s = k @ q64[t, h] * scale
+            w = np.exp(s - s.max())
+            w /= w.sum()
+            e = 2.0 ** -21 * np.abs(q64[t, h]).max() * np.abs(k).max() * hd * scale
+            assert np.all(np.abs(got[t, h] - w @ v) <= (2 * e + 2.0 ** -19) * np.abs(v).max()), (t, h)
+
+
+def test_attention_shares_cover_no_token_past_the_dispatch(quipu, dev):
+    """A Paso of more tokens than the dispatch covers: the others' outputs stay as they were (shares of the keys keep
+    partial states for the covered tokens only)."""
+    hd, nh, nkv, rows = 64, 2, 1, 600
+    rng = np.random.default_rng(82)
+    q, kc, vc = (rng.standard_normal(s).astype(np.float32) for s in ((9, nh * hd), (rows, hd), (rows, hd)))
+    o = dev.buf(np.full((9, nh * hd), 5.0, np.float32))
+    quipu.dispatch("atencion", [("u", hd), ("u", nh), ("u", nkv), ("u", 0), ("f", 0.125), ("u", 0), ("u", 0), ("u", 0),
+                                ("u", 0), ("u", rows)],
+                   [dev.paso(9, 500), dev.buf(q), dev.buf(kc), dev.buf(vc), o], (nh, 2))
+    got = dev.get(o, (9, nh * hd))
+    assert np.all(got[2:] == 5.0) and not np.any(got[:2] == 5.0)

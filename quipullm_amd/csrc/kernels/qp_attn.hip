@@ -330,20 +330,30 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
         QpAttnArgs a) { attn_x_body<HD, F16, 2>(a); }
 ATTN_X(64, f32, false) ATTN_X(128, f32, false) ATTN_X(64, f16, true) ATTN_X(128, f16, true)
 
-// The splits' partial states of each (query, head) row -> o, in split order: grid rows, hd threads.
+// The shares' partial states of each (query, head) row -> o, in their order: grid rows, hd threads (at most 64 shares).
 KERNEL __launch_bounds__(128) void qp_attn_x_comb(QpAttnArgs a) {
-    const uint32_t t = blockIdx.x / a.nh, d = threadIdx.x;
+    __shared__ float wt[64], den;
+    const uint32_t t = blockIdx.x / a.nh, d = threadIdx.x, ns = a.nsplit;
     if (t >= paso_T(a.paso)) return;
-    const uint64_t row = blockIdx.x;
-    const uint64_t ml = a.part_ml + 8 * row * a.nsplit, po = a.part_o + 4 * (row * a.nsplit * a.hd + d);
-    float M = -3.0e38f;
-    for (uint32_t s = 0; s < a.nsplit; s++) M = fmaxf(M, gload<float>(ml + 8 * s));
-    float L = 0.0f, o = 0.0f;
-    for (uint32_t s = 0; s < a.nsplit; s++) {
-        const float lw = gload<float>(ml + 8 * s + 4), f = lw != 0.0f ? __builtin_amdgcn_exp2f(gload<float>(ml + 8 * s) - M) : 0.0f;
-        const float v = gload<float>(po + 4ull * s * a.hd);
-        L += lw * f;
-        o += f != 0.0f ? v * f : 0.0f;
+    const uint64_t row = blockIdx.x, po = a.part_o + 4 * (row * ns * a.hd + d);
+    float v[8];
+#pragma unroll
+    for (uint32_t s = 0; s < 8; s++) v[s] = s < ns ? gload<float>(po + 4ull * s * a.hd) : 0.0f;
+    if (d < 64) {
+        const float2 ml = d < ns ? gload<float2>(a.part_ml + 8 * (row * ns + d)) : make_float2(-3.0e38f, 0.0f);
+        const float M = wave_max_v(ml.x, d), f = ml.y != 0.0f ? __builtin_amdgcn_exp2f(ml.x - M) : 0.0f;
+        wt[d] = f;
+        const float L = wave_sum_v(ml.y * f, d);
+        if (d == 0) den = L;
     }
-    gstore<float>(a.o + 4 * (row * a.hd + d), o / L);
+    __syncthreads();
+    float o = 0.0f;
+    for (uint32_t s0 = 0; s0 < ns; s0 += 8) {
+#pragma unroll
+        for (uint32_t s = 0; s < 8; s++)
+            if (s0 + s < ns && wt[s0 + s] != 0.0f) o += v[s] * wt[s0 + s];
+#pragma unroll
+        for (uint32_t s = 0; s < 8; s++) v[s] = s0 + 8 + s < ns ? gload<float>(po + 4ull * (s0 + 8 + s) * a.hd) : 0.0f;
+    }
+    gstore<float>(a.o + 4 * (row * a.hd + d), o / den);
 }

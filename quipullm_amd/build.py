@@ -1,6 +1,6 @@
 """Builds the native parts in-tree (quipullm_amd/lib/):
 
-* quipu_kernels.hsaco, quipu_small.hsaco, quipu_attn.hsaco -- the gfx950 kernels (hipcc --genco), loaded with hipModuleLoad;
+* quipu_kernels.hsaco, quipu_{small,attn,tile}.hsaco -- the gfx950 kernels (hipcc --genco), loaded with hipModuleLoad;
 * libquipu.so         -- the C ABI of include/quipu.h (HIP runtime, op table);
 * quipu_napi.node     -- the Node.js (N-API) addon over libquipu.so, for the JavaScript host.
 
@@ -23,7 +23,7 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 NODE_INC = "/usr/include/node"
 
 HSACO = os.path.join(LIB, "quipu_kernels.hsaco")
-OBJECTS = ("kernels", "small", "attn")   # qp_<name>.hip -> quipu_<name>.hsaco
+OBJECTS = ("kernels", "small", "attn", "tile")   # qp_<name>.hip -> quipu_<name>.hsaco
 SO = os.path.join(LIB, "libquipu.so")
 NAPI = os.path.join(LIB, "quipu_napi.node")
 

@@ -14,23 +14,7 @@
 // exchange of the four lane groups (v_permlane32_swap, v_permlane16_swap) gives lane group g the g-th dword of every
 // chunk, its operand of the instruction: inputs 4g..4g+3 and 16+4g..16+4g+3 of each 32.  X is read as operands made
 // once by qp_split_f16 in that order.  The K slices of a workgroup's wavefronts are added through LDS at the end.
-#include "qp_common.h"
-
-#define KERNEL extern "C" __global__
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// X as operands: for each tile of 16 rows and chunk of 256 inputs, 8 steps of 32 inputs x (high, low) x 64 lanes x 16
-// bytes, then one operand of the chunk's 16 sums of 16 inputs (lane groups 0, 1: their high parts, 2, 3: low parts).
-// Lane g * 16 + m of step j holds row m's inputs 32 j + {4g, 4g + 2, 4g + 1, 4g + 3, 16 + 4g, 18 + 4g, 17 + 4g,
-// 19 + 4g}.  The chunks' scales (one float per row and chunk: the stored values times it are X) follow all tiles.
-constexpr uint32_t XF_CHUNK = 17 * 1024;
-
-QP_DEV uint32_t xf_row(uint32_t row, uint32_t nch) { return (row >> 4) * nch * XF_CHUNK + (row & 15) * 16; }
-
-QP_DEV h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
+#include "qp_ints.h"
 
 // A workgroup per (chunk, tile), each of its four wavefronts 64 inputs of the 16 rows.
 KERNEL __launch_bounds__(256) void qp_split_f16(QpSplitArgs a) {
@@ -46,7 +30,26 @@ KERNEL __launch_bounds__(256) void qp_split_f16(QpSplitArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const uint32_t k = ch * 256 + wave * 64 + j * 16 + 4 * g;
-        v[j] = row < rows && k < a.k ? gload<float4>(a.x + 4 * ((uint64_t)row * a.k + k)) : make_float4(0, 0, 0, 0);
+        v[j] = make_float4(0, 0, 0, 0);
+        if (row >= rows || k >= a.k) continue;
+        if (a.mode == 2) {
+            const uint64_t at = a.x + ((uint64_t)((k >> 5) * 4 + ((k >> 3) & 3)) * a.prows + row) * 16 + (k & 7) * 2;
+            const uint2 h = gload<uint2>(at), l = gload<uint2>(at + 2ull * a.prows * a.k);
+            v[j] = make_float4(__uint_as_float(h.x << 16) + __uint_as_float(l.x << 16),
+                               __uint_as_float(h.x & 0xffff0000u) + __uint_as_float(l.x & 0xffff0000u),
+                               __uint_as_float(h.y << 16) + __uint_as_float(l.y << 16),
+                               __uint_as_float(h.y & 0xffff0000u) + __uint_as_float(l.y & 0xffff0000u));
+            continue;
+        }
+        v[j] = gload<float4>(a.x + 4 * ((uint64_t)row * a.k + k));
+        if (a.mode == 1) {
+            float* f = &v[j].x;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const __bf16 h = (__bf16)f[i];
+                f[i] = (float)h + (float)(__bf16)(f[i] - (float)h);
+            }
+        }
     }
     float mx = 0.0f;
 #pragma unroll
@@ -62,7 +65,8 @@ KERNEL __launch_bounds__(256) void qp_split_f16(QpSplitArgs a) {
     if (mx == 0.0f) e = 9;
     if (e < -117) e = -117;
     const float up = __uint_as_float((uint32_t)(9 - e + 127) << 23);
-    const uint64_t base = a.xs + ((uint64_t)blockIdx.y * nch + ch) * XF_CHUNK + lane * 16;
+    const uint64_t base = a.xs + ((uint64_t)blockIdx.y * nch + ch) * XF_CHUNK + (a.mul ? m * 128 + g * 16 : lane * 16);
+    const uint32_t low = a.mul ? XF_LOW : 1024;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const float s[8] = {v[2 * j].x * up, v[2 * j].z * up, v[2 * j].y * up, v[2 * j].w * up,
@@ -75,7 +79,7 @@ KERNEL __launch_bounds__(256) void qp_split_f16(QpSplitArgs a) {
             lo[i] = (_Float16)(d == d ? d : 0.0f);  // (an infinite value has no remainder)
         }
         gstore<h8>(base + (wave * 2 + j) * 2048, hi);
-        gstore<h8>(base + (wave * 2 + j) * 2048 + 1024, lo);
+        gstore<h8>(base + (wave * 2 + j) * 2048 + low, lo);
         float s0 = (s[0] + s[1]) + (s[2] + s[3]), s1 = (s[4] + s[5]) + (s[6] + s[7]);
         s0 += bfly_f<4>(s0, lane);
         s1 += bfly_f<4>(s1, lane);
@@ -116,184 +120,41 @@ QP_DEV u32x4 sk_transpose(u32x4 v) {
 // The dword of lane `from` / 4.
 QP_DEV uint32_t sk_from(uint32_t v, uint32_t from) { return (uint32_t)__builtin_amdgcn_ds_bpermute((int)from, (int)v); }
 
-// Two bytes of w as f16 times 2^-SH (-5 <= SH <= 6) plus off * 2^-SH: the byte in the low mantissa bits
-// of a power of two (1024 at SH = 0), which the addition takes away.
-template <int SH>
-QP_DEV h2 sk_dup(uint32_t w, uint32_t sel, float off = 0.0f) {
-    constexpr uint32_t top = 0x64u - SH * 4;  // high byte of 2^(10 - SH)
-    constexpr float unit = SH >= 0 ? 1.0f / (1 << (SH > 0 ? SH : 0)) : (float)(1 << (SH < 0 ? -SH : 0));
-    const float c = (off - 1024.0f) * unit;
-    const h2 o = {(_Float16)c, (_Float16)c};
-    return as_h2(__builtin_amdgcn_perm(top * 0x01010101u, w, sel)) + o;
-}
-constexpr uint32_t sk_sel(int i, int j) { return 0x04000400u | (uint32_t)i | ((uint32_t)j << 16); }
-
-// The quants stay where they are in the low 10 bits of a half, which as f16 is a subnormal: value * 2^-24 times the
-// power of two of their position (exact).  The scale they are multiplied by takes the position's power away and carries
-// 32 times the power of two SkK::UP, so that the products are normal f16: the matrix instructions take subnormal
-// operands, but align them as if their leading bit were set, and drop the low bits of the sum (Q2_K 4e-6 off instead of
-// 3e-7 at K = 1024).  The block's f32 scale takes all of it away.
-
-// ------------------------------------------------------------------ K-quants
-template <int FMT> struct SkK;
-template <> struct SkK<QP_Q4_K> { static constexpr int NC = 9, HDR = 0, RB = 144, UP = 2; static constexpr bool MIN = true, LO = false; };
-template <> struct SkK<QP_Q5_K> { static constexpr int NC = 11, HDR = 0, RB = 176, UP = 2; static constexpr bool MIN = true, LO = false; };
-template <> struct SkK<QP_Q6_K> { static constexpr int NC = 13, HDR = 12, RB = 208, UP = 0; static constexpr bool MIN = true, LO = true; };
-template <> struct SkK<QP_Q3_K> { static constexpr int NC = 7, HDR = 6, RB = 112, UP = 2; static constexpr bool MIN = false, LO = false; };
-template <> struct SkK<QP_Q2_K> { static constexpr int NC = 5, HDR = 0, RB = 80, UP = 4; static constexpr bool MIN = true, LO = false; };
-
 // One block of one row, from the point of view of a lane: its dwords t[chunk] of the data chunks and the whole header.
-// The block is d * 2^(19 - UP) * sum(step products) - dmin * sum(mins * sums of 16 inputs).
 template <int FMT>
-struct SkBlock {
+struct SkBlock : SkScales<FMT> {
     uint32_t t[SkK<FMT>::NC];
-    uint32_t h[4];    // the header chunk
-    uint32_t sc[4];   // scales times 2^UP: Q4_K/Q5_K sub-blocks 0..7 in sc[0..1] (minima in sc[2..3]); others 16 bytes
-    uint32_t dd;      // Q6_K: d, Q2_K: d, dmin (the arrays after the rows)
 
-    QP_DEV void setup() {
-        if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) {
-            sc[0] = (h[1] << 2) & 0xfcfcfcfcu;
-            sc[1] = ((h[3] << 2) & 0x3c3c3c3cu) | (h[1] & 0xc0c0c0c0u);
-            sc[2] = h[2] & 0x3f3f3f3fu;
-            sc[3] = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-        } else if constexpr (FMT == QP_Q6_K) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) sc[i] = h[i] ^ 0x80808080u;
-        } else if constexpr (FMT == QP_Q3_K) {
-            const uint32_t k1 = 0xc0c0c0c0u, k2 = 0x3c3c3c3cu;
-            sc[0] = ((h[0] << 2) & k2) | ((h[2] << 6) & k1);
-            sc[1] = ((h[1] << 2) & k2) | ((h[2] << 4) & k1);
-            sc[2] = ((h[0] >> 2) & k2) | ((h[2] << 2) & k1);
-            sc[3] = ((h[1] >> 2) & k2) | (h[2] & k1);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; i++) sc[i] = (h[i] << 4) & 0xf0f0f0f0u;
-        }
-    }
-    QP_DEV float d() const {
-        if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) return h2f(h[0]);
-        else if constexpr (FMT == QP_Q3_K) return h2f(h[3]);
-        else return h2f(dd);
-    }
-    QP_DEV float dmin() const {
-        if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) return h2f(h[0] >> 16);
-        else if constexpr (FMT == QP_Q2_K) return h2f(dd >> 16);
-        else return h2f(dd);  // Q6_K: d * 32 * scale is taken from every input
-    }
-    // The minima's operand: lane groups 0 and 2: of the first eight sums of 16 inputs, 1 and 3: of the others.
-    QP_DEV h8 mins(uint32_t g) const {
-        h2 v[4];
-        if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) {
-            const uint32_t m = (g & 1) ? sc[3] : sc[2];
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = sk_dup<0>(m, sk_sel(i, i));
-        } else {
-            const uint32_t a = (g & 1) ? (FMT == QP_Q6_K ? sc[2] : h[2]) : (FMT == QP_Q6_K ? sc[0] : h[0]);
-            const uint32_t b = (g & 1) ? (FMT == QP_Q6_K ? sc[3] : h[3]) : (FMT == QP_Q6_K ? sc[1] : h[1]);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t w = i < 2 ? a : b, sel = sk_sel(2 * (i & 1), 2 * (i & 1) + 1);
-                if constexpr (FMT == QP_Q6_K) v[i] = sk_dup<-5>(w, sel, -128.0f);  // 32 times the scale
-                else v[i] = sk_dup<0>((w >> 4) & 0x0f0f0f0fu, sel);
-            }
-        }
-        h8 r;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            r[2 * i] = v[i][0];
-            r[2 * i + 1] = v[i][1];
-        }
-        return r;
-    }
-    // scale * quant * 2^(UP - 19) of this lane's eight inputs of step j (32 inputs), as f16 (lo: what is left of Q6_K's
-    // products, which reach 8064).
+    // The products of this lane's eight inputs of step j (32 inputs).
     template <int j>
     QP_DEV void step(h8& hi, h8& lo) const {
-        h2 q[4], s[2];
-        if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) {
-            constexpr int c = (FMT == QP_Q4_K ? 1 : 3) + 2 * (j >> 1), at = (j & 1) * 4;
-            s[0] = s[1] = sk_dup<at - 5>(sc[j >> 2], sk_sel(j & 3, j & 3));
+        using S = SkStep<FMT, j>;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)];
-                uint32_t v = w & (0x000f000fu << at);
-                if constexpr (FMT == QP_Q5_K) {  // bit j of the fifth bits' byte, to bit 4 of the quant
-                    constexpr int up = 4 + at - j;
-                    const uint32_t hb = t[1 + (i >> 1)];
-                    const uint32_t x = (i & 1) ? (up >= 8 ? hb << (up >= 8 ? up - 8 : 0) : hb >> (up >= 8 ? 0 : 8 - up))
-                                               : (up >= 0 ? hb << (up >= 0 ? up : 0) : hb >> (up >= 0 ? 0 : -up));
-                    v |= x & (0x00100010u << at);
-                }
-                q[i] = as_h2(v) * s[0];
+        for (int i = 0; i < 2; i++) {
+            h2 q[2], l[2];
+            sk_quad<FMT, j>(t[S::CHUNK + i], S::HIGH >= 0 ? t[S::HIGH + i] : 0u, this->template scale<j, S::AT>(i), q, l);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                hi[4 * i + k] = q[k >> 1][k & 1];
+                if constexpr (FMT == QP_Q6_K) lo[4 * i + k] = l[k >> 1][k & 1];
             }
-        } else if constexpr (FMT == QP_Q2_K) {
-            constexpr int c = 1 + 2 * (j >> 2), at = 2 * (j & 3);
-#pragma unroll
-            for (int i = 0; i < 2; i++) s[i] = sk_dup<at - 5>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3));
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)];
-                q[i] = as_h2(w & (0x00030003u << at)) * s[i >> 1];
-            }
-        } else if constexpr (FMT == QP_Q3_K) {
-            constexpr int c = 2 + 2 * (j >> 2), at = 2 * (j & 3), up = 2 + at - j;  // third bit: bit j of its byte
-            h2 o[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                s[i] = sk_dup<at - 5>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3), -128.0f);
-                const float m4 = -4.0f * (1 << at) * 0x1p-24f;
-                o[i] = s[i] * h2{(_Float16)m4, (_Float16)m4};
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)], hb = t[i >> 1];
-                const uint32_t x = (i & 1) ? (up >= 8 ? hb << (up >= 8 ? up - 8 : 0) : hb >> (up >= 8 ? 0 : 8 - up))
-                                           : (up >= 0 ? hb << (up >= 0 ? up : 0) : hb >> (up >= 0 ? 0 : -up));
-                const uint32_t v = (w & (0x00030003u << at)) | (x & (0x00040004u << at));
-                q[i] = __builtin_elementwise_fma(as_h2(v), s[i >> 1], o[i >> 1]);  // (q - 4) scale, exact
-            }
-        } else {
-            constexpr int hh = j >> 2, qd = j & 3, c = 4 * hh + (qd & 1) * 2, at = (qd >> 1) * 4, up = 4 + at - 2 * qd;
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                s[i] = sk_dup<at - 5>(sc[(2 * j + i) >> 2], sk_sel((2 * j + i) & 3, (2 * j + i) & 3), -128.0f);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t w = (i & 1) ? t[c + (i >> 1)] >> 8 : t[c + (i >> 1)], hb = t[8 + 2 * hh + (i >> 1)];
-                const uint32_t x = (i & 1) ? (up >= 8 ? hb << (up >= 8 ? up - 8 : 0) : hb >> (up >= 8 ? 0 : 8 - up))
-                                           : (up >= 0 ? hb << (up >= 0 ? up : 0) : hb >> (up >= 0 ? 0 : -up));
-                const h2 v = as_h2((w & (0x000f000fu << at)) | (x & (0x00300030u << at)));
-                q[i] = v * s[i >> 1];
-                const h2 r = __builtin_elementwise_fma(v, s[i >> 1], -q[i]);
-                lo[2 * i] = r[0];
-                lo[2 * i + 1] = r[1];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            hi[2 * i] = q[i][0];
-            hi[2 * i + 1] = q[i][1];
         }
     }
 };
-
-QP_DEV f32x4 sk_mfma(h8 a, h8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
 // The X operands of one step for the NT token tiles.
 template <int NT>
 struct SkX {
     h8 hi[NT], lo[NT];
-    QP_DEV void load(__amdgpu_buffer_rsrc_t xr, const uint32_t* xo, uint32_t soff) {
+    QP_DEV void load(__amdgpu_buffer_rsrc_t xr, const uint32_t* xo, uint32_t soff, uint32_t low) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             hi[t] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[t], soff, 0));
-            lo[t] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[t], soff + 1024, 0));
+            lo[t] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[t], soff + low, 0));
         }
     }
 };
 
-template <int V> struct SkInt { static constexpr int v = V; };
 
 // Where a wavefront's weights are: a buffer resource over its rows and the offset of this lane's row.
 struct SkRows {
@@ -304,7 +165,7 @@ struct SkRows {
 // K-quants: groups of four blocks of 256 inputs, group gi0 + i * gs < gi1.
 template <int FMT, int NT, int R, class Sc>
 QP_DEV void sk_kq(const SkRows (&rw)[R], uint32_t nb, uint32_t gi0, uint32_t gi1, uint32_t gs, __amdgpu_buffer_rsrc_t xr,
-                  const uint32_t* xo, Sc&& scales, f32x4 (&tot)[R][NT]) {
+                  const uint32_t* xo, uint32_t low, Sc&& scales, f32x4 (&tot)[R][NT]) {
     using F = SkK<FMT>;
     const uint32_t g = (threadIdx.x & 63) >> 4;
     u32x4 w[R][F::NC];
@@ -329,7 +190,7 @@ QP_DEV void sk_kq(const SkRows (&rw)[R], uint32_t nb, uint32_t gi0, uint32_t gi1
     SkX<NT> x[PD];
     load(gi0);
 #pragma unroll
-    for (int j = 0; j < PD; j++) x[j].load(xr, xo, 4 * gi0 * XF_CHUNK + j * 2048);
+    for (int j = 0; j < PD; j++) x[j].load(xr, xo, 4 * gi0 * XF_CHUNK + j * 2048, low);
     for (uint32_t gi = gi0; gi < gi1; gi += gs) {
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -389,7 +250,7 @@ QP_DEV void sk_kq(const SkRows (&rw)[R], uint32_t nb, uint32_t gi0, uint32_t gi1
                             for (int t = 0; t < NT; t++) p[r][t] = sk_mfma(X.hi[t], lo, p[r][t]);
                         }
                     }
-                    X.load(xr, xo, j + PD < 8 ? so + (j + PD) * 2048 : nx * XF_CHUNK + (j + PD - 8) * 2048);
+                    X.load(xr, xo, j + PD < 8 ? so + (j + PD) * 2048 : nx * XF_CHUNK + (j + PD - 8) * 2048, low);
                     __builtin_amdgcn_sched_barrier(0xf);  // (the loads stay at their step: hoisted, they would spill)
                 };
                 step(SkInt<0>()); step(SkInt<1>()); step(SkInt<2>()); step(SkInt<3>());
@@ -423,7 +284,7 @@ QP_DEV void sk_kq(const SkRows (&rw)[R], uint32_t nb, uint32_t gi0, uint32_t gi1
 // Q8_0, IQ4_NL and f32: chunks of 256 inputs ch0 + i * cs < ch1; the scale of each 32 inputs multiplies their sums.
 template <int FMT, int NT, int R, class Sc>
 QP_DEV void sk_pl(const SkRows (&rw)[R], uint32_t K, uint32_t ch0, uint32_t ch1, uint32_t cs, __amdgpu_buffer_rsrc_t xr,
-                  const uint32_t* xo, Sc&& scales, f32x4 (&tot)[R][NT]) {
+                  const uint32_t* xo, uint32_t low, Sc&& scales, f32x4 (&tot)[R][NT]) {
     constexpr int NL = FMT == QP_F32 ? 16 : FMT == QP_Q8_0 ? 4 : 2;  // 16-byte loads per lane and chunk
     const uint32_t g = (threadIdx.x & 63) >> 4;
     const uint32_t rowb = FMT == QP_F32 ? 4 * K : FMT == QP_Q8_0 ? K : K / 2;  // bytes of a row (without scales)
@@ -465,10 +326,10 @@ QP_DEV void sk_pl(const SkRows (&rw)[R], uint32_t K, uint32_t ch0, uint32_t ch1,
         scales(ch, s);
         const uint32_t so = ch * XF_CHUNK;
         SkX<NT> x[2];
-        x[0].load(xr, xo, so);
+        x[0].load(xr, xo, so, low);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            if (j < 7) x[(j + 1) & 1].load(xr, xo, so + (j + 1) * 2048);
+            if (j < 7) x[(j + 1) & 1].load(xr, xo, so + (j + 1) * 2048, low);
             const SkX<NT>& X = x[j & 1];
 #pragma unroll
             for (int r = 0; r < R; r++) {
@@ -599,11 +460,11 @@ QP_DEV void sk_body(const QpSkArgs& a) {
         for (int t = 0; t < NT; t++) {
             if (dense) {
                 const bool in = (uint32_t)t * 16 < cnt;  // (the tile's rows past T are zeros)
-                xo[t] = in ? xf_row(t0 + t * 16, nch) + lane * 16 : QP_NOOFF;
+                xo[t] = in ? xf_tile(t0 + t * 16, nch) + lane * 16 : QP_NOOFF;
                 so[t][0] = in ? ((t0 >> 4) + t) * nch * 64 + g * 16 : QP_NOOFF;
             } else {
                 const uint32_t j = jobs[t * 16 + n16];
-                xo[t] = j == QP_NOOFF ? QP_NOOFF : xf_row(j / a.tfijo, nch) + g * 256;
+                xo[t] = j == QP_NOOFF ? QP_NOOFF : xf_tile(j / a.tfijo, nch) + ((j / a.tfijo) & 15) * 128 + g * 16;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const uint32_t ji = jobs[t * 16 + 4 * g + i], x = ji / a.tfijo;
@@ -629,8 +490,8 @@ QP_DEV void sk_body(const QpSkArgs& a) {
 #pragma unroll
             for (int t = 0; t < NT; t++) tot[r][t] = f32x4{0, 0, 0, 0};
         if (work && kw < units) {
-            if constexpr (KQ) sk_kq<FMT, NT, R>(rw, nch, kw, units, a.kw, xr, xo, scales, tot);
-            else sk_pl<FMT, NT, R>(rw, a.k, kw, units, a.kw, xr, xo, scales, tot);
+            if constexpr (KQ) sk_kq<FMT, NT, R>(rw, nch, kw, units, a.kw, xr, xo, dense ? 1024 : XF_LOW, scales, tot);
+            else sk_pl<FMT, NT, R>(rw, a.k, kw, units, a.kw, xr, xo, dense ? 1024 : XF_LOW, scales, tot);
         }
         // the K slices' sums, added in their order; wavefront kw of a row group finishes its share of the tiles
         if (a.kw > 1) {

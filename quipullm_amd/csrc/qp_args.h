@@ -143,6 +143,18 @@ typedef struct {
     uint32_t xrows, yrows, nlst, pad2;
 } QpSkArgs;
 
+// qp_tile_<fmt>, qp_tile_glu_<fmt> (K-quants, qp_tile.hip): 128 x 128 tiles, mt x nt of them (grouped by expert, lst != 0:
+// at most mt tiles of 128 jobs in nexp experts) in grid x (a multiple of 8), grid z K splits of kb blocks of 256 inputs.
+// xs: X as operands (qp_split_f16) of `rows` rows.  ws: 0, or the splits' sums [splits][rows][n].  glu: w gate, w2 up, 64
+// rows of each per tile; yplanes: 0, or y receives the next matmul's input planes of that many token rows.
+typedef struct {
+    uint64_t w, w2, xs, y, ws, paso, lst, off, wrows;
+    uint32_t n, k, acc, rows;
+    uint32_t mt, nt, kb, nexp;
+    uint32_t tfijo, xrows, yrows, nlst;
+    uint32_t yplanes, pad;
+} QpTileArgs;
+
 // moe_group: lst[off[e] .. off[e + 1]) = the jobs i < T * n (in increasing order) with sel[i] == e, e < n_exp;
 // off[n_exp] = the number listed.  nsel: entries of sel and lst that exist.
 typedef struct {
@@ -152,7 +164,9 @@ typedef struct {
 // x [T][k] -> bf16 high / low planes (hi = bf16(v), lo = bf16(v - hi)) at xs and xs + 2*rows*k.  mul != 0: the
 // first min(T * mul, cap) rows of x instead of T, in row-major planes ([rows][k rounded up to 32]: the grouped
 // expert matmul, whose tiles gather rows), not the chunk-quarter layout of the 256-token tiles.
-typedef struct { uint64_t x, xs, paso; uint32_t k, rows, mul, cap; } QpSplitArgs;
+// qp_split_f16 (the integer-weight matmuls' operands) takes the same: mul as there; mode 0: X to 22 bits, 1: X as its bf16
+// high + low parts first, 2: x holds those parts (qp_split_bf16's planes of prows token rows).
+typedef struct { uint64_t x, xs, paso; uint32_t k, rows, mul, cap, mode, prows; } QpSplitArgs;
 // y[t][n] = (acc ? y : 0) + sum over s (in order) of ws[s][t][n].
 typedef struct { uint64_t ws, y, paso; uint32_t n, rows, splits, acc; } QpReduceArgs;
 

@@ -79,32 +79,39 @@ enum Kid {
 #define K(name) K_##name,
 #define M(name) K_##name,
 #define A(name) K_##name,
+#define T(name) K_##name,
 #include "qp_kernel_list.inc"
 #undef K
 #undef M
 #undef A
+#undef T
     K_COUNT
 };
 const char* kNames[] = {
 #define K(name) "qp_" #name,
 #define M(name) "qp_" #name,
 #define A(name) "qp_" #name,
+#define T(name) "qp_" #name,
 #include "qp_kernel_list.inc"
 #undef K
 #undef M
 #undef A
+#undef T
 };
 // The code objects (beside each other; one source file each) and which of them holds a kernel.
-constexpr int kObjects = 3;
-const char* kObjectNames[kObjects] = {"quipu_kernels.hsaco", "quipu_small.hsaco", "quipu_attn.hsaco"};
+constexpr int kObjects = 4;
+const char* kObjectNames[kObjects] = {"quipu_kernels.hsaco", "quipu_small.hsaco", "quipu_attn.hsaco",
+                                        "quipu_tile.hsaco"};
 const uint8_t kObject[] = {
 #define K(name) 0,
 #define M(name) 1,
 #define A(name) 2,
+#define T(name) 3,
 #include "qp_kernel_list.inc"
 #undef K
 #undef M
 #undef A
+#undef T
 };
 hipFunction_t g_fn[K_COUNT];
 
@@ -439,7 +446,7 @@ int workspace(uint64_t bytes, uint64_t* out) {
 struct SplitMemo {
     uint64_t x, xs, paso;
     uint32_t k, rows, mul, cap, gen;
-    bool ints;  // qp_split_f16's operands, not qp_split_bf16's planes
+    int ints;  // -1: qp_split_bf16's planes, else qp_split_f16's operands of that mode
     bool valid;
 } g_split_memo = {};
 // While a graph is captured nothing runs, so a split recorded then proves nothing about the planes' contents now,
@@ -447,14 +454,14 @@ struct SplitMemo {
 // and graph launches invalidate it.
 // mul, cap: rows T * mul of x, at most cap (QpSplitArgs); 0: T rows.
 int split_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse,
-                uint32_t mul = 0, uint32_t cap = 0, bool ints = false) {
+                uint32_t mul = 0, uint32_t cap = 0, int ints = -1, uint32_t prows = 0) {
     const SplitMemo& m = g_split_memo;
     if (reuse && !g_capturing && m.valid && m.x == x && m.xs == xs && m.paso == paso && m.k == K && m.rows == rows &&
         m.mul == mul && m.cap == cap && m.gen == g_ws_gen && m.ints == ints)
         return 0;
-    QpSplitArgs sa = {x, xs, paso, K, rows, mul, cap};
+    QpSplitArgs sa = {x, xs, paso, K, rows, mul, cap, ints < 0 ? 0u : (uint32_t)ints, prows};
     g_split_memo = {x, xs, paso, K, rows, mul, cap, g_ws_gen, ints, false};
-    if (int e = ints ? launch(K_split_f16, cdiv(K, 256), rows / 16, 1, 256, 0, sa)
+    if (int e = ints >= 0 ? launch(K_split_f16, cdiv(K, 256), rows / 16, 1, 256, 0, sa)
                      : launch(K_split_bf16, grid_cap((uint64_t)tmax * K / 8), 1, 1, 256, 0, sa))
         return e;
     g_split_memo.valid = !g_capturing;
@@ -463,7 +470,7 @@ int split_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t row
 
 // ---- integer-weight matmul of few token rows (qp_small.hip): X as operands, 16 R weight rows per wavefront.
 // Bytes of the operands and scales of `rows` rows (a multiple of 16) of K inputs.
-uint64_t sk_bytes(uint32_t rows, uint32_t K) { return (uint64_t)(rows / 16) * cdiv(K, 256) * (17 * 1024 + 64); }
+uint64_t sk_bytes(uint32_t rows, uint32_t K) { return (uint64_t)(rows / 16) * cdiv(K, 256) * (18 * 1024 + 64); }
 
 Kid sk_kid(int fmt, uint32_t nt, uint32_t R) {
 #define SK_R1(F) {K_sk_##F##_t1r1, K_sk_##F##_t2r1, K_sk_##F##_t4r1}
@@ -491,15 +498,17 @@ int run_sk(int fmt, QpSkArgs& a, uint32_t nt, uint32_t tpe, uint32_t E, uint32_t
 
 // The dense matmuls that take this path (the others: the 128- and 256-token tiles of op_matmul_mt), by the tokens the
 // dispatch covers, measured with weights past the last-level cache, this path against the tiles in us:
-//   K-quants below 256 tokens: Q4_K 14336 x 4096 at 64 / 128 / 192 tokens 43 / 79 / 117 against 79 / 87 / 149, Q6_K
-//     4096 x 14336 66 / 100 / 180 against 105 / 119 / 173; at 256 tokens 144 against 129 (14336 x 4096);
+//   K-quants up to 64 tokens, and below 256 where the matrix is small (qp_tile.hip's tiles then run in K splits whose
+//     sums are added after): this path against those tiles at 65 / 128 / 129 / 192 tokens Q4_K 14336 x 4096 72 / 81 /
+//     109 / 114 against 58 / 65 / 94 / 99, Q6_K 4096 x 14336 89 / 94 / 161 / 170 against 82 / 89 / 150 / 153; Q4_K
+//     4096 x 4096 24 / 26 / 41 / 43 against 32 / 34 / 41 / 43, 1024 x 4096 19 / 21 / 21 / 23 against 27 / 29 / 30 / 30;
 //   Q8_0 and IQ4_NL (whose sums are scaled every 32 inputs) up to 64 tokens, and below 256 where the product is small:
 //     Q8_0 11008 x 4096 at 64 / 128 tokens 59 / 103 against 66 / 73; 2816 x 1024 at 256 tokens 21 against 30;
 //   f32 always: 128 x 2048 (a router) at 64 / 2048 tokens 26 / 34 against 38 / 50, 4096 x 4096 49 / 689 against 71 / 738.
 // Below 64 tokens the other path is the vector-unit kernel (Q4_K 14336 x 4096 at 32 tokens 27 against 1120).
 bool sk_takes(int fmt, uint32_t tmax, uint32_t N, uint32_t K) {
     if (fmt == QP_F32) return true;
-    if (is_kq(fmt)) return tmax < 256;
+    if (is_kq(fmt)) return tmax <= 64 || (tmax < 256 && (uint64_t)N * K < 32u << 20);
     return tmax <= 64 || (tmax < 256 && (uint64_t)N * K * cdiv(tmax, 64) <= 12u << 20);
 }
 // 16-row tiles per wavefront: two where that leaves enough workgroups (X is read once per 16 R rows): 8192 rows times
@@ -509,6 +518,20 @@ uint32_t sk_rows(int fmt, uint32_t nt, uint32_t yb, uint32_t N) {
     if (planar(fmt)) return 1;
     if (fmt == QP_F32) return nt == 4 && (uint64_t)N * yb >= 4096 ? 2 : 1;
     return (uint64_t)N * yb >= 8192 ? 2 : 1;
+}
+
+// K-quant matmuls of many token rows (qp_tile.hip): 128 x 128 tiles, two workgroups per CU.
+int run_tile(int fmt, QpTileArgs& a, bool glu, uint32_t ns) {
+    static const Kid kt[2][5] = {{K_tile_q4k, K_tile_q5k, K_tile_q6k, K_tile_q3k, K_tile_q2k},
+                                 {K_tile_glu_q4k, K_tile_glu_q5k, K_tile_glu_q6k, K_tile_glu_q3k, K_tile_glu_q2k}};
+    a.nt = cdiv(a.n, glu ? 64 : 128);
+    const uint32_t lds = 2 * 17408 + (fmt == QP_Q6_K ? 32768 : 16384) + 8192 + 4096 + 1024 + 512;  // (qp_tile.hip's)
+    return launch(kt[glu][kq_index(fmt)], 8 * cdiv((uint64_t)a.mt * a.nt, 8), 1, ns, 256, lds, a);
+}
+// X of a dense K-quant matmul's tiles as operands.  From 256 tokens on (where a caller's input planes may take the place
+// of the f32 rows: planes, rows in whole 256s) by way of the rows' bf16 high + low parts, so that both give the same bits.
+int tile_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse, bool planes) {
+    return split_input(x, xs, paso, K, rows, tmax, reuse, 0, 0, planes ? 2 : tmax >= 256 ? 1 : 0, planes ? cdiv(tmax, 256) * 256 : 0);
 }
 
 int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z) {
@@ -547,8 +570,47 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         const uint32_t nt = t1 <= 16 ? 1 : t1 <= 32 ? 2 : 4, yb = cdiv(t1, 16 * nt);
         s.rows = 16 * cdiv(t1, 16);
         if (int e = workspace(sk_bytes(s.rows, K), &s.xs)) return e;
-        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, true)) return e;
+        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, 0)) return e;
         return run_sk(fmt, s, nt, yb, 1, sk_rows(fmt, nt, yb, N));
+    }
+    const uint32_t rows16 = cdiv(t1, 16) * 16;
+    // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip), where qp_dispatch_noalloc's scratch holds
+    // X's operands.  Against the tiles below at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 108 / 183 / 340 /
+    // 597 against 133 / 224 / 383 / 720, 1024 x 4096 32 / 35 / 51 / 75 against 31 / 39 / 54 / 84; Q6_K 4096 x 14336 164 /
+    // 263 / 455 / 830 against 150 / 270 / 479 / 840; Q5_K 14336 x 4096 118 / 201 / 362 / 632 against 143 / 237 / 424 / 791.
+    if (is_kq(fmt) && tmax > 64 && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") &&
+        (!g_noalloc || sk_bytes(rows16, K) <= QP_SCRATCH_BYTES)) {
+        if (xplanes)
+            if (int e = need_room(a.x, 4ull * cdiv(t1, 256) * 256 * K, name, "the input planes' buffer")) return e;
+        QpTileArgs s = {};
+        s.w = a.w;
+        s.y = a.y;
+        s.paso = a.paso;
+        s.n = N;
+        s.k = K;
+        s.acc = acc;
+        s.wrows = N;
+        s.rows = rows16;
+        s.mt = cdiv(t1, 128);
+        const uint32_t nb = K / 256, tiles = s.mt * cdiv(N, 128), slots = 2 * (uint32_t)(g_cus > 0 ? g_cus : 1);
+        const uint64_t xs_bytes = sk_bytes(rows16, K);
+        uint32_t ns = 1;  // K splits: while the tiles leave half the places idle and a split keeps two blocks
+        while (tiles * ns * 2 <= slots && nb / (ns * 2) >= 2) ns *= 2;
+        uint64_t ws_bytes;
+        for (;;) {
+            s.kb = cdiv(nb, ns);
+            ns = cdiv(nb, s.kb);
+            ws_bytes = ns > 1 ? 4ull * ns * rows16 * N : 0;
+            if (!g_noalloc || ns == 1 || xs_bytes + ws_bytes <= QP_SCRATCH_BYTES) break;
+            ns /= 2;
+        }
+        if (int e = workspace(xs_bytes + ws_bytes, &s.xs)) return e;
+        s.ws = ns > 1 ? s.xs + xs_bytes : 0;
+        if (int e = tile_input(a.x, s.xs, a.paso, K, rows16, tmax, c.U(4) == 1, xplanes)) return e;
+        if (int e = run_tile(fmt, s, false, ns)) return e;
+        if (ns == 1) return 0;
+        QpReduceArgs ra = {s.ws, a.y, a.paso, N, rows16, ns, acc};
+        return launch(K_gemm_reduce, grid_cap((uint64_t)tmax * N), 1, 1, 256, 0, ra);
     }
     if (tmax >= 64 && !getenv_flag("QP_NO_MFMA")) {
         // matrix cores: 128 x 128 tiles (the kernel reads T from paso; tiles past it exit)
@@ -673,6 +735,29 @@ int op_matmul_glu(const Ctx& c, int fmt, const char* name) {
     if (a.yplanes) {
         if (N % 32) return fail(QP_E_ARG, "%s: the input planes need N %% 32 == 0 (N = %u)", name, N);
         if (int e = need_room(a.y, 4ull * a.rows * N, name, "the output planes' buffer")) return e;
+    }
+    const uint32_t rows16 = cdiv(tmax, 16) * 16;
+    // Integer weights in tiles of 128 tokens x (64 gate + 64 up) rows (qp_tile.hip), where qp_dispatch_noalloc's scratch
+    // holds X's operands: 14336 x 4096 of Q4_K at 2048 tokens 1208 us against 1320, of Q5_K at 333 334 against 357.
+    if (!g_noalloc || sk_bytes(rows16, K) <= QP_SCRATCH_BYTES) {
+        const bool xp = c.U(3) == 1;
+        if (xp)
+            if (int e = need_room(a.x, 4ull * a.rows * K, name, "the input planes' buffer")) return e;
+        QpTileArgs s = {};
+        s.w = a.w;
+        s.w2 = a.w2;
+        s.y = a.y;
+        s.paso = a.paso;
+        s.n = N;
+        s.k = K;
+        s.wrows = N;
+        s.rows = rows16;
+        s.mt = cdiv(tmax, 128);
+        s.kb = K / 256;
+        s.yplanes = a.yplanes ? a.rows : 0;
+        if (int e = workspace(sk_bytes(rows16, K), &s.xs)) return e;
+        if (int e = tile_input(a.x, s.xs, a.paso, K, rows16, tmax, false, xp)) return e;
+        return run_tile(fmt, s, true, 1);
     }
     // One workgroup per CU (the kernel takes the whole LDS), so the tiles run in rounds of g_cus.  When the last
     // round would leave at least half the CUs idle, its tiles run as K halves instead (two items each, the second to
@@ -1181,12 +1266,16 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
     // same planes: the sums are bit-equal).  P[5] = 1: the previous matmul split the same x (see split_input).  Not while capturing a graph or
     // under qp_dispatch_noalloc (the planes need the workspace): there x is split in the tiles as without P[4].
     const uint32_t m = c.U(4);
-    // Few jobs per expert: integer weights, 16 jobs per token tile (qp_small.hip).  Jobs per token: tfijo of the gate and
-    // up products, P[4] of the down product (8 where it says none).  128 experts of Q4_K 768 x 2048, 8 per token, the
-    // whole FFN in us against the 128-job tiles: 32 tokens 193 against 615, 512 983 against 1980, 1024 (64 jobs per
-    // expert) 2023 against 2118, 2048 4464 against 2371.
+    // Integer weights: few jobs per expert in token tiles of 16 (qp_small.hip), more of K-quants in tiles of 128 jobs x
+    // 128 rows (qp_tile.hip).  Jobs per token: tfijo of the gate and up products, P[4] of the down product (8 where it
+    // says none).  128 experts of Q4_K 768 x 2048, 8 per token, the whole FFN in us, the first against the second: 128
+    // tokens (8 jobs per expert) 252 / 492, 256 423 / 502, 384 473 / 520, 512 657 / 541; against the tiles below 32 tokens
+    // 185 / 615, 512 541 / 1980, 1024 636 / 2118, 2048 854 / 2371.  Q8_0 and IQ4_NL take the first up to 64 jobs per
+    // expert, then the tiles below.
     const uint32_t per_tok = tfijo > 1 ? tfijo : m ? m : 8;
-    if (!g_capturing && !g_noalloc && !getenv_flag("QP_NO_MFMA") && 32ull * tz * per_tok <= 64ull * E) {
+    const uint64_t max_jobs = 32ull * tz * per_tok;
+    const bool few = (max_jobs < a.nlst ? max_jobs : a.nlst) <= (is_kq(fmt) ? 24ull : 64ull) * E;
+    if (!g_capturing && !g_noalloc && !getenv_flag("QP_NO_MFMA") && (few || is_kq(fmt))) {
         // (without P[4]: every row of x that a job of y can read)
         const uint64_t rows = m ? (uint64_t)32 * tz * m : ((uint64_t)a.yrows + tfijo - 1) / tfijo;
         QpSkArgs s = {};
@@ -1205,8 +1294,28 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
         s.xrows = (uint32_t)(rows < a.xrows ? rows : a.xrows);
         s.rows = cdiv(s.xrows, 16) * 16;
         if (int e = workspace(sk_bytes(s.rows, K), &s.xs)) return e;
-        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, s.rows, c.U(5) == 1, m ? m : s.xrows, s.xrows, true)) return e;
-        return run_sk(fmt, s, 1, a.tpe, E, is_kq(fmt) ? 2 : 1);
+        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, s.rows, c.U(5) == 1, m ? m : s.xrows, s.xrows, 0)) return e;
+        if (few) return run_sk(fmt, s, 1, a.tpe, E, is_kq(fmt) ? 2 : 1);
+        QpTileArgs q = {};
+        q.w = s.w;
+        q.xs = s.xs;
+        q.y = s.y;
+        q.paso = s.paso;
+        q.lst = s.lst;
+        q.off = s.off;
+        q.wrows = s.wrows;
+        q.n = N;
+        q.k = K;
+        q.acc = acc;
+        q.rows = s.rows;
+        q.mt = s.nlst / 128 + E;  // the list's whole 128s and a tile more per expert
+        q.nexp = E;
+        q.kb = K / 256;
+        q.tfijo = tfijo;
+        q.xrows = s.xrows;
+        q.yrows = s.yrows;
+        q.nlst = s.nlst;
+        return run_tile(fmt, q, false, 1);
     }
     if (m && !g_capturing && !g_noalloc) {
         if (K % 8) return fail(QP_E_ARG, "%s: input planes need K %% 8 == 0", name);

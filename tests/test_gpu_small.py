@@ -116,6 +116,79 @@ def test_few_jobs_per_expert(quipu, dev, oracle, fmt):
             assert np.all(np.abs(outs[0][j] - (xr.astype(np.float64) @ W[e].T)[0]) <= bound(W[e], xr)[0]), j
 
 
+def split_bound(W, x):
+    """x read as its bfloat16 high + low parts, each input off by at most 2^-18 of itself, roundings of either sign."""
+    return bound(W, x) + 4 * 2.0 ** -18 * np.sqrt(x.astype(np.float64) ** 2 @ (W ** 2).T)
+
+
+KQ = [f for f in FMTS if f not in PLANAR and f != capi.F32]
+
+
+@pytest.mark.parametrize("fmt", KQ)
+@pytest.mark.parametrize("T,N,K", [(256, 128, 256), (257, 1, 512), (321, 129, 768), (383, 250, 1280), (448, 64, 2304),
+                                   (70, 8200, 4096)])
+def test_many_tokens(quipu, dev, oracle, fmt, T, N, K):
+    """The 128 x 128 tiles: whole ones, one row, one token and one row past a tile, tiles of at most 64 tokens, one block of
+    256 inputs, K splits with a shorter last one; a large matrix below 256 tokens."""
+    if N > 8000 and fmt != capi.Q4_K:
+        pytest.skip("one format is enough for the large matrix")
+    raw = raw_matrix(fmt, N, K, 81)
+    W = weights(oracle, fmt, raw, N, K)
+    rng = np.random.default_rng(82)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    y0 = rng.standard_normal((T, N)).astype(np.float32) if T % 2 else None
+    got = matmul(quipu, dev, fmt, raw, N, K, x, y0)
+    want = x.astype(np.float64) @ W.T + (0 if y0 is None else y0)
+    assert np.all(np.abs(got - want) <= split_bound(W, x) + (0 if y0 is None else 2.0 ** -23 * np.abs(y0)))
+
+
+@pytest.mark.parametrize("fmt", KQ)
+@pytest.mark.parametrize("T,N,K", [(256, 64, 256), (300, 97, 768), (390, 200, 512)])
+def test_many_tokens_swiglu(quipu, dev, oracle, fmt, T, N, K):
+    """matmul_<fmt>_t_swiglu: silu(g) u of the two products; |silu'| < 1.1, and 2^-20 for the exponential, the division and
+    the product."""
+    raw = [raw_matrix(fmt, N, K, 83 + i) for i in range(2)]
+    W = [weights(oracle, fmt, r, N, K) for r in raw]
+    x = (np.random.default_rng(85).standard_normal((T, K)) / np.sqrt(K) / np.abs(W[0]).max()).astype(np.float32)
+    y = dev.buf(np.full((T + 1, N), 7.0, np.float32))
+    quipu.dispatch("matmul_%s_t_swiglu" % capi.FMT_NAME[fmt], [("u", N), ("u", K)],
+                   [dev.paso(T, 0)] + [dev.matrix(fmt, r, N, K) for r in raw] + [dev.buf(x), y], (1, 1, (T + 31) // 32))
+    got = dev.get(y, (T + 1, N))
+    assert np.all(got[T] == 7.0)
+    g, u = (x.astype(np.float64) @ w.T for w in W)
+    silu = g / (1 + np.exp(-g))
+    bg, bu = (split_bound(w, x) for w in W)
+    assert np.all(np.abs(got[:T] - silu * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(silu) * bu + 2.0 ** -20 * np.abs(silu * u))
+
+
+@pytest.mark.parametrize("fmt", KQ)
+def test_many_jobs_per_expert(quipu, dev, oracle, fmt):
+    """matmul_<fmt>_eg in tiles of 128 jobs: more than 64 experts (their counts are scanned 64 at a time), some without jobs,
+    one with every token, others with a few or just over 128; the same bits with and without P[4]."""
+    E, N, K, k, T = 70, 130, 512, 3, 700
+    rng = np.random.default_rng(86)
+    sel = np.stack([np.concatenate([[66], rng.permutation(8)[:2] * 9]) for _ in range(T)]).astype(np.uint32).ravel()
+    raw = raw_matrix(fmt, E * N, K, 87)
+    W = weights(oracle, fmt, raw, E * N, K).reshape(E, N, K)
+    hw = dev.matrix(fmt, raw, E * N, K)
+    sb, lb, ob = dev.buf(sel), dev.zeros(4 * T * k), dev.zeros(4 * (E + 1))
+    p = dev.paso(T, 0)
+    quipu.dispatch("moe_group", [("u", E), ("u", k)], [p, sb, lb, ob])
+    for tfijo, m in ((k, 1), (1, k)):
+        x = rng.standard_normal((T * k // tfijo, K)).astype(np.float32)
+        xb, outs = dev.buf(x), []
+        for extra in ([("u", m), ("u", 0)], []):
+            y = dev.zeros(4 * T * k * N)
+            quipu.dispatch("matmul_%s_eg" % capi.FMT_NAME[fmt], [("u", N), ("u", K), ("u", 0), ("u", tfijo)] + extra,
+                           [p, hw, xb, y, lb, ob], ((N + 63) // 64, E, (T + 31) // 32))
+            outs.append(dev.get(y, (T * k, N)))
+        assert np.array_equal(outs[0], outs[1])
+        for e in np.unique(sel):
+            js = np.flatnonzero(sel == e)
+            xe = x[js // tfijo]
+            assert np.all(np.abs(outs[0][js] - xe.astype(np.float64) @ W[e].T) <= bound(W[e], xe)), e
+
+
 @pytest.mark.parametrize("f16", [0, 1])
 @pytest.mark.parametrize("hd,nh,nkv,T,pos0,swa,cap", [
     (128, 8, 8, 1, 0, 0, 0),          # one key

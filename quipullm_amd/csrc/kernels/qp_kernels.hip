@@ -4833,70 +4833,149 @@ QP_DEV float topk_val(uint64_t k) {
 }
 QP_DEV uint32_t topk_id(uint64_t k) { return 0xffffffffu - (uint32_t)k; }
 
-// Descending bitonic sort of n (a power of two) keys in LDS by nt threads.
-QP_DEV void bitonic_desc(uint64_t* s, uint32_t n, uint32_t tid, uint32_t nt) {
-    for (uint32_t size = 2; size <= n; size <<= 1)
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            for (uint32_t t = tid; t < n / 2; t += nt) {
-                const uint32_t i = 2 * t - (t & (stride - 1)), j = i + stride;
-                const uint64_t x = s[i], y = s[j];
-                if ((i & size) == 0 ? x < y : x > y) {
-                    s[i] = y;
-                    s[j] = x;
-                }
-            }
-            __syncthreads();
+// The largest keys of a workgroup, C per thread in registers (o: the value's word, lo: the id's; both 0: no key; from
+// nc on none): returns T, L such that the kp largest are those with o > T or (o == T and lo >= L) (all keys, when there
+// are no more than kp).  T is found two bits at a time from counts of the keys at or above three candidates, down to
+// the bit where exactly kp are, L likewise and only where equal values straddle the limit.  cnt: 33 words of LDS, zero (and a barrier since).
+template <int C>
+QP_DEV uint2 topk_limit(const uint32_t (&o)[C], const uint32_t (&lo)[C], uint32_t nc, uint32_t kp, uint64_t* cnt) {
+    const uint32_t lane = threadIdx.x & 63;
+    // the workgroup's sum of three counts (21 bits each) per wavefront
+    auto total = [&](uint64_t v, uint32_t slot) -> uint64_t {
+        if (lane == 0) atomicAdd(reinterpret_cast<unsigned long long*>(cnt + slot), (unsigned long long)v);
+        __syncthreads();
+        return cnt[slot];
+    };
+    uint32_t T = 0, at_T = 0xffffffffu;  // keys with o >= T
+    for (int b = 30; b >= 0 && at_T != kp; b -= 2) {
+        uint32_t n[3] = {0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            if ((uint32_t)c >= nc) break;
+#pragma unroll
+            for (uint32_t i = 0; i < 3; i++) n[i] += __popcll(__ballot(o[c] >= (T | ((i + 1) << b))));
         }
+        const uint64_t t = total(n[0] | (uint64_t)n[1] << 21 | (uint64_t)n[2] << 42, (30 - b) / 2);
+        const uint32_t m = (1u << 21) - 1, t1 = t & m, t2 = (t >> 21) & m, t3 = (uint32_t)(t >> 42);
+        if (t3 >= kp) { T |= 3u << b; at_T = t3; }
+        else if (t2 >= kp) { T |= 2u << b; at_T = t2; }
+        else if (t1 >= kp) { T |= 1u << b; at_T = t1; }
+    }
+    uint32_t L = 0;
+    if (T != 0 && at_T != kp) {
+        uint32_t above = 0;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            if ((uint32_t)c >= nc) break;
+            above += __popcll(__ballot(o[c] > T));
+        }
+        const uint32_t need = kp - (uint32_t)total(above, 16);
+        for (int b = 30; b >= 0; b -= 2) {
+            uint32_t n[3] = {0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                if ((uint32_t)c >= nc) break;
+#pragma unroll
+                for (uint32_t i = 0; i < 3; i++) n[i] += __popcll(__ballot(o[c] == T && lo[c] >= (L | ((i + 1) << b))));
+            }
+            const uint64_t t = total(n[0] | (uint64_t)n[1] << 21 | (uint64_t)n[2] << 42, 17 + (30 - b) / 2);
+            const uint32_t m = (1u << 21) - 1;
+            if ((uint32_t)(t >> 42) >= need) L |= 3u << b;
+            else if (((t >> 21) & m) >= need) L |= 2u << b;
+            else if ((t & m) >= need) L |= 1u << b;
+        }
+    }
+    return make_uint2(T, L);
 }
 
-// Stage 1: workgroup g sorts logits [2048 g, 2048 g + 2048) and keeps its kp = k + 1 largest keys, plus a NaN
-// flag.  part: kp keys per workgroup, then one u32 flag per workgroup.
+// Stage 1: workgroup g keeps the kp = k + 1 largest keys of logits [2048 g, 2048 g + 2048) (in no order, zeros after
+// them where there are fewer), plus a NaN flag.  part: kp keys per workgroup, then one u32 flag per workgroup.
+// Latency bound, like stage 2: the limit takes at most 16 counting steps of a barrier each where sorting the 2048 keys took 66
+// passes over LDS (128256 logits, k = 40: 7.2 us against 50.3, stage 2 11.9 against 38.5).
 KERNEL __launch_bounds__(256) void qp_topk_part(QpCandArgs a) {
-    __shared__ uint64_t s[2048];
+    __shared__ uint64_t cnt[33];
+    __shared__ uint32_t fill;
     const uint32_t tid = threadIdx.x, base = blockIdx.x * 2048;
-    const float* lg = cptr<float>(a.logits);
+    float v[8];
+#pragma unroll
+    for (uint32_t c = 0; c < 8; c++) v[c] = base + c * 256 + tid < a.n ? gload<float>(a.logits + 4ull * (base + c * 256 + tid)) : 0.0f;
+    if (tid < 33) cnt[tid] = 0;
+    if (tid == 0) fill = 0;
+    uint32_t o[8], lo[8];
     int nan = 0;
-    for (uint32_t i = tid; i < 2048; i += 256) {
-        const uint32_t g = base + i;
-        uint64_t key = 0;  // padding sorts below every non-NaN value
-        if (g < a.n) {
-            const float v = lg[g];
-            nan |= v != v;
-            key = topk_key(v, g);
-        }
-        s[i] = key;
+#pragma unroll
+    for (uint32_t c = 0; c < 8; c++) {
+        const uint32_t g = base + c * 256 + tid;
+        const uint64_t key = g < a.n ? topk_key(v[c], g) : 0;
+        nan |= v[c] != v[c];
+        o[c] = (uint32_t)(key >> 32);
+        lo[c] = (uint32_t)key;
     }
     nan = __syncthreads_or(nan);
-    bitonic_desc(s, 2048, tid, 256);
-    uint64_t* part = mptr<uint64_t>(a.part);
-    for (uint32_t i = tid; i < a.kp; i += 256) part[(uint64_t)blockIdx.x * a.kp + i] = s[i];
-    if (tid == 0) reinterpret_cast<uint32_t*>(part + (uint64_t)a.g * a.kp)[blockIdx.x] = nan ? 1u : 0u;
+    const uint2 lim = topk_limit<8>(o, lo, 8, a.kp, cnt);
+    const uint64_t part = a.part + 8ull * blockIdx.x * a.kp;
+#pragma unroll
+    for (uint32_t c = 0; c < 8; c++)
+        if ((o[c] > lim.x || (o[c] == lim.x && lo[c] >= lim.y)) && (o[c] | lo[c])) {
+            const uint32_t at = atomicAdd(&fill, 1u);  // (past kp: NaNs alone, whose o can be 0; the flag tells)
+            if (at < a.kp) gstore<uint64_t>(part + 8 * at, (uint64_t)o[c] << 32 | lo[c]);
+        }
+    __syncthreads();
+    for (uint32_t i = fill + tid; i < a.kp; i += 256) gstore<uint64_t>(part + 8 * i, 0);
+    if (tid == 0) gstore<uint32_t>(a.part + 8ull * a.g * a.kp + 4 * blockIdx.x, nan ? 1u : 0u);
 }
 
-// Stage 2 (one workgroup): merges the g*kp partial keys (n2 = next power of two, in dynamic LDS) and writes
-// out = {flags, k, (value bits, id) x k} in descending order.  flags bit 0: a NaN logit; bit 1: two equal values
-// among the k + 1 largest (float equality, so -0 == +0), i.e. the candidate set or its order would depend on the
-// reference's heap; the host then takes the whole logits array.
+// Stage 2 (one workgroup): the kp largest of the g * kp partial keys (at most 16384), each placed by the number of
+// larger ones; writes out = {flags, k, (value bits, id) x k} in descending order.  flags bit 0: a NaN logit; bit 1: two
+// equal values among the k + 1 largest (float equality, so -0 == +0), i.e. the candidate set or its order would depend
+// on the reference's heap; the host then takes the whole logits array.
 KERNEL __launch_bounds__(1024) void qp_topk_merge(QpCandArgs a) {
-    extern __shared__ float4 smk[];
-    uint64_t* s = reinterpret_cast<uint64_t*>(smk);
-    const uint32_t tid = threadIdx.x, tot = a.g * a.kp;
-    const uint64_t* part = cptr<uint64_t>(a.part);
-    const uint32_t* pf = reinterpret_cast<const uint32_t*>(part + tot);
-    for (uint32_t i = tid; i < a.n2; i += 1024) s[i] = i < tot ? part[i] : 0ull;
+    __shared__ uint64_t cnt[33], s[132], r[132];
+    __shared__ uint32_t fill;
+    const uint32_t tid = threadIdx.x, tot = a.g * a.kp, nc = (tot + 1023) / 1024;
+    uint32_t o[16], lo[16];
+#pragma unroll
+    for (uint32_t c = 0; c < 16; c++) {
+        if (c >= nc) break;
+        const uint64_t key = c * 1024 + tid < tot ? gload<uint64_t>(a.part + 8ull * (c * 1024 + tid)) : 0;
+        o[c] = (uint32_t)(key >> 32);
+        lo[c] = (uint32_t)key;
+    }
+    if (tid < 33) cnt[tid] = 0;
+    if (tid < 132) s[tid] = 0;
+    if (tid == 0) fill = 0;
     int nan = 0;
-    for (uint32_t i = tid; i < a.g; i += 1024) nan |= pf[i] != 0;
+    for (uint32_t i = tid; i < a.g; i += 1024) nan |= gload<uint32_t>(a.part + 8ull * tot + 4 * i) != 0;
     nan = __syncthreads_or(nan);
-    bitonic_desc(s, a.n2, tid, 1024);
-    const int tie = __syncthreads_or(tid < a.k && topk_val(s[tid]) == topk_val(s[tid + 1]));
-    uint32_t* out = mptr<uint32_t>(a.out);
+    const uint2 lim = topk_limit<16>(o, lo, nc, a.kp, cnt);
+#pragma unroll
+    for (uint32_t c = 0; c < 16; c++) {
+        if (c >= nc) break;
+        if ((o[c] > lim.x || (o[c] == lim.x && lo[c] >= lim.y)) && (o[c] | lo[c])) {
+            const uint32_t at = atomicAdd(&fill, 1u);
+            if (at < a.kp) s[at] = (uint64_t)o[c] << 32 | lo[c];
+        }
+    }
+    __syncthreads();
+    // eight threads a key count the larger ones (kp <= 129 of 132 slots, zeros after the kp)
+    for (uint32_t i = tid >> 3; i < a.kp; i += 128) {
+        const uint64_t mine = s[i];
+        uint32_t above = 0;
+        for (uint32_t j = tid & 7; j < a.kp; j += 8) above += s[j] > mine;
+        above += __shfl_xor(above, 1, 64);
+        above += __shfl_xor(above, 2, 64);
+        above += __shfl_xor(above, 4, 64);
+        if ((tid & 7) == 0) r[above] = mine;
+    }
+    __syncthreads();
+    const int tie = __syncthreads_or(tid < a.k && topk_val(r[tid]) == topk_val(r[tid + 1]));
     if (tid == 0) {
-        out[0] = (nan ? 1u : 0u) | (tie ? 2u : 0u);
-        out[1] = a.k;
+        gstore<uint32_t>(a.out, (nan ? 1u : 0u) | (tie ? 2u : 0u));
+        gstore<uint32_t>(a.out + 4, a.k);
     }
     if (tid < a.k) {
-        out[2 + 2 * tid] = __float_as_uint(topk_val(s[tid]));
-        out[3 + 2 * tid] = topk_id(s[tid]);
+        gstore<uint32_t>(a.out + 8 + 8 * tid, __float_as_uint(topk_val(r[tid])));
+        gstore<uint32_t>(a.out + 12 + 8 * tid, topk_id(r[tid]));
     }
 }
 

@@ -1650,14 +1650,11 @@ int op_topk_cand(const Ctx& c) {
     const uint64_t tot = (uint64_t)a.g * a.kp;
     if (tot > 16384) return fail(QP_E_ARG, "topk_cand: V=%u, k=%u: %llu partial candidates exceed 16384", a.n, a.k,
                                  (unsigned long long)tot);
-    uint32_t n2 = 2;
-    while (n2 < tot) n2 <<= 1;
-    a.n2 = n2;
     a.logits = c.B(0);
     a.part = c.B(1);
     a.out = c.B(2);
     if (int e = launch(K_topk_part, a.g, 1, 1, 256, 0, a)) return e;
-    return launch(K_topk_merge, 1, 1, 1, 1024, n2 * 8, a);
+    return launch(K_topk_merge, 1, 1, 1, 1024, 0, a);
 }
 
 // repack_q2k .. repack_q6k: P{nblocks lo, hi, K}; repack_q8: P{nblocks lo, hi}; [paso|0, src, dst].  K (the row

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from quipullm_amd import capi
-from test_gpu_ops import FMTS, PLANAR, dev, raw_matrix  # noqa: F401
+from test_gpu_ops import FMTS, PLANAR, dev, raw_matrix, topk_cand  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -256,3 +256,24 @@ def test_attention_shares_cover_no_token_past_the_dispatch(quipu, dev):
                    [dev.paso(9, 500), dev.buf(q), dev.buf(kc), dev.buf(vc), o], (nh, 2))
     got = dev.get(o, (9, nh * hd))
     assert np.all(got[2:] == 5.0) and not np.any(got[:2] == 5.0)
+
+
+@pytest.mark.parametrize("V,k", [(5, 4), (2047, 128), (2050, 100), (6145, 40), (128256, 128)])
+@pytest.mark.parametrize("kind", ["equal", "few", "infinite", "signs", "nan"])
+def test_topk_equal_values(quipu, dev, V, k, kind):
+    """topk_cand where values repeat within a chunk of 2048, across chunks and at the limit: the lower ids first, +0 before
+    -0, infinities at their ends, and the flags (bit 1: equal values among the k + 1 largest, bit 0: a NaN)."""
+    rng = np.random.default_rng(V + k)
+    v = {"equal": np.full(V, -3.25), "few": rng.integers(-2, 3, V) * 0.5, "infinite": np.where(rng.random(V) < 0.5, -np.inf, 1.0),
+         "signs": np.where(rng.random(V) < 0.5, -0.0, 0.0), "nan": np.zeros(V)}[kind].astype(np.float32)
+    if kind == "infinite":
+        v[V // 2] = np.inf
+    if kind == "nan":
+        v.view(np.uint32)[:] = 0xffffffff
+        assert topk_cand(quipu, dev, v, k)[0] & 1
+        return
+    flags, kk, vals, ids = topk_cand(quipu, dev, v, k)
+    order = np.lexsort((np.arange(V), np.signbit(v), -v))[:k + 1]
+    assert kk == k and flags == (2 if (v[order[:-1]] == v[order[1:]]).any() else 0)
+    assert ids.tolist() == order[:k].tolist()
+    assert vals.view(np.uint32).tolist() == v[order[:k]].view(np.uint32).tolist()

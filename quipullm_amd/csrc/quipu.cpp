@@ -1083,6 +1083,8 @@ int op_moe_topk(const Ctx& c) {
     a.lg = c.B(1);
     a.sel = c.B(2);
     a.wts = c.B(3);
+    // a wavefront per token where its lanes can hold the probabilities and the choices
+    if (a.e <= 256 && a.k <= 64) return launch(K_moe_topk_w, (c.gx ? c.gx : 1) * 16, 1, 1, 256, 0, a);
     return launch(K_moe_topk, (c.gx ? c.gx : 1) * 64, 1, 1, 256, 0, a);
 }
 
@@ -1198,7 +1200,7 @@ uint64_t buf_room(uint64_t p) {
     return 0;
 }
 
-// moe_group (kds.js:491-516): P{E, n}; [paso, sel, lst, off]; one workgroup.  lst[off[e] .. off[e+1]) = the jobs
+// moe_group (kds.js:491-516): P{E, n}; [paso, sel, lst, off].  lst[off[e] .. off[e+1]) = the jobs
 // i < T*n with sel[i] == e, in increasing order.
 int op_moe_group(const Ctx& c) {
     if (int e = need_bufs(c, 4, "moe_group")) return e;
@@ -1217,7 +1219,7 @@ int op_moe_group(const Ctx& c) {
     const uint64_t ns = (rs < rl ? rs : rl) / 4;
     if (ns > 65535) return fail(QP_E_ARG, "moe_group: sel and lst hold %llu jobs; at most 65535", (unsigned long long)ns);
     a.nsel = (uint32_t)ns;
-    return launch(K_moe_group, 1, 1, 1, 256, 256 * a.n_exp * 2 + 4 + 4 * a.n_exp, a);
+    return launch(K_moe_group, a.n_exp, 1, 1, 1024, 0, a);
 }
 
 // matmul_<fmt>_eg (kquants.js:386-460, the expert matmul grouped by expert): P{N, K, acc, tfijo};

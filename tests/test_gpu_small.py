@@ -277,3 +277,16 @@ def test_topk_equal_values(quipu, dev, V, k, kind):
     assert kk == k and flags == (2 if (v[order[:-1]] == v[order[1:]]).any() else 0)
     assert ids.tolist() == order[:k].tolist()
     assert vals.view(np.uint32).tolist() == v[order[:k]].view(np.uint32).tolist()
+
+
+@pytest.mark.parametrize("E,k,T", [(1, 1, 1), (63, 8, 5), (64, 64, 3), (65, 2, 130), (256, 64, 7), (257, 8, 3), (300, 70, 2)])
+def test_moe_topk_sizes(quipu, dev, oracle, E, k, T):
+    """moe_topk by a wavefront per token (E <= 256, k <= 64) and by a workgroup: the experts exactly, equal logits to the
+    lower index; the weights to the exponential's and the sums' rounding (as test_swiglu_moe_ops)."""
+    lg = np.random.default_rng(E + k).integers(-12, 13, (T, E)).astype(np.float32) * np.float32(0.5)
+    sel, wts = dev.zeros(T * k * 4), dev.zeros(T * k * 4)
+    quipu.dispatch("moe_topk", [("u", E), ("u", k), ("u", 1), ("f", 1.5)], [dev.paso(T, 0), dev.buf(lg), sel, wts],
+                   ((T + 63) // 64,))
+    s_want, w_want = oracle.moe_topk(lg, E, k, 1, 1.5)
+    np.testing.assert_array_equal(dev.get(sel, (T * k,), np.uint32), s_want)
+    np.testing.assert_allclose(dev.get(wts, (T * k,)), w_want, rtol=2e-6, atol=1e-7)

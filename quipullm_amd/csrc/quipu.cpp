@@ -1274,6 +1274,7 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
     // tokens (8 jobs per expert) 252 / 492, 256 423 / 502, 384 473 / 520, 512 657 / 541; against the tiles below 32 tokens
     // 185 / 615, 512 541 / 1980, 1024 636 / 2118, 2048 854 / 2371.  Q8_0 and IQ4_NL take the first up to 64 jobs per
     // expert, then the tiles below.
+    // K-quants take 32 weight rows per wavefront in the first (32 tokens: 180 us; 16 rows, X read twice as often, 205).
     const uint32_t per_tok = tfijo > 1 ? tfijo : m ? m : 8;
     const uint64_t max_jobs = 32ull * tz * per_tok;
     const bool few = (max_jobs < a.nlst ? max_jobs : a.nlst) <= (is_kq(fmt) ? 24ull : 64ull) * E;

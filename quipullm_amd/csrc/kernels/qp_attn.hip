@@ -1,22 +1,25 @@
 // Causal attention over f32 caches, sliding windows and rings (the reference's atencion, gpu.js:467-539) on the matrix
-// cores, at f32 accuracy.
+// cores.
 //
 // A workgroup takes 16 RG (query, head) rows of one KV head and a share of the key tiles of 32 slots, dealt to its four
 // wavefronts; each keeps its own softmax state and they meet in LDS.  Scores are S^T = K Q^T and outputs O^T += V^T P^T
 // with v_mfma_f32_16x16x32_f16: a lane holds 8 scores of one row, which are its operand of the second product.  Every
-// f32 operand is an f16 high and low part (22 bits) below a power of two: of the row for Q, of the largest magnitude that
-// the wavefront has met so far for K and V (so a tile is never scaled past f16's range, and values down to 2^-12 of the
-// largest keep all 22 bits), 2^10 for P.  Three products per pair (high high, high low, low high); f16 caches need two.
-// Probabilities, their sums, the maxima and the outputs are f32.
-#include "qp_common.h"
-
-#define KERNEL extern "C" __global__
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// f32 operand is an f16 high and low part (22 bits, two fewer than f32) below a power of two: of the row for Q, 16 times
+// the wavefront's first tile's largest magnitude for K and V, 2^10 for P.  Three products per pair (high high, high low,
+// low high; low low lies below the sums' rounding); f16 caches need two.  Scores, sums, maxima and outputs are f32,
+// probabilities 2^x in f32 before their split.  Distance from 64 bits (2-norm, 128 dimensions, random operands): one token
+// behind 3000 keys 3.4e-7, 32 behind 480 3.1e-7, 333 behind 1000 3.3e-7; the general kernel's f32 sums 1.1e-6, 5.6e-7, 7.2e-7.
+//
+// One scale for several keys is only sound while their magnitudes are alike: a row must not lose bits to a key that it
+// does not see, or gives no weight.  So each lane compares its pieces of the operands (32 inputs of a query or key, 4 or 8
+// of a value) with that scale: where one lies above it (an infinity always does) or is not zero and below 2^-14 of it, the
+// wavefront takes its remaining tiles in f32 (v_mfma_f32_16x16x4_f32 on the same registers, an eighth of the rate or less).
+// (A NaN needs no such care: it stays with its key and its row, and in a value it reaches every row of the block either way.)
+// The comparisons cost 0 to 1 % of a pass: two windowed layers at 500 tokens 1119 us, 1107 without them.
+#include "qp_ints.h"
 
 QP_DEV f32x4 ax_mfma(h8 a, h8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+QP_DEV f32x4 ax_mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // f16 high and low parts of eight values already below 2^10.
 QP_DEV void ax_split(const float* v, float up, h8& hi, h8& lo) {
@@ -33,8 +36,17 @@ QP_DEV int ax_exp(float m) {
     return e < -117 ? -117 : e;
 }
 QP_DEV float ax_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+// Magnitudes that operands scaled by 2^(9 - e) may have: below 2^(e + 1), and from 2^(e - 14) on.
+QP_DEV float ax_top(int e) { return __uint_as_float((uint32_t)(min(e + 1, 128) + 127) << 23); }
+QP_DEV float ax_low(int e) { return __uint_as_float(e - 14 > -127 ? (uint32_t)(e - 14 + 127) << 23 : 1u); }
+// The scale of a wavefront's tiles, from the largest magnitude of the first: 16 times it (finite values only).
+QP_DEV int ax_anchor(float mx, uint32_t lane) {
+    return min(__builtin_amdgcn_readfirstlane(ax_exp(wave_max_v(fminf(mx, 3.4e38f), lane))) + 4, 127);
+}
 
 constexpr float AX_LOG2E = 1.4426950408889634f;
+
+typedef uint16_t us2 __attribute__((ext_vector_type(2)));
 
 template <int HD, bool F16, int RG>
 QP_DEV void attn_x_body(const QpAttnArgs& a) {
@@ -51,11 +63,12 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
     h8 qh[RG][KS], ql[RG][KS];
     float qs[RG];         // score = accumulator * qs (times the keys' scale), in units of log2
     int lim[RG], low[RG]; // keys low < key <= lim
+    bool alike = true;    // the operands so far are of like magnitudes (this lane's)
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         const uint32_t row = r0 + r * 16 + n16, rc = min(row, nrow - 1), t = rc / G, h = kvh * G + rc % G;
         float v[KS][8];
-        float mx = 0.0f;
+        float mine = 0.0f;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
             const uint64_t at = a.q + 4 * (((uint64_t)t * a.nh + h) * HD + s * 32 + g * 8);
@@ -64,12 +77,13 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 v[s][i] = w[i];
-                mx = fmaxf(mx, fabsf(w[i]));
+                mine = fmaxf(mine, fabsf(w[i]));
             }
         }
-        mx = fmaxf(mx, bfly_f<4>(mx, lane));
-        mx = fmaxf(mx, bfly_f<5>(mx, lane));
-        const int e = ax_exp(mx);
+        float all = fmaxf(mine, bfly_f<4>(mine, lane));
+        all = fmaxf(all, bfly_f<5>(all, lane));
+        const int e = ax_exp(all);
+        alike = alike & (all < __builtin_inff()) & ((mine == 0.0f) | (mine >= ax_low(e)));
 #pragma unroll
         for (int s = 0; s < KS; s++) ax_split(v[s], ax_pow2(9 - e), qh[r][s], ql[r][s]);
         qs[r] = ax_pow2(e - 9) * a.scale * AX_LOG2E;
@@ -126,9 +140,23 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
         }
     };
 
+    // value x (of 8) of step c of the lane's key h, and the lane's key j's value at dimension d
+    auto key = [&](int h, int c, int x) __attribute__((always_inline)) -> float {
+        if constexpr (F16) return h2f(kw[h][c][x >> 1] >> (16 * (x & 1)));
+        else return __uint_as_float(kw[h][2 * c + (x >> 2)][x & 3]);
+    };
+    auto val = [&](int j, int d) __attribute__((always_inline)) -> float {
+        if constexpr (F16) return h2f(vw[d][j >> 1] >> (16 * (j & 1)));
+        else return __uint_as_float(vw[j * (DT / 4) + (d >> 2)][d & 3]);
+    };
+    // the f16 caches' largest magnitudes, two halves at a time
+    auto pk_max = [&](uint32_t m, uint32_t w) __attribute__((always_inline)) -> uint32_t {
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, m), __builtin_bit_cast(us2, w & 0x7fff7fffu)));
+    };
+
     f32x4 o[RG][DT];
-    float m[RG], l[RG];
-    int ek = -117, ev = -117;  // exponents of the largest key and value so far
+    float m[RG], l[RG], p[RG][8], corr[RG];
+    int ek = 0, ev = 0;     // the keys' and values' scale
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         m[r] = -3.0e38f;
@@ -136,58 +164,14 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
 #pragma unroll
         for (int d = 0; d < DT; d++) o[r][d] = f32x4{0, 0, 0, 0};
     }
-    uint32_t i = i0 + wave;
-    load_k(i);
-    load_v(i);
-    for (; i < i1; i += 4) {
-        const Tile t = tile(i);
-        // ---- S^T = K Q^T
-        float upk = 1.0f, ck = 1.0f;
-        if constexpr (!F16) {
-            float mx = 0.0f;
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-#pragma unroll
-                for (int c = 0; c < KL; c++)
-#pragma unroll
-                    for (int x = 0; x < 4; x++) mx = fmaxf(mx, fabsf(__uint_as_float(kw[h][c][x])));
-            ek = max(ek, __builtin_amdgcn_readfirstlane(ax_exp(wave_max_v(mx, lane))));
-            upk = ax_pow2(9 - ek);
-            ck = ax_pow2(ek - 9);
-        }
-        f32x4 s[RG][2];
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int c = 0; c < KS; c++) {
-                h8 kh, kl;
-                if constexpr (F16) {
-                    kh = __builtin_bit_cast(h8, kw[h][c]);
-                } else {
-                    float v[8];
-#pragma unroll
-                    for (int x = 0; x < 8; x++) v[x] = __uint_as_float(kw[h][2 * c + (x >> 2)][x & 3]);
-                    ax_split(v, upk, kh, kl);
-                }
-#pragma unroll
-                for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kh, qh[r][c], c ? s[r][h] : f32x4{0, 0, 0, 0});
-#pragma unroll
-                for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kh, ql[r][c], s[r][h]);
-                if constexpr (!F16) {
-#pragma unroll
-                    for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kl, qh[r][c], s[r][h]);
-                }
-            }
-        load_k(i + 4);
-        // ---- softmax of the lane's 8 keys of each of its rows
+    // softmax of the lane's 8 keys of each of its rows: scores s times unit (and qs), in units of log2
+    auto softmax = [&](const Tile& t, const f32x4 (&s)[RG][2], auto Split, float unit) __attribute__((always_inline)) {
         // all slots hold keys that every row of the block sees
         const bool whole = t.slot >= t.lo && t.slot + 32 <= t.hi && (int)t.slot + 31 + t.off <= (int)(pos0 + t_lo) &&
                            (!a.swa || (int)t.slot + t.off > (int)(pos0 + t_hi) - (int)a.swa);
-        h8 ph[RG], pl[RG];
-        float corr[RG];
 #pragma unroll
         for (int r = 0; r < RG; r++) {
-            const float c = qs[r] * ck;
+            const float c = Split.v ? qs[r] * unit : unit;
             float x[8], mx = -3.0e38f;
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -207,58 +191,147 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
             float sum = 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const float p = __builtin_amdgcn_exp2f(x[j] - mn);
-                sum += p;
-                const float p10 = p * 1024.0f;
-                ph[r][j] = (_Float16)p10;
-                pl[r][j] = (_Float16)(p10 - (float)ph[r][j]);
+                p[r][j] = __builtin_amdgcn_exp2f(x[j] - mn);
+                sum += p[r][j];
             }
             l[r] = l[r] * corr[r] + sum;
         }
-        // ---- O^T += V^T P^T
-        float upv = 1.0f, ratio = 1.0f;
-        if constexpr (!F16) {
-            float mx = 0.0f;
+    };
+    // f16 values: slots without a key may hold anything
+    auto mask_v = [&](const Tile& t) __attribute__((always_inline)) {
+        if (!F16 || (t.slot >= t.lo && t.slot + 32 <= t.hi)) return;
 #pragma unroll
-            for (int c = 0; c < VL; c++)
+        for (int j = 0; j < 4; j++) {
+            const uint32_t sl = t.slot + (j >> 1) * 16 + 4 * g + 2 * (j & 1);
+            const uint32_t keep = (sl >= t.lo && sl < t.hi ? 0xffffu : 0u) | (sl + 1 >= t.lo && sl + 1 < t.hi ? 0xffff0000u : 0u);
 #pragma unroll
-                for (int x = 0; x < 4; x++) mx = fmaxf(mx, fabsf(__uint_as_float(vw[c][x])));
-            const int en = max(ev, __builtin_amdgcn_readfirstlane(ax_exp(wave_max_v(mx, lane))));
-            ratio = ev - en < -120 ? 0.0f : ax_pow2(ev - en);
-            ev = en;
-            upv = ax_pow2(9 - ev);
+            for (int d = 0; d < VL; d++) vw[d][j] &= keep;
         }
-        float keep = ratio;
-        bool same = true;
+    };
+    auto rescale = [&](float f) __attribute__((always_inline)) {
+        bool same = f == 1.0f;
 #pragma unroll
-        for (int r = 0; r < RG; r++) same = same && corr[r] * ratio == 1.0f;
-        if (!__builtin_amdgcn_readfirstlane(__all(same))) {
+        for (int r = 0; r < RG; r++) same = same && corr[r] == 1.0f;
+        if (__all(same)) return;
 #pragma unroll
-            for (int r = 0; r < RG; r++) {
-                const float f = corr[r] * keep;
+        for (int r = 0; r < RG; r++)
 #pragma unroll
-                for (int d = 0; d < DT; d++)
+            for (int d = 0; d < DT; d++)
 #pragma unroll
-                    for (int x = 0; x < 4; x++) o[r][d][x] *= f;
+                for (int x = 0; x < 4; x++) o[r][d][x] *= corr[r] * f;
+    };
+    auto pv_f32 = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int r = 0; r < RG; r++) o[r][d] = ax_mfma(val(j, d), p[r][j], o[r][d]);
+    };
+    uint32_t i = i0 + wave;
+    load_k(i);
+    load_v(i);
+    bool first_tile = true, pending = false;  // pending: tile i's scores are done, its values not
+    for (; i < i1; i += 4) {
+        const Tile t = tile(i);
+        // ---- S^T = K Q^T
+        if constexpr (F16) {  // (a key's rounding is its own: only infinities matter)
+            uint32_t mx = 0;
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int c = 0; c < KL; c++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) mx = pk_max(mx, kw[h][c][x]);
+            alike = alike & ((mx & 0xffffu) < 0x7c00u) & ((mx >> 16) < 0x7c00u);
+        } else {
+            float kx[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int c = 0; c < KS; c++)
+#pragma unroll
+                    for (int x = 0; x < 8; x++) kx[h] = fmaxf(kx[h], fabsf(key(h, c, x)));
+            if (first_tile) ek = ax_anchor(fmaxf(kx[0], kx[1]), lane);
+            const float top = ax_top(ek), lo = ax_low(ek);
+#pragma unroll
+            for (int h = 0; h < 2; h++) alike = alike & (kx[h] < top) & ((kx[h] == 0.0f) | (kx[h] >= lo));
+        }
+        if (!__all(alike)) break;
+        f32x4 s[RG][2];
+        const float upk = F16 ? 1.0f : ax_pow2(9 - ek);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int c = 0; c < KS; c++) {
+                h8 kh, kl;
+                if constexpr (F16) {
+                    kh = __builtin_bit_cast(h8, kw[h][c]);
+                } else {
+                    float v[8];
+#pragma unroll
+                    for (int x = 0; x < 8; x++) v[x] = key(h, c, x);
+                    ax_split(v, upk, kh, kl);
+                }
+#pragma unroll
+                for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kh, qh[r][c], c ? s[r][h] : f32x4{0, 0, 0, 0});
+#pragma unroll
+                for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kh, ql[r][c], s[r][h]);
+                if constexpr (!F16) {
+#pragma unroll
+                    for (int r = 0; r < RG; r++) s[r][h] = ax_mfma(kl, qh[r][c], s[r][h]);
+                }
+            }
+        load_k(i + 4);
+        softmax(t, s, SkInt<1>(), F16 ? 1.0f : ax_pow2(ek - 9));
+        // ---- O^T += V^T P^T
+        mask_v(t);
+        float vx[8];
+        if constexpr (F16) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int d = 0; d < DT; d++) w = pk_max(w, vw[d][j]);
+                vx[2 * j] = h2f(w);
+                vx[2 * j + 1] = h2f(w >> 16);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                vx[j] = 0.0f;
+#pragma unroll
+                for (int d = 0; d < DT; d++) vx[j] = fmaxf(vx[j], fabsf(val(j, d)));
             }
         }
-        const bool inside = t.slot >= t.lo && t.slot + 32 <= t.hi;
+        if (first_tile) {
+            float all = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) all = fmaxf(all, vx[j]);
+            ev = ax_anchor(all, lane);
+        }
+        first_tile = false;
+        const float top = ax_top(ev), lo = ax_low(ev);
+#pragma unroll
+        for (int j = 0; j < 8; j++) alike = alike & (vx[j] < top) & ((vx[j] == 0.0f) | (vx[j] >= lo));
+        if (!__all(alike)) {
+            pending = true;
+            break;
+        }
+        rescale(1.0f);
+        const float upv = F16 ? 1.0f : ax_pow2(9 - ev);
+        h8 ph[RG], pl[RG];
+#pragma unroll
+        for (int r = 0; r < RG; r++) ax_split(p[r], 1024.0f, ph[r], pl[r]);
 #pragma unroll
         for (int d = 0; d < DT; d++) {
             h8 vh, vl;
             if constexpr (F16) {
                 vh = __builtin_bit_cast(h8, vw[d]);
-                if (!inside) {  // slots without a key may hold anything
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const uint32_t sl = t.slot + (j >> 2) * 16 + 4 * g + (j & 3);
-                        vh[j] = sl >= t.lo && sl < t.hi ? vh[j] : (_Float16)0.0f;
-                    }
-                }
             } else {
                 float v[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = __uint_as_float(vw[j * (DT / 4) + (d >> 2)][d & 3]);
+                for (int j = 0; j < 8; j++) v[j] = val(j, d);
                 ax_split(v, upv, vh, vl);
             }
 #pragma unroll
@@ -272,11 +345,49 @@ QP_DEV void attn_x_body(const QpAttnArgs& a) {
         }
         load_v(i + 4);
     }
+    float back = (F16 ? 1.0f : ax_pow2(ev - 9)) * 0x1p-10f;  // o times it: the outputs
+    if (i < i1) {  // the other tiles in f32
+        if (!pending) {
+#pragma unroll
+            for (int r = 0; r < RG; r++) corr[r] = 1.0f;
+        }
+        rescale(back);
+        back = 1.0f;
+        if (pending) {
+            pv_f32();
+            load_v(i + 4);
+            i += 4;
+        }
+        for (; i < i1; i += 4) {
+            const Tile t = tile(i);
+            f32x4 s[RG][2];
+#pragma unroll
+            for (int r = 0; r < RG; r++) {
+                const uint32_t rc = min(r0 + r * 16 + n16, nrow - 1);
+                const uint64_t at = a.q + 4 * (((uint64_t)(rc / G) * a.nh + kvh * G + rc % G) * HD + g * 8);
+                s[r][0] = s[r][1] = f32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int c = 0; c < KS; c++) {
+                    const float4 q0 = gload<float4>(at + c * 128), q1 = gload<float4>(at + c * 128 + 16);
+                    const float q[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+                    for (int x = 0; x < 8; x++)
+#pragma unroll
+                        for (int h = 0; h < 2; h++) s[r][h] = ax_mfma(key(h, c, x), q[x], s[r][h]);
+                }
+            }
+            load_k(i + 4);
+            softmax(t, s, SkInt<0>(), a.scale * AX_LOG2E);
+            mask_v(t);
+            rescale(1.0f);
+            pv_f32();
+            load_v(i + 4);
+        }
+    }
     // ---- the four wavefronts' states meet: [wave][row][HD + 4], then [wave][row] (m, l)
     constexpr int LD = HD + 4;
     float* ol = reinterpret_cast<float*>(ax_lds);
     float* ml = ol + 4 * RG * 16 * LD;
-    const float back = (F16 ? 1.0f : ax_pow2(ev - 9)) * 0x1p-10f;
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         float lt = l[r];

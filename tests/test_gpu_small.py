@@ -244,6 +244,71 @@ def test_attention_any_cache(quipu, dev, hd, nh, nkv, T, pos0, swa, cap, f16):
             assert np.all(np.abs(got[t, h] - w @ v) <= (2 * e + 2.0 ** -19) * np.abs(v).max()), (t, h)
 
 
+@pytest.mark.parametrize("f16", [0, 1])
+@pytest.mark.parametrize("hd,nh,nkv,T,pos0,swa,cap", [(128, 8, 4, 24, 40, 0, 0),   # two blocks of 32 rows, f32 or window
+                                                      (64, 4, 4, 9, 300, 40, 64),   # a block of 16 rows, a ring
+                                                      (128, 6, 2, 1, 700, 600, 0)])  # one token, keys shared out
+@pytest.mark.parametrize("kind", ["k_infinite", "k_minus_infinite", "k_huge", "v_huge", "v_without_weight", "q_spread"])
+def test_attention_unlike_magnitudes(quipu, dev, hd, nh, nkv, T, pos0, swa, cap, f16, kind):
+    """Keys and values far larger than the others, infinities among them: a row that does not see such a key, or gives it
+    no weight, has the result that it would have without it.
+
+    Bound as in test_attention_any_cache, over the keys with a weight above 1e-36 only (below it a weight is 0 in float32)."""
+    if f16 and not swa:
+        swa = 1000  # (f16 caches without a window take another kernel)
+    rng = np.random.default_rng(83)
+    kvd, n = nkv * hd, pos0 + T
+    q = rng.standard_normal((T, nh, hd)).astype(np.float32)
+    q[..., 0] = 4.0
+    kf, vf = (rng.standard_normal((n, kvd)).astype(np.float32) for _ in range(2))
+    late = pos0 + T // 2  # seen by the later half of the chunk only (one token: by that token)
+    big = np.float32(6e4 if f16 else 2.0 ** 60)
+    if kind == "k_infinite":
+        kf[late, 5::hd] = np.inf
+    elif kind == "k_minus_infinite":
+        kf[late, 0::hd] = -np.inf  # (q's first input is positive: no weight)
+    elif kind == "k_huge":
+        kf[late, 7::hd] = big
+    elif kind == "v_huge":
+        vf *= np.float32(1e-3)
+        vf[late] = big
+    elif kind == "v_without_weight":
+        vf *= np.float32(1e-3)
+        vf[pos0 - 3] = big
+        kf[pos0 - 3] = 0
+        kf[pos0 - 3, 0::hd] = -3000
+    else:
+        q[T // 2:, :, 3] *= np.float32(2.0 ** 30)
+        kf[:, 3::hd] = 0
+    dt = np.float16 if f16 else np.float32
+    kf, vf = kf.astype(dt).astype(np.float32), vf.astype(dt).astype(np.float32)
+    slots = cap or n + 9
+    kc, vc = (np.full((slots, kvd), np.nan, dt) for _ in range(2))
+    for p in range(max(0, n - slots), n):
+        kc[p % slots], vc[p % slots] = kf[p], vf[p]
+    import refs
+    o = dev.zeros(4 * T * nh * hd)
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    quipu.dispatch("atencion", [("u", hd), ("u", nh), ("u", nkv), ("u", swa), ("f", scale), ("u", cap), ("u", 0), ("u", 0),
+                                ("u", f16), ("u", slots)],
+                   [dev.paso(T, pos0), dev.buf(q), dev.buf(kc), dev.buf(refs.v_tiled(vc, kvd) if f16 else vc), o], (nh, T))
+    got = dev.get(o, (T, nh, hd))
+    q64, k64, v64 = q.astype(np.float64), *(a.astype(np.float64).reshape(n, nkv, hd) for a in (kf, vf))
+    for t in range(T):
+        a, b = max(0, pos0 + t + 1 - swa) if swa else 0, pos0 + t + 1
+        for h in range(nh):
+            k, v = k64[a:b, h * nkv // nh], v64[a:b, h * nkv // nh]
+            s = k @ q64[t, h] * scale
+            if s.max() == np.inf:
+                assert not np.isfinite(got[t, h]).any(), (t, h)
+                continue
+            w = np.exp(s - s.max())
+            w /= w.sum()
+            on = w > 1e-36
+            e = 2.0 ** -21 * (np.abs(k[on]) @ np.abs(q64[t, h])).max() * scale
+            assert np.all(np.abs(got[t, h] - w[on] @ v[on]) <= (2 * e + 2.0 ** -19) * np.abs(v[on]).max()), (t, h)
+
+
 def test_attention_shares_cover_no_token_past_the_dispatch(quipu, dev):
     """A Paso of more tokens than the dispatch covers: the others' outputs stay as they were (shares of the keys keep
     partial states for the covered tokens only)."""

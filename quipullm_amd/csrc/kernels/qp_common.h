@@ -103,6 +103,11 @@ QP_DEV void vm_drain() { __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xf << 8)); }
 
 // Paso in device memory: {T, pos0, a, b}
 QP_DEV uint32_t paso_T(uint64_t p) { return cptr<uint32_t>(p)[0]; }
+// Tokens from tbase on, at most rows.
+QP_DEV uint32_t pass_T(uint64_t p, uint32_t tbase, uint32_t rows) {
+    const uint32_t T = paso_T(p);
+    return T > tbase ? min(T - tbase, rows) : 0;
+}
 QP_DEV uint32_t paso_pos(uint64_t p) { return cptr<uint32_t>(p)[1]; }
 
 // ------------------------------------------------------------------ timeline (profiling builds only)

@@ -2204,7 +2204,7 @@ KERNEL __launch_bounds__(256) void qp_split_bf16(QpSplitArgs a) {
 
 // y[t][n] = (acc ? y : 0) + (ws[0] + ws[1] + ...)[t][n], the splits summed in order.
 KERNEL __launch_bounds__(256) void qp_gemm_reduce(QpReduceArgs a) {
-    const uint64_t tn = (uint64_t)paso_T(a.paso) * a.n, plane = (uint64_t)a.rows * a.n;
+    const uint64_t tn = (uint64_t)pass_T(a.paso, a.tbase, a.rows) * a.n, plane = (uint64_t)a.rows * a.n;
     const float* ws = cptr<float>(a.ws);
     float* y = mptr<float>(a.y);
     if ((a.n & 3) == 0 && a.splits <= 8 && ((a.ws | a.y) & 15) == 0) {

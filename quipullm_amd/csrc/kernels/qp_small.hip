@@ -21,8 +21,8 @@ KERNEL __launch_bounds__(256) void qp_split_f16(QpSplitArgs a) {
     __shared__ float mxs[4][16];
     __shared__ float sums[16][17];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, m = lane & 15;
-    const uint32_t ch = blockIdx.x, nch = gridDim.x, T = paso_T(a.paso);
-    uint64_t rows = a.mul ? (uint64_t)T * a.mul : T;
+    const uint32_t ch = blockIdx.x, nch = gridDim.x;
+    uint64_t rows = a.mul ? (uint64_t)paso_T(a.paso) * a.mul : pass_T(a.paso, a.tbase, a.rows);
     if (a.mul && rows > a.cap) rows = a.cap;
     const uint32_t row = blockIdx.y * 16 + m;
     if (blockIdx.y * 16 >= rows) return;
@@ -409,7 +409,7 @@ QP_DEV void sk_body(const QpSkArgs& a) {
         o0 = __builtin_amdgcn_readfirstlane(gload<uint32_t>(a.off + 4ull * e));
         o1 = __builtin_amdgcn_readfirstlane(min(gload<uint32_t>(a.off + 4ull * e + 4), a.nlst));
     } else {
-        o1 = min(paso_T(a.paso), a.rows);
+        o1 = pass_T(a.paso, a.tbase, a.rows);
     }
     const uint32_t nch = (a.k + 255) / 256, kw = wave % a.kw, rg = wave / a.kw;
     const uint32_t row0 = (blockIdx.x * (4 / a.kw) + rg) * 16 * R;

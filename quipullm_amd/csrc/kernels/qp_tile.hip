@@ -63,7 +63,7 @@ QP_DEV void tile_body(const QpTileArgs& a) {
         const uint32_t grp = L / (a.mt * 8), rem = L % (a.mt * 8), in = min(8u, a.nt - grp * 8);
         t0 = (rem / in) * 128;
         nti = grp * 8 + rem % in;
-        const uint32_t T = min(paso_T(a.paso), a.rows);
+        const uint32_t T = pass_T(a.paso, a.tbase, a.rows);
         if (t0 >= T) return;
         cnt = min(T - t0, 128u);
     } else {  // the experts' 128-job tiles that are there, in order: the experts' counts scanned by every wavefront

@@ -135,24 +135,25 @@ typedef struct {
 // qp_sk_<fmt>: matmul of few token rows on integer weights (qp_small.hip).  xs: X as operands (qp_split_f16) of `rows`
 // rows (a multiple of 16).  kw: K slices per workgroup (1, 2 or 4).  Grid y: tpe slots (of each expert), each taking
 // every tpe-th block of 16 NT rows.  lst != 0: grouped by expert as in QpGemmArgs; xrows, yrows, nlst: rows of X's
-// operands and y and entries of lst that exist.  wrows: rows of the whole tensor.
+// operands and y and entries of lst that exist.  wrows: rows of the whole tensor.  tbase: the token that the first row of
+// xs and y is (a call in several passes over its tokens).
 typedef struct {
     uint64_t w, xs, y, paso, lst, off, wrows;
     uint32_t n, k, acc, rows;
-    uint32_t kw, tpe, tfijo, pad;
-    uint32_t xrows, yrows, nlst, pad2;
+    uint32_t kw, tpe, tfijo, tbase;
+    uint32_t xrows, yrows, nlst, pad;
 } QpSkArgs;
 
 // qp_tile_<fmt>, qp_tile_glu_<fmt> (K-quants, qp_tile.hip): 128 x 128 tiles, mt x nt of them (grouped by expert, lst != 0:
 // at most mt tiles of 128 jobs in nexp experts) in grid x (a multiple of 8), grid z K splits of kb blocks of 256 inputs.
 // xs: X as operands (qp_split_f16) of `rows` rows.  ws: 0, or the splits' sums [splits][rows][n].  glu: w gate, w2 up, 64
-// rows of each per tile; yplanes: 0, or y receives the next matmul's input planes of that many token rows.
+// rows of each per tile; yplanes: 0, or y receives the next matmul's input planes of that many token rows.  tbase: as above.
 typedef struct {
     uint64_t w, w2, xs, y, ws, paso, lst, off, wrows;
     uint32_t n, k, acc, rows;
     uint32_t mt, nt, kb, nexp;
     uint32_t tfijo, xrows, yrows, nlst;
-    uint32_t yplanes, pad;
+    uint32_t yplanes, tbase;
 } QpTileArgs;
 
 // moe_group: lst[off[e] .. off[e + 1]) = the jobs i < T * n (in increasing order) with sel[i] == e, e < n_exp;
@@ -165,10 +166,11 @@ typedef struct {
 // first min(T * mul, cap) rows of x instead of T, in row-major planes ([rows][k rounded up to 32]: the grouped
 // expert matmul, whose tiles gather rows), not the chunk-quarter layout of the 256-token tiles.
 // qp_split_f16 (the integer-weight matmuls' operands) takes the same: mul as there; mode 0: X to 22 bits, 1: X as its bf16
-// high + low parts first, 2: x holds those parts (qp_split_bf16's planes of prows token rows).
-typedef struct { uint64_t x, xs, paso; uint32_t k, rows, mul, cap, mode, prows; } QpSplitArgs;
-// y[t][n] = (acc ? y : 0) + sum over s (in order) of ws[s][t][n].
-typedef struct { uint64_t ws, y, paso; uint32_t n, rows, splits, acc; } QpReduceArgs;
+// high + low parts first, 2: x holds those parts (qp_split_bf16's planes of prows token rows).  tbase (mul = 0): the token
+// that x's first row is.
+typedef struct { uint64_t x, xs, paso; uint32_t k, rows, mul, cap, mode, prows, tbase, pad; } QpSplitArgs;
+// y[t][n] = (acc ? y : 0) + sum over s (in order) of ws[s][t][n], for the tokens tbase + t, t < rows.
+typedef struct { uint64_t ws, y, paso; uint32_t n, rows, splits, acc, tbase, pad; } QpReduceArgs;
 
 // ---------------------------------------------------------------- elementwise / small ops
 typedef struct { uint64_t w, ids, y, paso; uint32_t fmt, d, rows, tseq; } QpEmbedArgs;  // rows: tensor rows

@@ -445,7 +445,7 @@ int workspace(uint64_t bytes, uint64_t* out) {
 // there (the same x, paso, K, planes and workspace allocation), else x is split.
 struct SplitMemo {
     uint64_t x, xs, paso;
-    uint32_t k, rows, mul, cap, gen;
+    uint32_t k, rows, mul, cap, gen, tbase;
     int ints;  // -1: qp_split_bf16's planes, else qp_split_f16's operands of that mode
     bool valid;
 } g_split_memo = {};
@@ -454,13 +454,13 @@ struct SplitMemo {
 // and graph launches invalidate it.
 // mul, cap: rows T * mul of x, at most cap (QpSplitArgs); 0: T rows.
 int split_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse,
-                uint32_t mul = 0, uint32_t cap = 0, int ints = -1, uint32_t prows = 0) {
+                uint32_t mul = 0, uint32_t cap = 0, int ints = -1, uint32_t prows = 0, uint32_t tbase = 0) {
     const SplitMemo& m = g_split_memo;
     if (reuse && !g_capturing && m.valid && m.x == x && m.xs == xs && m.paso == paso && m.k == K && m.rows == rows &&
-        m.mul == mul && m.cap == cap && m.gen == g_ws_gen && m.ints == ints)
+        m.mul == mul && m.cap == cap && m.gen == g_ws_gen && m.tbase == tbase && m.ints == ints)
         return 0;
-    QpSplitArgs sa = {x, xs, paso, K, rows, mul, cap, ints < 0 ? 0u : (uint32_t)ints, prows};
-    g_split_memo = {x, xs, paso, K, rows, mul, cap, g_ws_gen, ints, false};
+    QpSplitArgs sa = {x, xs, paso, K, rows, mul, cap, ints < 0 ? 0u : (uint32_t)ints, prows, tbase, 0};
+    g_split_memo = {x, xs, paso, K, rows, mul, cap, g_ws_gen, tbase, ints, false};
     if (int e = ints >= 0 ? launch(K_split_f16, cdiv(K, 256), rows / 16, 1, 256, 0, sa)
                      : launch(K_split_bf16, grid_cap((uint64_t)tmax * K / 8), 1, 1, 256, 0, sa))
         return e;
@@ -471,6 +471,14 @@ int split_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t row
 // ---- integer-weight matmul of few token rows (qp_small.hip): X as operands, 16 R weight rows per wavefront.
 // Bytes of the operands and scales of `rows` rows (a multiple of 16) of K inputs.
 uint64_t sk_bytes(uint32_t rows, uint32_t K) { return (uint64_t)(rows / 16) * cdiv(K, 256) * (18 * 1024 + 64); }
+
+// Rows of one pass of a dense matmul of rows16 rows (a multiple of 16): all, or as many whole 128s as have operands that
+// the kernels' 31-bit offsets reach (QP_NOOFF, the offset of lanes without work, must lie past them): 30,848 rows at
+// K = 15360.
+uint32_t pass_rows(uint32_t rows16, uint32_t K) {
+    const uint64_t fit = ((1ull << 31) - 1) / sk_bytes(16, K);
+    return rows16 <= fit * 16 ? rows16 : (uint32_t)(fit / 8 * 128);
+}
 
 Kid sk_kid(int fmt, uint32_t nt, uint32_t R) {
 #define SK_R1(F) {K_sk_##F##_t1r1, K_sk_##F##_t2r1, K_sk_##F##_t4r1}
@@ -530,8 +538,10 @@ int run_tile(int fmt, QpTileArgs& a, bool glu, uint32_t ns) {
 }
 // X of a dense K-quant matmul's tiles as operands.  From 256 tokens on (where a caller's input planes may take the place
 // of the f32 rows: planes, rows in whole 256s) by way of the rows' bf16 high + low parts, so that both give the same bits.
-int tile_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse, bool planes) {
-    return split_input(x, xs, paso, K, rows, tmax, reuse, 0, 0, planes ? 2 : tmax >= 256 ? 1 : 0, planes ? cdiv(tmax, 256) * 256 : 0);
+// Token tbase on, tmax of them in all (a token's 16 bytes of a plane's 8 inputs lie side by side).
+int tile_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse, bool planes, uint32_t tbase) {
+    return split_input(x + (planes ? 16ull : 4ull * K) * tbase, xs, paso, K, rows, tmax, reuse, 0, 0,
+                       planes ? 2 : tmax >= 256 ? 1 : 0, planes ? cdiv(tmax, 256) * 256 : 0, tbase);
 }
 
 int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z) {
@@ -556,7 +566,7 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
     if (xplanes && (!is_kq(fmt) || tmax < 256 || (g_capturing && !g_noalloc) || getenv_flag("QP_NO_MFMA")))
         return fail(QP_E_ARG, "%s: P[4] = 2 (x holds input planes) needs K-quant weights and a chunk of 256 tokens "
                               "or more on the matrix cores", name);
-    const uint32_t t1 = tmax ? tmax : 1;
+    const uint32_t t1 = tmax ? tmax : 1, rows16 = cdiv(t1, 16) * 16;
     if (!xplanes && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") && sk_takes(fmt, t1, N, K) &&
         (!g_noalloc || sk_bytes(cdiv(t1, 16) * 16, K) <= QP_SCRATCH_BYTES)) {
         QpSkArgs s = {};
@@ -567,13 +577,16 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         s.k = K;
         s.acc = acc;
         s.wrows = N;
-        const uint32_t nt = t1 <= 16 ? 1 : t1 <= 32 ? 2 : 4, yb = cdiv(t1, 16 * nt);
-        s.rows = 16 * cdiv(t1, 16);
-        if (int e = workspace(sk_bytes(s.rows, K), &s.xs)) return e;
-        if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, 0)) return e;
-        return run_sk(fmt, s, nt, yb, 1, sk_rows(fmt, nt, yb, N));
+        const uint32_t nt = t1 <= 16 ? 1 : t1 <= 32 ? 2 : 4, R = sk_rows(fmt, nt, cdiv(t1, 16 * nt), N), step = pass_rows(rows16, K);
+        if (int e = workspace(sk_bytes(step, K), &s.xs)) return e;
+        for (s.tbase = 0; s.tbase < rows16; s.tbase += step, s.y += 4ull * step * N) {
+            s.rows = rows16 - s.tbase < step ? rows16 - s.tbase : step;
+            if (int e = split_input(a.x + 4ull * s.tbase * K, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, 0, 0, s.tbase))
+                return e;
+            if (int e = run_sk(fmt, s, nt, cdiv(s.rows, 16 * nt), 1, R)) return e;
+        }
+        return 0;
     }
-    const uint32_t rows16 = cdiv(t1, 16) * 16;
     // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip), where qp_dispatch_noalloc's scratch holds
     // X's operands.  Against the tiles below at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 108 / 183 / 340 /
     // 597 against 133 / 224 / 383 / 720, 1024 x 4096 32 / 35 / 51 / 75 against 31 / 39 / 54 / 84; Q6_K 4096 x 14336 164 /
@@ -590,27 +603,31 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         s.k = K;
         s.acc = acc;
         s.wrows = N;
-        s.rows = rows16;
-        s.mt = cdiv(t1, 128);
-        const uint32_t nb = K / 256, tiles = s.mt * cdiv(N, 128), slots = 2 * (uint32_t)(g_cus > 0 ? g_cus : 1);
-        const uint64_t xs_bytes = sk_bytes(rows16, K);
+        const uint32_t nb = K / 256, tiles = cdiv(t1, 128) * cdiv(N, 128), slots = 2 * (uint32_t)(g_cus > 0 ? g_cus : 1);
+        const uint32_t step = pass_rows(rows16, K);
+        const uint64_t xs_bytes = sk_bytes(step, K);
         uint32_t ns = 1;  // K splits: while the tiles leave half the places idle and a split keeps two blocks
         while (tiles * ns * 2 <= slots && nb / (ns * 2) >= 2) ns *= 2;
         uint64_t ws_bytes;
         for (;;) {
             s.kb = cdiv(nb, ns);
             ns = cdiv(nb, s.kb);
-            ws_bytes = ns > 1 ? 4ull * ns * rows16 * N : 0;
+            ws_bytes = ns > 1 ? 4ull * ns * step * N : 0;
             if (!g_noalloc || ns == 1 || xs_bytes + ws_bytes <= QP_SCRATCH_BYTES) break;
             ns /= 2;
         }
         if (int e = workspace(xs_bytes + ws_bytes, &s.xs)) return e;
         s.ws = ns > 1 ? s.xs + xs_bytes : 0;
-        if (int e = tile_input(a.x, s.xs, a.paso, K, rows16, tmax, c.U(4) == 1, xplanes)) return e;
-        if (int e = run_tile(fmt, s, false, ns)) return e;
-        if (ns == 1) return 0;
-        QpReduceArgs ra = {s.ws, a.y, a.paso, N, rows16, ns, acc};
-        return launch(K_gemm_reduce, grid_cap((uint64_t)tmax * N), 1, 1, 256, 0, ra);
+        for (s.tbase = 0; s.tbase < rows16; s.tbase += step, s.y += 4ull * step * N) {
+            s.rows = rows16 - s.tbase < step ? rows16 - s.tbase : step;
+            s.mt = cdiv(s.rows, 128);
+            if (int e = tile_input(a.x, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, xplanes, s.tbase)) return e;
+            if (int e = run_tile(fmt, s, false, ns)) return e;
+            if (ns == 1) continue;
+            QpReduceArgs ra = {s.ws, s.y, a.paso, N, s.rows, ns, acc, s.tbase, 0};
+            if (int e = launch(K_gemm_reduce, grid_cap((uint64_t)s.rows * N), 1, 1, 256, 0, ra)) return e;
+        }
+        return 0;
     }
     if (tmax >= 64 && !getenv_flag("QP_NO_MFMA")) {
         // matrix cores: 128 x 128 tiles (the kernel reads T from paso; tiles past it exit)
@@ -684,7 +701,7 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
                 return e;
             }
             if (ns == 1) return 0;
-            QpReduceArgs ra = {a.ws, a.y, a.paso, N, a.rows, ns, acc};
+            QpReduceArgs ra = {a.ws, a.y, a.paso, N, a.rows, ns, acc, 0, 0};
             return launch(K_gemm_reduce, grid_cap((uint64_t)tmax * N), 1, 1, 256, 0, ra);
         }
         if (fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K)
@@ -751,13 +768,17 @@ int op_matmul_glu(const Ctx& c, int fmt, const char* name) {
         s.n = N;
         s.k = K;
         s.wrows = N;
-        s.rows = rows16;
-        s.mt = cdiv(tmax, 128);
         s.kb = K / 256;
         s.yplanes = a.yplanes ? a.rows : 0;
-        if (int e = workspace(sk_bytes(rows16, K), &s.xs)) return e;
-        if (int e = tile_input(a.x, s.xs, a.paso, K, rows16, tmax, false, xp)) return e;
-        return run_tile(fmt, s, true, 1);
+        const uint32_t step = pass_rows(rows16, K);
+        if (int e = workspace(sk_bytes(step, K), &s.xs)) return e;
+        for (s.tbase = 0; s.tbase < rows16; s.tbase += step, s.y += (s.yplanes ? 16ull : 4ull * N) * step) {
+            s.rows = rows16 - s.tbase < step ? rows16 - s.tbase : step;
+            s.mt = cdiv(s.rows, 128);
+            if (int e = tile_input(a.x, s.xs, a.paso, K, s.rows, tmax, false, xp, s.tbase)) return e;
+            if (int e = run_tile(fmt, s, true, 1)) return e;
+        }
+        return 0;
     }
     // One workgroup per CU (the kernel takes the whole LDS), so the tiles run in rounds of g_cus.  When the last
     // round would leave at least half the CUs idle, its tiles run as K halves instead (two items each, the second to

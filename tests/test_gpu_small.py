@@ -161,6 +161,42 @@ def test_many_tokens_swiglu(quipu, dev, oracle, fmt, T, N, K):
     assert np.all(np.abs(got[:T] - silu * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(silu) * bu + 2.0 ** -20 * np.abs(silu * u))
 
 
+@pytest.mark.parametrize("op,fmt", [("t", capi.F32), ("4", capi.F32), ("t", capi.Q4_K), ("swiglu", capi.Q4_K)])
+def test_operands_past_4_gib(quipu, dev, oracle, op, fmt):
+    """62720 token rows of K = 15360 (their operands would take 4.5 GB, past the kernels' offsets): every row like any other.
+    All rows are ones but for some at the edges of the passes that such a call is made in and of 4 GiB."""
+    T, N, K = 62720, 16, 15360
+    rows = np.array([0, 1, 30847, 30848, 30849, 61695, 61696, 62143, 62144, T - 1])
+    rng = np.random.default_rng(88)
+    xs = (rng.standard_normal((len(rows), K)) / np.sqrt(K)).astype(np.float32)
+    raw = [raw_matrix(fmt, N, K, 89 + i) for i in range(2)]
+    hw = [dev.matrix(fmt, r, N, K) for r in raw]
+    x, y = quipu.alloc(4 * T * K), dev.buf(np.full((T + 1, N), 7.0, np.float32))
+    dev.hs.append(x)
+    quipu.dispatch("fill_u32", [("u", 0x38000000), ("u", T * K), ("u", 0)], [0, x])  # 2^-15
+    for r, v in zip(rows, xs):
+        quipu.upload(x, v, int(r) * 4 * K)
+    p = dev.paso(T, 0)
+    name = "matmul_%s_t_swiglu" % capi.FMT_NAME[fmt] if op == "swiglu" else "matmul_%s_%s" % (capi.FMT_NAME[fmt], op)
+    grid = capi.dim2((N + 7) // 8) + ((T + 3) // 4,) if op == "4" else ((N + 63) // 64, 1, (T + 31) // 32)
+    quipu.dispatch(name, [("u", N), ("u", K), ("u", 0), ("u", 0)], [p] + hw[:2 if op == "swiglu" else 1] + [x, y], grid)
+    got = dev.get(y, (T + 1, N))
+    assert np.all(got[T] == 7.0)
+    other = np.ones(T, bool)
+    other[rows] = False
+    assert np.all(got[:T][other] == got[2])
+    x64 = np.vstack([xs, np.full((1, K), 2.0 ** -15, np.float32)])
+    got = np.vstack([got[rows], got[2:3]])
+    W = [weights(oracle, fmt, r, N, K) for r in raw]
+    g, u = (x64.astype(np.float64) @ w.T for w in W)
+    bg, bu = ((bound if fmt == capi.F32 else split_bound)(w, x64) for w in W)
+    if op != "swiglu":
+        assert np.all(np.abs(got - g) <= bg)
+        return
+    silu = g / (1 + np.exp(-np.clip(g, -700, None)))
+    assert np.all(np.abs(got - silu * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(silu) * bu + 2.0 ** -20 * np.abs(silu * u))
+
+
 @pytest.mark.parametrize("fmt", KQ)
 def test_many_jobs_per_expert(quipu, dev, oracle, fmt):
     """matmul_<fmt>_eg in tiles of 128 jobs: more than 64 experts (their counts are scanned 64 at a time), some without jobs,

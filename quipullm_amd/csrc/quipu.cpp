@@ -1299,9 +1299,13 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
     const uint32_t per_tok = tfijo > 1 ? tfijo : m ? m : 8;
     const uint64_t max_jobs = 32ull * tz * per_tok;
     const bool few = (max_jobs < a.nlst ? max_jobs : a.nlst) <= (is_kq(fmt) ? 24ull : 64ull) * E;
-    if (!g_capturing && !g_noalloc && !getenv_flag("QP_NO_MFMA") && (few || is_kq(fmt))) {
-        // (without P[4]: every row of x that a job of y can read)
-        const uint64_t rows = m ? (uint64_t)32 * tz * m : ((uint64_t)a.yrows + tfijo - 1) / tfijo;
+    // The rows to convert: T * P[4]; without it every row of x that a job of y can read, which the buffers' room tells, where
+    // that is no more than the dispatch's tokens have (buffers made for this call).  Larger buffers, and operands that the
+    // kernels' 31-bit offsets do not reach, take the tiles below, which read the listed rows of x and nothing else.
+    const uint64_t room = m ? (uint64_t)32 * tz * m : ((uint64_t)a.yrows + tfijo - 1) / tfijo;
+    const uint64_t rows = room < a.xrows ? room : a.xrows;
+    const bool whole = (m || rows <= 32ull * tz * (tfijo > 1 ? 1 : 8)) && (rows + 15) / 16 * sk_bytes(16, K) < (1ull << 31);
+    if (!g_capturing && !g_noalloc && !getenv_flag("QP_NO_MFMA") && (few || is_kq(fmt)) && whole) {
         QpSkArgs s = {};
         s.w = a.w;
         s.y = a.y;
@@ -1315,7 +1319,7 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
         s.tfijo = tfijo;
         s.yrows = a.yrows;
         s.nlst = a.nlst;
-        s.xrows = (uint32_t)(rows < a.xrows ? rows : a.xrows);
+        s.xrows = (uint32_t)rows;
         s.rows = cdiv(s.xrows, 16) * 16;
         if (int e = workspace(sk_bytes(s.rows, K), &s.xs)) return e;
         if (int e = split_input(a.x, s.xs, a.paso, K, s.rows, s.rows, c.U(5) == 1, m ? m : s.xrows, s.xrows, 0)) return e;

@@ -225,6 +225,43 @@ def test_many_jobs_per_expert(quipu, dev, oracle, fmt):
             assert np.all(np.abs(outs[0][js] - xe.astype(np.float64) @ W[e].T) <= bound(W[e], xe)), e
 
 
+@pytest.mark.parametrize("fmt,T", [(capi.Q4_K, 5), (capi.Q4_K, 100), (capi.Q8_0, 5), (capi.F32, 5)])
+@pytest.mark.parametrize("m", [0, 1])
+def test_grouped_matmul_in_large_buffers(quipu, dev, oracle, fmt, T, m):
+    """matmul_<fmt>_eg on the first rows of buffers with room for 3.7 million (whose operands would take 4 GiB and 2 KB): the
+    listed jobs' results, and no workspace that follows the room."""
+    import ctypes
+    E, N, K, k = 3, 20, 256, 2
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    rng = np.random.default_rng(90)
+    sel = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32).ravel()
+    raw = raw_matrix(fmt, E * N, K, 91)
+    W = weights(oracle, fmt, raw, E * N, K).reshape(E, N, K)
+    hw = dev.matrix(fmt, raw, E * N, K)
+    wb = [hw, capi.scale_plane(fmt, hw, E * N, K)] if fmt in PLANAR else [hw]
+    rows = 233017 * 16
+    x, y, lb = quipu.alloc(4 * rows * K), quipu.alloc(4 * rows * k * N), quipu.alloc(4 * 60000)
+    dev.hs += [x, y, lb]
+    sb, ob, p = dev.buf(sel), dev.zeros(4 * (E + 1)), dev.paso(T, 0)
+    xs = rng.standard_normal((T, K)).astype(np.float32)
+    quipu.upload(x, xs)
+    quipu.dispatch("moe_group", [("u", E), ("u", k)], [p, sb, lb, ob])
+    quipu.sync()
+    before = free_bytes()
+    quipu.dispatch("matmul_%s_eg" % capi.FMT_NAME[fmt], [("u", N), ("u", K), ("u", 0), ("u", k)] + [("u", m)] * (m > 0),
+                   [p] + wb + [x, y, lb, ob], ((N + 63) // 64, E, (T + 31) // 32))
+    got = dev.get(y, (T * k, N))
+    assert before - free_bytes() < 1 << 28
+    for j in range(T * k):
+        xr = xs[j // k][None]
+        assert np.all(np.abs(got[j] - (xr.astype(np.float64) @ W[sel[j]].T)[0]) <= split_bound(W[sel[j]], xr)[0]), j
+
+
 @pytest.mark.parametrize("f16", [0, 1])
 @pytest.mark.parametrize("hd,nh,nkv,T,pos0,swa,cap", [
     (128, 8, 8, 1, 0, 0, 0),          # one key

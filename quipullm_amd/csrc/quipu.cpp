@@ -472,11 +472,16 @@ int split_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t row
 // Bytes of the operands and scales of `rows` rows (a multiple of 16) of K inputs.
 uint64_t sk_bytes(uint32_t rows, uint32_t K) { return (uint64_t)(rows / 16) * cdiv(K, 256) * (18 * 1024 + 64); }
 
-// Rows of one pass of a dense matmul of rows16 rows (a multiple of 16): all, or as many whole 128s as have operands that
-// the kernels' 31-bit offsets reach (QP_NOOFF, the offset of lanes without work, must lie past them): 30,848 rows at
-// K = 15360.
-uint32_t pass_rows(uint32_t rows16, uint32_t K) {
+// 16-row tiles of operands that the kernels' 31-bit offsets reach (QP_NOOFF, the offset of lanes without work, must lie past
+// them) and that qp_split_f16's grid takes.
+uint64_t max_tiles(uint32_t K) {
     const uint64_t fit = ((1ull << 31) - 1) / sk_bytes(16, K);
+    return fit < 65535 ? fit : 65535;
+}
+// Rows of one pass of a dense matmul of rows16 rows (a multiple of 16): all, or as many whole 128s as one pass can take
+// (30,848 at K = 15360).
+uint32_t pass_rows(uint32_t rows16, uint32_t K) {
+    const uint64_t fit = max_tiles(K);
     return rows16 <= fit * 16 ? rows16 : (uint32_t)(fit / 8 * 128);
 }
 
@@ -1304,7 +1309,7 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
     // kernels' 31-bit offsets do not reach, take the tiles below, which read the listed rows of x and nothing else.
     const uint64_t room = m ? (uint64_t)32 * tz * m : ((uint64_t)a.yrows + tfijo - 1) / tfijo;
     const uint64_t rows = room < a.xrows ? room : a.xrows;
-    const bool whole = (m || rows <= 32ull * tz * (tfijo > 1 ? 1 : 8)) && (rows + 15) / 16 * sk_bytes(16, K) < (1ull << 31);
+    const bool whole = (m || rows <= 32ull * tz * (tfijo > 1 ? 1 : 8)) && (rows + 15) / 16 <= max_tiles(K);
     if (!g_capturing && !g_noalloc && !getenv_flag("QP_NO_MFMA") && (few || is_kq(fmt)) && whole) {
         QpSkArgs s = {};
         s.w = a.w;

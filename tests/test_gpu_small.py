@@ -197,6 +197,16 @@ def test_operands_past_4_gib(quipu, dev, oracle, op, fmt):
     assert np.all(np.abs(got - silu * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(silu) * bu + 2.0 ** -20 * np.abs(silu * u))
 
 
+def test_more_than_a_million_rows(quipu, dev):
+    """1050000 token rows: more 16-row tiles than a launch's grid takes in one dimension."""
+    T, N, K = 1050000, 4, 16
+    rng = np.random.default_rng(92)
+    raw = raw_matrix(capi.F32, N, K, 93)
+    x = rng.standard_normal((T, K), dtype=np.float32)
+    W = raw.view(np.float32).reshape(N, K).astype(np.float64)
+    assert np.all(np.abs(matmul(quipu, dev, capi.F32, raw, N, K, x) - x.astype(np.float64) @ W.T) <= bound(W, x))
+
+
 @pytest.mark.parametrize("fmt", KQ)
 def test_many_jobs_per_expert(quipu, dev, oracle, fmt):
     """matmul_<fmt>_eg in tiles of 128 jobs: more than 64 experts (their counts are scanned 64 at a time), some without jobs,

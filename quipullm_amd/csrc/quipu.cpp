@@ -479,10 +479,19 @@ uint64_t max_tiles(uint32_t K) {
     return fit < 65535 ? fit : 65535;
 }
 // Rows of one pass of a dense matmul of rows16 rows (a multiple of 16): all, or as many whole 128s as one pass can take
-// (30,848 at K = 15360).
+// (30,848 at K = 15360; in qp_dispatch_noalloc's scratch 384).
 uint32_t pass_rows(uint32_t rows16, uint32_t K) {
-    const uint64_t fit = max_tiles(K);
+    const uint64_t most = max_tiles(K), hold = QP_SCRATCH_BYTES / sk_bytes(16, K), fit = g_noalloc && hold < most ? hold : most;
     return rows16 <= fit * 16 ? rows16 : (uint32_t)(fit / 8 * 128);
+}
+
+// qp_dispatch_noalloc takes a dense matmul whose operands its scratch holds at once, one that reads input planes, and one
+// whose rows would fit it as input planes (4 bytes per input, rows in whole 128s or 256s), in passes.
+int noalloc_room(const char* name, uint32_t rows16, uint32_t K, uint32_t tmax, uint32_t whole) {
+    const uint64_t bytes = 4ull * cdiv(tmax, whole) * whole * ((K + 31) / 32 * 32);
+    if (!g_noalloc || sk_bytes(rows16, K) <= QP_SCRATCH_BYTES || bytes <= QP_SCRATCH_BYTES) return 0;
+    return fail(QP_E_ARG, "qp_dispatch_noalloc: %s needs %llu bytes of workspace; the scratch holds %u (fewer tokens per call)", name,
+                (unsigned long long)bytes, QP_SCRATCH_BYTES);
 }
 
 Kid sk_kid(int fmt, uint32_t nt, uint32_t R) {
@@ -572,8 +581,8 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         return fail(QP_E_ARG, "%s: P[4] = 2 (x holds input planes) needs K-quant weights and a chunk of 256 tokens "
                               "or more on the matrix cores", name);
     const uint32_t t1 = tmax ? tmax : 1, rows16 = cdiv(t1, 16) * 16;
-    if (!xplanes && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") && sk_takes(fmt, t1, N, K) &&
-        (!g_noalloc || sk_bytes(cdiv(t1, 16) * 16, K) <= QP_SCRATCH_BYTES)) {
+    if (!xplanes && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") && sk_takes(fmt, t1, N, K)) {
+        if (int e = noalloc_room(name, rows16, K, tmax, 128)) return e;
         QpSkArgs s = {};
         s.w = a.w;
         s.y = a.y;
@@ -592,14 +601,15 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         }
         return 0;
     }
-    // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip), where qp_dispatch_noalloc's scratch holds
-    // X's operands.  Against the tiles below at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 108 / 183 / 340 /
+    // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip).  Against the tiles below at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 108 / 183 / 340 /
     // 597 against 133 / 224 / 383 / 720, 1024 x 4096 32 / 35 / 51 / 75 against 31 / 39 / 54 / 84; Q6_K 4096 x 14336 164 /
     // 263 / 455 / 830 against 150 / 270 / 479 / 840; Q5_K 14336 x 4096 118 / 201 / 362 / 632 against 143 / 237 / 424 / 791.
-    if (is_kq(fmt) && tmax > 64 && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") &&
-        (!g_noalloc || sk_bytes(rows16, K) <= QP_SCRATCH_BYTES)) {
-        if (xplanes)
+    if (is_kq(fmt) && tmax > 64 && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA")) {
+        if (xplanes) {
             if (int e = need_room(a.x, 4ull * cdiv(t1, 256) * 256 * K, name, "the input planes' buffer")) return e;
+        } else if (int e = noalloc_room(name, rows16, K, tmax, tmax >= 256 || fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K ? 256 : 128)) {
+            return e;
+        }
         QpTileArgs s = {};
         s.w = a.w;
         s.y = a.y;
@@ -759,12 +769,14 @@ int op_matmul_glu(const Ctx& c, int fmt, const char* name) {
         if (int e = need_room(a.y, 4ull * a.rows * N, name, "the output planes' buffer")) return e;
     }
     const uint32_t rows16 = cdiv(tmax, 16) * 16;
-    // Integer weights in tiles of 128 tokens x (64 gate + 64 up) rows (qp_tile.hip), where qp_dispatch_noalloc's scratch
-    // holds X's operands: 14336 x 4096 of Q4_K at 2048 tokens 1208 us against 1320, of Q5_K at 333 334 against 357.
-    if (!g_noalloc || sk_bytes(rows16, K) <= QP_SCRATCH_BYTES) {
+    // Integer weights in tiles of 128 tokens x (64 gate + 64 up) rows (qp_tile.hip): 14336 x 4096 of Q4_K at 2048 tokens 1208 us against 1320, of Q5_K at 333 334 against 357.
+    {
         const bool xp = c.U(3) == 1;
-        if (xp)
+        if (xp) {
             if (int e = need_room(a.x, 4ull * a.rows * K, name, "the input planes' buffer")) return e;
+        } else if (int e = noalloc_room(name, rows16, K, tmax, 256)) {
+            return e;
+        }
         QpTileArgs s = {};
         s.w = a.w;
         s.w2 = a.w2;
@@ -1289,10 +1301,11 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
     a.tpe = cdiv(32 * tz, 128);
     if ((uint64_t)E * a.tpe > 65535) return fail(QP_E_ARG, "%s: %u experts x %u job tiles", name, E, a.tpe);
     // P[4] = m (not a reference word; absent: 0): x holds m rows per token (1: gate/up, whose job j reads token
-    // row j / tfijo; the top-k count: down, job rows), and its first T * m rows are split into bf16 planes once
-    // (row-major: a tile gathers rows), which every tile then copies instead of loading and splitting f32 rows (the
-    // same planes: the sums are bit-equal).  P[5] = 1: the previous matmul split the same x (see split_input).  Not while capturing a graph or
-    // under qp_dispatch_noalloc (the planes need the workspace): there x is split in the tiles as without P[4].
+    // row j / tfijo; the top-k count: down, job rows), and its first T * m rows are converted once, to the integer
+    // weights' operands or for the tiles below to bf16 planes (row-major: a tile gathers rows), which every tile then
+    // copies.  P[5] = 1: the previous matmul split the same x (see split_input).  While capturing a graph and under
+    // qp_dispatch_noalloc (both need the workspace) the tiles below split the f32 rows that they read themselves: bf16
+    // parts, as the planes, so those two give the same bits; the integer weights' sums differ within the error bound.
     const uint32_t m = c.U(4);
     // Integer weights: few jobs per expert in token tiles of 16 (qp_small.hip), more of K-quants in tiles of 128 jobs x
     // 128 rows (qp_tile.hip).  Jobs per token: tfijo of the gate and up products, P[4] of the down product (8 where it

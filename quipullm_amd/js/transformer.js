@@ -103,9 +103,10 @@ class ModeloTransformer {
     // K-quant matmuls that read it (rmsnorm_planes; Q, K, V with P[4] = 2, the fused gate/up with P[3] = 1) instead
     // of f32 rows that each matmul splits; false: rmsnorm
     this.planosNorma = op.norm_planes !== false;
-    // MoE prompt batches grouped by expert: each expert matmul's input split into bf16 planes once (matmul_<fmt>_eg
-    // P[4] = rows per token: 1 for gate and up, the top-k count for down; up reuses gate's planes, P[5] = 1) instead
-    // of in every tile that reads a row; the same sums bit for bit.  false: f32 rows split in the tiles
+    // MoE prompt batches grouped by expert: each expert matmul's input converted to matrix operands once
+    // (matmul_<fmt>_eg P[4] = rows per token: 1 for gate and up, the top-k count for down; up reuses gate's, P[5] = 1)
+    // instead of in every tile that reads a row.  false: without P[4], by the backend's rule for such calls (the same
+    // results within the matmul's error bound)
     this.planosMoe = op.moe_planes !== false;
     // one-token step: the split-K attention's partials merged by the last workgroup of each grid column in the same
     // launch (dec_attn P[12] = 1) instead of a dec_attn_comb launch.  A column takes at most 4 query heads: groups of

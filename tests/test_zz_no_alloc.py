@@ -165,6 +165,40 @@ def test_noalloc_matches_dispatch(quipu, fmt, N, K, Ts):
         b.close()
 
 
+@pytest.mark.parametrize("planes", [0, 1])
+def test_noalloc_in_passes_matches_dispatch(quipu, planes):
+    """2048 tokens at K = 4096 and 4352: the rows fit the scratch as input planes (or are given as planes), but the matmuls'
+    operands (4.5 bytes per input) do not, so they run in two passes.  Bit for bit qp_dispatch's results: the plain
+    matmul, the fused gate/up, and with planes the chain rmsnorm, gate/up and down that hands planes on."""
+    fmt, D, F, T = capi.Q4_K, 4096, 4352, 2048
+    b = Bufs(quipu)
+    try:
+        wg, wu, wd = b.matrix(fmt, F, D, 14), b.matrix(fmt, F, D, 15), b.matrix(fmt, D, F, 16)
+        x = np.random.default_rng(80).standard_normal((T, D)).astype(np.float32)
+        if not planes:
+            for f, args in ((matmul, (wg,)), (glu, (wg, wu))):
+                want, got = (f(quipu, b, fmt, *args, F, D, T, x, n) for n in (False, True))
+                assert np.isfinite(got).all()
+                np.testing.assert_array_equal(got, want)
+            return
+        paso, xb, nw = b.put(np.array([T, 0, 0, 0], np.uint32)), b.put(x), b.put(np.ones(D, np.float32))
+        xs, h = b.put(np.zeros(T * D, np.float32)), b.put(np.zeros(T * F, np.float32))
+        quipu.dispatch("rmsnorm_planes", [("u", D), ("f", 1e-5)], [paso, xb, nw, xs], (T // 8,))
+        outs = []
+        for n in (False, True):
+            y = b.put(np.full((T, D), 3.0, np.float32))
+            quipu.upload(h, np.zeros(T * F, np.float32))
+            quipu.dispatch("matmul_q4k_t_swiglu", [("u", F), ("u", D), ("u", 1), ("u", 1)], [paso, wg, wu, xs, h],
+                           (F // 64, 1, T // 32), noalloc=n)
+            quipu.dispatch("matmul_q4k_t", [("u", D), ("u", F), ("u", 1), ("u", 0), ("u", 2)], [paso, wd, h, y],
+                           (D // 64, 1, T // 32), noalloc=n)
+            outs.append(quipu.download(y, (T, D)))
+        assert np.isfinite(outs[1]).all() and not np.any(outs[1] == 3.0)
+        np.testing.assert_array_equal(outs[1], outs[0])
+    finally:
+        b.close()
+
+
 def test_noalloc_rejects_a_workspace_past_the_scratch(quipu):
     b = Bufs(quipu)
     try:

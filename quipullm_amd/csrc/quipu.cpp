@@ -508,10 +508,14 @@ Kid sk_kid(int fmt, uint32_t nt, uint32_t R) {
     return r1[fmt == QP_Q8_0 ? 5 : fmt == QP_IQ4_NL ? 6 : 7][t];
 }
 
+// K slices per workgroup (K-quants: of whole groups of four blocks).
+uint32_t sk_slices(int fmt, uint32_t K) {
+    const uint32_t nch = cdiv(K, 256), units = is_kq(fmt) ? cdiv(nch, 4) : nch;
+    return units >= 4 ? 4 : units >= 2 ? 2 : 1;
+}
 // a: everything but the split of the work, in token blocks of 16 nt rows, tpe slots of them and E experts (dense: 1).
 int run_sk(int fmt, QpSkArgs& a, uint32_t nt, uint32_t tpe, uint32_t E, uint32_t R) {
-    const uint32_t nch = cdiv(a.k, 256), units = is_kq(fmt) ? cdiv(nch, 4) : nch;
-    a.kw = units >= 4 ? 4 : units >= 2 ? 2 : 1;
+    a.kw = sk_slices(fmt, a.k);
     a.tpe = tpe;
     const uint32_t gx = cdiv(a.n, 16 * R * (4 / a.kw));
     const uint32_t lds = a.kw > 1 ? 4 * R * nt * 64 * 16 : 0;
@@ -528,10 +532,19 @@ int run_sk(int fmt, QpSkArgs& a, uint32_t nt, uint32_t tpe, uint32_t E, uint32_t
 //     Q8_0 11008 x 4096 at 64 / 128 tokens 59 / 103 against 66 / 73; 2816 x 1024 at 256 tokens 21 against 30;
 //   f32 always: 128 x 2048 (a router) at 64 / 2048 tokens 26 / 34 against 38 / 50, 4096 x 4096 49 / 689 against 71 / 738.
 // Below 64 tokens the other path is the vector-unit kernel (Q4_K 14336 x 4096 at 32 tokens 27 against 1120).
+//   K-quants from 256 tokens on: while the workgroups are no more than the CUs and tokens times K slices no more than 2048
+//     (a workgroup of more slices reads the operands of fewer rows each time; qp_tile.hip's tiles leave CUs idle there or
+//     add K splits; in parentheses the 256-token tiles of bf16 parts that both replaced): Q4_K 1024 x 4096 at 256 / 512 tokens
+//     23 / 28 against 32 / 33 (30 / 39), 768 x 2048 at 256 / 1024 / 2048 20 / 28 / 47 against 28 / 34 / 43 (26 / 32 / 45), 2816
+//     x 1024 at 512 / 768 24 / 40 against 34 / 39 (29 / 38); Q6_K 2048 x 2048 at 256 / 512 30 / 32 against 37 / 38 (30 / 37);
+//     Q2_K 512 x 4096 at 512 / 768 27 / 41 against 33 / 33 (35 / 38).
+uint32_t sk_rows(int fmt, uint32_t nt, uint32_t yb, uint32_t N);
 bool sk_takes(int fmt, uint32_t tmax, uint32_t N, uint32_t K) {
-    if (fmt == QP_F32) return true;
-    if (is_kq(fmt)) return tmax <= 64 || (tmax < 256 && (uint64_t)N * K < 32u << 20);
-    return tmax <= 64 || (tmax < 256 && (uint64_t)N * K * cdiv(tmax, 64) <= 12u << 20);
+    if (fmt == QP_F32 || tmax <= 64) return true;
+    if (!is_kq(fmt)) return tmax < 256 && (uint64_t)N * K * cdiv(tmax, 64) <= 12u << 20;
+    if (tmax < 256) return (uint64_t)N * K < 32u << 20;
+    const uint32_t yb = cdiv(tmax, 64), kw = sk_slices(fmt, K), wgs = cdiv(N, 16 * sk_rows(fmt, 4, yb, N) * (4 / kw)) * yb;
+    return wgs <= (uint32_t)g_cus && tmax * kw <= 2048;
 }
 // 16-row tiles per wavefront: two where that leaves enough workgroups (X is read once per 16 R rows): 8192 rows times
 // 64-token blocks (Q4_K 14336 x 4096 at 32 tokens 27 against 36 us with one; 4096 x 4096 18.6 against 14.9).  Q8_0 and
@@ -550,7 +563,7 @@ int run_tile(int fmt, QpTileArgs& a, bool glu, uint32_t ns) {
     const uint32_t lds = 2 * 17408 + (fmt == QP_Q6_K ? 32768 : 16384) + 8192 + 4096 + 1024 + 512;  // (qp_tile.hip's)
     return launch(kt[glu][kq_index(fmt)], 8 * cdiv((uint64_t)a.mt * a.nt, 8), 1, ns, 256, lds, a);
 }
-// X of a dense K-quant matmul's tiles as operands.  From 256 tokens on (where a caller's input planes may take the place
+// X of a dense K-quant matmul as operands.  From 256 tokens on (where a caller's input planes may take the place
 // of the f32 rows: planes, rows in whole 256s) by way of the rows' bf16 high + low parts, so that both give the same bits.
 // Token tbase on, tmax of them in all (a token's 16 bytes of a plane's 8 inputs lie side by side).
 int tile_input(uint64_t x, uint64_t xs, uint64_t paso, uint32_t K, uint32_t rows, uint32_t tmax, bool reuse, bool planes, uint32_t tbase) {
@@ -581,8 +594,11 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         return fail(QP_E_ARG, "%s: P[4] = 2 (x holds input planes) needs K-quant weights and a chunk of 256 tokens "
                               "or more on the matrix cores", name);
     const uint32_t t1 = tmax ? tmax : 1, rows16 = cdiv(t1, 16) * 16;
-    if (!xplanes && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") && sk_takes(fmt, t1, N, K)) {
-        if (int e = noalloc_room(name, rows16, K, tmax, 128)) return e;
+    if (xplanes)
+        if (int e = need_room(a.x, 4ull * cdiv(t1, 256) * 256 * K, name, "the input planes' buffer")) return e;
+    if ((!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA") && sk_takes(fmt, t1, N, K)) {
+        if (!xplanes)
+            if (int e = noalloc_room(name, rows16, K, tmax, is_kq(fmt) && tmax >= 256 ? 256 : 128)) return e;
         QpSkArgs s = {};
         s.w = a.w;
         s.y = a.y;
@@ -595,7 +611,8 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         if (int e = workspace(sk_bytes(step, K), &s.xs)) return e;
         for (s.tbase = 0; s.tbase < rows16; s.tbase += step, s.y += 4ull * step * N) {
             s.rows = rows16 - s.tbase < step ? rows16 - s.tbase : step;
-            if (int e = split_input(a.x + 4ull * s.tbase * K, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, 0, 0, s.tbase))
+            if (int e = is_kq(fmt) ? tile_input(a.x, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, xplanes, s.tbase)
+                                   : split_input(a.x + 4ull * s.tbase * K, s.xs, a.paso, K, s.rows, tmax, c.U(4) == 1, 0, 0, 0, 0, s.tbase))
                 return e;
             if (int e = run_sk(fmt, s, nt, cdiv(s.rows, 16 * nt), 1, R)) return e;
         }
@@ -605,11 +622,9 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
     // 597 against 133 / 224 / 383 / 720, 1024 x 4096 32 / 35 / 51 / 75 against 31 / 39 / 54 / 84; Q6_K 4096 x 14336 164 /
     // 263 / 455 / 830 against 150 / 270 / 479 / 840; Q5_K 14336 x 4096 118 / 201 / 362 / 632 against 143 / 237 / 424 / 791.
     if (is_kq(fmt) && tmax > 64 && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA")) {
-        if (xplanes) {
-            if (int e = need_room(a.x, 4ull * cdiv(t1, 256) * 256 * K, name, "the input planes' buffer")) return e;
-        } else if (int e = noalloc_room(name, rows16, K, tmax, tmax >= 256 || fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K ? 256 : 128)) {
-            return e;
-        }
+        if (!xplanes)
+            if (int e = noalloc_room(name, rows16, K, tmax, tmax >= 256 || fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K ? 256 : 128))
+                return e;
         QpTileArgs s = {};
         s.w = a.w;
         s.y = a.y;

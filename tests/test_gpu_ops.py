@@ -9,6 +9,7 @@ on the host before any launch).
 """
 import numpy as np
 import pytest
+import torch
 
 import refs
 from quipullm_amd import capi, synth
@@ -303,22 +304,36 @@ def test_matmul_prefill_mfma(quipu, dev, oracle, fmt, T, N, K, acc):
 KQ_FMTS = [capi.Q2_K, capi.Q3_K, capi.Q4_K, capi.Q5_K, capi.Q6_K]
 
 
+def input_planes(x):
+    """x [T][K] as the matmuls' bf16 input planes: high parts, then low parts, [K / 8][rows][8], rows a multiple of 256
+    (those past T hold NaN: they must not be read into a result)."""
+    T, K = x.shape
+    rows = -(-T // 256) * 256
+    t = torch.from_numpy(x)
+    hi = t.bfloat16()
+    out = np.full((2, K // 8, rows, 8), 0x7fff, np.uint16)
+    for p, v in enumerate((hi, (t - hi.float()).bfloat16())):
+        out[p, :, :T] = v.view(torch.int16).numpy().view(np.uint16).reshape(T, K // 8, 8).transpose(1, 0, 2)
+    return out
+
+
 @pytest.mark.parametrize("fmt", KQ_FMTS)
-@pytest.mark.parametrize("tiles", ["wide", "narrow"])
+@pytest.mark.parametrize("x_as", ["rows", "planes"])
 @pytest.mark.parametrize("T,N,K,acc", [(256, 300, 2048, 1), (512, 520, 1024, 0), (300, 700, 4864, 1),
-                                        (768, 256, 512, 0)])
-def test_matmul_prefill_tile_kinds(quipu, dev, oracle, monkeypatch, fmt, tiles, T, N, K, acc):
-    """Both K-quant tile kinds from 256 tokens on, forced (QP_GEMM_TILES): 256 x 256 tiles (8 wavefronts of 128
-    tokens x 64 rows, each thread staging two weight rows) and 256 x 128 tiles, at partial token and row tiles,
-    small grids split along K (the last split partial at K = 4864, 19 blocks)."""
-    monkeypatch.setenv("QP_GEMM_TILES", tiles)
+                                        (768, 256, 512, 0), (600, 700, 4864, 1), (2048, 1100, 256, 0)])
+def test_matmul_prefill_tile_kinds(quipu, dev, oracle, fmt, x_as, T, N, K, acc):
+    """Both K-quant kernels from 256 tokens on, from f32 rows and from given input planes (P[4] = 2): matrices of so few
+    workgroups that each wavefront keeps its weights, and (the last two shapes) 128 x 128 tiles, at partial token and
+    row tiles, small grids split along K (the last split partial at K = 4864, 19 blocks)."""
     raw = raw_matrix(fmt, N, K, 67)
     W = oracle.dequant(fmt, raw, N * K).reshape(N, K)
     x = (np.random.default_rng(14).standard_normal((T, K)) * 3).astype(np.float32)
     y0 = np.random.default_rng(15).standard_normal((T, N)).astype(np.float32)
     y = dev.buf(y0)
-    quipu.dispatch("matmul_%s_t" % capi.FMT_NAME[fmt], [("u", N), ("u", K), ("u", acc), ("u", 0)],
-                   [dev.paso(T, 0), dev.matrix(fmt, raw, N, K), dev.buf(x), y], ((N + 63) // 64, 1, (T + 31) // 32))
+    planes = x_as == "planes"
+    quipu.dispatch("matmul_%s_t" % capi.FMT_NAME[fmt], [("u", N), ("u", K), ("u", acc), ("u", 0), ("u", 2 * planes)],
+                   [dev.paso(T, 0), dev.matrix(fmt, raw, N, K), dev.buf(input_planes(x) if planes else x), y],
+                   ((N + 63) // 64, 1, (T + 31) // 32))
     got = dev.get(y, (T, N))
     want = (W.astype(np.float64) @ x.astype(np.float64).T).T + (y0 if acc else 0)
     bound = (np.abs(W.astype(np.float64)) @ np.abs(x.astype(np.float64)).T).T * 2e-5 + 2e-7 * np.abs(y0) + 1e-30

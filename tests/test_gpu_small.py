@@ -125,13 +125,13 @@ KQ = [f for f in FMTS if f not in PLANAR and f != capi.F32]
 
 
 @pytest.mark.parametrize("fmt", KQ)
-@pytest.mark.parametrize("T,N,K", [(256, 128, 256), (257, 1, 512), (321, 129, 768), (383, 250, 1280), (448, 64, 2304),
-                                   (70, 8200, 4096)])
+@pytest.mark.parametrize("T,N,K", [
+    (256, 128, 256), (257, 1, 512), (321, 129, 768), (383, 250, 1280), (512, 512, 4096), (1000, 768, 2048),  # few workgroups
+    (2176, 1152, 256), (2049, 1100, 512), (577, 129, 3328), (513, 1, 4352), (832, 250, 5376)])               # 128 x 128 tiles
 def test_many_tokens(quipu, dev, oracle, fmt, T, N, K):
-    """The 128 x 128 tiles: whole ones, one row, one token and one row past a tile, tiles of at most 64 tokens, one block of
-    256 inputs, K splits with a shorter last one; a large matrix below 256 tokens."""
-    if N > 8000 and fmt != capi.Q4_K:
-        pytest.skip("one format is enough for the large matrix")
+    """256 tokens and more.  Matrices of so few workgroups that each wavefront keeps its weights (up to exactly a workgroup
+    per CU of 256): one block of 256 inputs to four K slices, one row, remainders.  The 128 x 128 tiles: whole ones, one row,
+    one token and one row past a tile, a tile of 64 tokens, one block of 256 inputs, K splits with a shorter last one."""
     raw = raw_matrix(fmt, N, K, 81)
     W = weights(oracle, fmt, raw, N, K)
     rng = np.random.default_rng(82)

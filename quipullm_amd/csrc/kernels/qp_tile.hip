@@ -58,7 +58,8 @@ QP_DEV void tile_body(const QpTileArgs& a) {
     const bool dense = GLU || !a.lst;
     const uint32_t in_xcd = blockIdx.x >> 3;
     if (dense) {  // eight row tiles at a time
-        const uint32_t total = a.mt * a.nt, chunk = (total + 7) / 8, L = (blockIdx.x & 7) * chunk + in_xcd;
+        const uint32_t parts = 8 / a.zx, total = a.mt * a.nt, chunk = (total + parts - 1) / parts;
+        const uint32_t L = (blockIdx.x & 7) / a.zx * chunk + in_xcd;
         if (in_xcd >= chunk || L >= total) return;
         const uint32_t grp = L / (a.mt * 8), rem = L % (a.mt * 8), in = min(8u, a.nt - grp * 8);
         t0 = (rem / in) * 128;
@@ -144,7 +145,8 @@ QP_DEV void tile_body(const QpTileArgs& a) {
         const uint32_t x = dense ? t0 + tid : jobs[tid] == QP_NOOFF ? 0 : jobs[tid] / a.tfijo;
         if (dense ? tid < cnt : jobs[tid] != QP_NOOFF) co = (x >> 4) * nb * 64 + (x & 15) * 4;
     }
-    const uint32_t b0 = blockIdx.z * a.kb, b1 = min(nb, b0 + a.kb);
+    const uint32_t split = a.zx > 1 ? (blockIdx.x & 7) % a.zx : blockIdx.z;
+    const uint32_t b0 = split * a.kb, b1 = min(nb, b0 + a.kb);
 
     u32x4 D[ND], H[NH > 0 ? NH : 1], hn;
     uint32_t ddn = 0;
@@ -391,7 +393,7 @@ QP_DEV void tile_body(const QpTileArgs& a) {
                     if (yr == QP_NOOFF) continue;
                 }
                 if (a.ws) {
-                    gstore<float>(a.ws + 4 * (((uint64_t)blockIdx.z * a.rows + yr) * a.n + n), tot[r][t][v]);
+                    gstore<float>(a.ws + 4 * (((uint64_t)split * a.rows + yr) * a.n + n), tot[r][t][v]);
                 } else {
                     const uint64_t o = a.y + 4 * ((uint64_t)yr * a.n + n);
                     gstore<float>(o, a.acc ? gload<float>(o) + tot[r][t][v] : tot[r][t][v]);

@@ -145,7 +145,8 @@ typedef struct {
 } QpSkArgs;
 
 // qp_tile_<fmt>, qp_tile_glu_<fmt> (K-quants, qp_tile.hip): 128 x 128 tiles, mt x nt of them (grouped by expert, lst != 0:
-// at most mt tiles of 128 jobs in nexp experts) in grid x (a multiple of 8), grid z K splits of kb blocks of 256 inputs.
+// at most mt tiles of 128 jobs in nexp experts) in grid x (a multiple of 8), grid z K splits of kb blocks of 256 inputs; zx
+// (1, 2, 4 or 8): above 1 the K splits are zx, in grid x, each on 8 / zx of the XCDs.
 // xs: X as operands (qp_split_f16) of `rows` rows.  ws: 0, or the splits' sums [splits][rows][n].  glu: w gate, w2 up, 64
 // rows of each per tile; yplanes: 0, or y receives the next matmul's input planes of that many token rows.  tbase: as above.
 typedef struct {
@@ -154,6 +155,7 @@ typedef struct {
     uint32_t mt, nt, kb, nexp;
     uint32_t tfijo, xrows, yrows, nlst;
     uint32_t yplanes, tbase;
+    uint32_t zx, pad;
 } QpTileArgs;
 
 // moe_group: lst[off[e] .. off[e + 1]) = the jobs i < T * n (in increasing order) with sel[i] == e, e < n_exp;

@@ -561,7 +561,13 @@ int run_tile(int fmt, QpTileArgs& a, bool glu, uint32_t ns) {
                                  {K_tile_glu_q4k, K_tile_glu_q5k, K_tile_glu_q6k, K_tile_glu_q3k, K_tile_glu_q2k}};
     a.nt = cdiv(a.n, glu ? 64 : 128);
     const uint32_t lds = 2 * 17408 + (fmt == QP_Q6_K ? 32768 : 16384) + 8192 + 4096 + 1024 + 512;  // (qp_tile.hip's)
-    return launch(kt[glu][kq_index(fmt)], 8 * cdiv((uint64_t)a.mt * a.nt, 8), 1, ns, 256, lds, a);
+    // Q6_K rows of 8192 inputs and more, whose 128 token rows of operands pass an XCD's L2 (4 MB), for two or more token tiles:
+    // the K splits are dealt to the XCDs, so that each reads its own slice of K for all tiles (4096 x 14336 at 192 / 256 / 512
+    // tokens 127 / 136 / 231 us, every XCD all splits of its own tiles 145 / 152 / 241; 5120 x 13824 187 / 198 / 343 against 192
+    // / 202 / 352).  Shorter rows and one token tile lose by it (14336 x 4096 at 128 tokens 96 against 86, 8192 x 2560 at 256 69
+    // against 63, 8192 x 8192 at 128 112 against 92), so do formats of fewer products (Q2_K 5120 x 13824 at 256 132 against 127).
+    a.zx = fmt == QP_Q6_K && a.mt > 1 && a.k >= 8192 && !a.lst && (ns == 2 || ns == 4 || ns == 8) ? ns : 1;
+    return launch(kt[glu][kq_index(fmt)], 8 * cdiv((uint64_t)a.mt * a.nt, 8 / a.zx), 1, a.zx > 1 ? 1 : ns, 256, lds, a);
 }
 // X of a dense K-quant matmul as operands.  From 256 tokens on (where a caller's input planes may take the place
 // of the f32 rows: planes, rows in whole 256s) by way of the rows' bf16 high + low parts, so that both give the same bits.
@@ -618,9 +624,12 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         }
         return 0;
     }
-    // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip).  Against the tiles below at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 108 / 183 / 340 /
-    // 597 against 133 / 224 / 383 / 720, 1024 x 4096 32 / 35 / 51 / 75 against 31 / 39 / 54 / 84; Q6_K 4096 x 14336 164 /
-    // 263 / 455 / 830 against 150 / 270 / 479 / 840; Q5_K 14336 x 4096 118 / 201 / 362 / 632 against 143 / 237 / 424 / 791.
+    // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip).  Against the 256-token tiles of bf16 high and
+    // low parts that they replaced, at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 95 / 153 / 290 / 560 against 109
+    // / 186 / 326 / 650, 4096 x 14336 105 / 163 / 296 / 561 against 116 / 206 / 375 / 681; Q6_K 4096 x 14336 130 / 216 / 401 /
+    // 770 against 129 / 228 / 416 / 781, 5120 x 13824 195 / 335 / 636 / 1049 against 185 / 334 / 612 / 1134.  Q6_K, whose weights
+    // take three products here too, gains no time (whole 256s of tokens lose up to 7 %: 4096 x 11008 at 256 112 against 104), but
+    // the sums are 2.5e-6 from 64 bits, not 4.3e-6.
     if (is_kq(fmt) && tmax > 64 && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA")) {
         if (!xplanes)
             if (int e = noalloc_room(name, rows16, K, tmax, tmax >= 256 || fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K ? 256 : 128))

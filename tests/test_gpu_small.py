@@ -142,6 +142,12 @@ def test_many_tokens(quipu, dev, oracle, fmt, T, N, K):
     assert np.all(np.abs(got - want) <= split_bound(W, x) + (0 if y0 is None else 2.0 ** -23 * np.abs(y0)))
 
 
+@pytest.mark.parametrize("T,N,K", [(513, 1000, 10240), (640, 2000, 8192), (1100, 2000, 8192), (130, 8200, 8192)])
+def test_k_splits_on_their_xcds(quipu, dev, oracle, T, N, K):
+    """Q6_K tiles of long rows in 8, 4, 2 and 2 K splits, each on its share of the XCDs, tiles that do not divide by it."""
+    test_many_tokens(quipu, dev, oracle, capi.Q6_K, T, N, K)
+
+
 @pytest.mark.parametrize("fmt", KQ)
 @pytest.mark.parametrize("T,N,K", [(256, 64, 256), (300, 97, 768), (390, 200, 512)])
 def test_many_tokens_swiglu(quipu, dev, oracle, fmt, T, N, K):

@@ -1772,7 +1772,9 @@ KERNEL __launch_bounds__(256) void qp_gemm_mt(QpGemmArgs a) {
 
 // ====================================================================================== prefill GEMM on MFMA
 // Y[t][n] (+)= sum_k X[t][k] * W[n][k] for T >= 64 tokens (the reference's tiled matmul_<fmt>_t and
-// matmul_<fmt>_4, kquants.js:309-386 and gpu.js:203-266, when a prefill chunk is large enough for matrix cores).
+// matmul_<fmt>_4, kquants.js:309-386 and gpu.js:203-266, when a prefill chunk is large enough for matrix cores): Q8_0 and
+// IQ4_NL, and for all formats what a capture records and the grouped expert matmuls without a workspace (the others:
+// qp_small.hip, qp_tile.hip).
 //
 // A workgroup computes a 128-token x 128-row tile with v_mfma_f32_32x32x16_bf16: 4 wavefronts in 2 x 2, each
 // 64 x 64 (2 x 2 MFMA blocks).  Per K step of 64 every thread dequantizes 32 weights of one row with the
@@ -2241,592 +2243,7 @@ KERNEL __launch_bounds__(256) void qp_gemm_reduce(QpReduceArgs a) {
     }
 }
 
-// ---- 256-token tiles (T >= 256, K-quant weights, the input split beforehand): 8 wavefronts in 4 x 2, each 64 x 64,
-// so each dequantized weight tile feeds 256 tokens.  K steps of 32 with two LDS buffers and three register
-// buffers: while the matrix instructions of step s read one LDS buffer, the waves dequantize step s + 1 into the
-// other (the arithmetic overlaps the matrix cores) and the global loads of step s + 2 are in flight; one barrier
-// per step.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// bf16 high/low parts of 8 floats, both rounded to nearest: 3 vector operations per value (the packed conversion
-// of a pair, unpacking the high parts, the exact difference).
-QP_DEV void split_store8_pk(const float (&v)[8], __bf16* hi, __bf16* lo) {
-    u32x4 h, l;
-#pragma unroll
-    for (int p = 0; p < 4; p++) {
-        const uint32_t hb = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){v[2 * p], v[2 * p + 1]}, bf16x2));
-        const float l0 = v[2 * p] - __uint_as_float(hb << 16), l1 = v[2 * p + 1] - __uint_as_float(hb & 0xffff0000u);
-        h[p] = hb;
-        l[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){l0, l1}, bf16x2));
-    }
-    *reinterpret_cast<u32x4*>(hi) = h;
-    *reinterpret_cast<u32x4*>(lo) = l;
-}
-
-// One thread's share of one 32-input K step: 16 inputs of one token row (both bf16 planes) and 8 weights of one
-// output row.
-struct MmW8 {
-    u32x4 x[4];   // bf16 high (x[0..1]) and low (x[2..3]) of the 16 inputs
-    u32x2 q;      // Q4_K: the 8 nibble bytes; Q6_K: the 8 low-bit bytes
-    u32x4 h;      // Q4_K: the super-block header (d, dmin, 12 scale bytes)
-    u32x2 qh;     // Q6_K: the 8 high-bit bytes; Q5_K: the 8 qh bytes
-    uint32_t sc;  // Q6_K: the dword holding this sub-block's scale byte
-    uint32_t d;   // Q6_K: the f16 super-block scale
-};
-
-// Per-thread byte offsets, fixed over the K loop; the step's own offsets are uniform (scalar soffset).  Weights of
-// row r, inputs 8*sub .. 8*sub + 7 of the step at k0.  Q4_K: sub-block j = (k0 % 256) / 32 is the low (j even) or
-// high (j odd) nibble of bytes l = 8*sub .. of the 32 qs bytes 32*(j/2) .., chunk 1 + 2*(j/2) + l/16.  Q6_K:
-// block half h, quarter qd: ql chunk h*4 + (qd%2)*2 + l/16, qh chunk 8 + h*2 + l/16, scale byte h*8 + qd*2 + l/16.
-struct MmOff {
-    uint32_t x, q, h, d;
-};
-
-// quarters q and q + 2 of the step's 32-input chunk (xs_off), high plane then low plane
-QP_DEV void mm8_xload(MmW8& r, const MmOff& o, __amdgpu_buffer_rsrc_t rx, uint32_t xplane, uint32_t xrows,
-                      uint32_t k0) {
-    const uint32_t xk = (k0 >> 5) * 64 * xrows, xq2 = 32 * xrows;
-    r.x[0] = __builtin_amdgcn_raw_buffer_load_b128(rx, o.x, xk, 0);
-    r.x[1] = __builtin_amdgcn_raw_buffer_load_b128(rx, o.x + xq2, xk, 0);
-    r.x[2] = __builtin_amdgcn_raw_buffer_load_b128(rx, o.x, xplane + xk, 0);
-    r.x[3] = __builtin_amdgcn_raw_buffer_load_b128(rx, o.x + xq2, xplane + xk, 0);
-}
-
-template <int FMT>
-QP_DEV void mm8_wload(MmW8& r, const MmOff& o, __amdgpu_buffer_rsrc_t rw, uint32_t nb, uint32_t k0) {
-    const uint32_t b = k0 >> 8, e0 = k0 & 255;
-    if constexpr (FMT == QP_Q4_K) {
-        const uint32_t j = e0 >> 5;
-        r.q = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + (1 + 2 * (j >> 1)) * nb * 16, 0);
-        r.h = __builtin_amdgcn_raw_buffer_load_b128(rw, o.h, b * 16, 0);
-    } else if constexpr (FMT == QP_Q3_K || FMT == QP_Q2_K) {
-        // element 128 n + 32 jj + l: Q3_K qs chunk 2 + 2n + l/16, hmask chunk l/16, scales and d chunk 6; Q2_K qs
-        // chunk 1 + 2n + l/16, the scale byte 8n + 2jj + l/16 in chunk 0, (d, dmin) in the array after the rows
-        const uint32_t n = e0 >> 7;
-        if constexpr (FMT == QP_Q3_K) {
-            r.q = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + (2 + 2 * n) * nb * 16, 0);
-            r.qh = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16, 0);
-            r.h = __builtin_amdgcn_raw_buffer_load_b128(rw, o.h, b * 16 + 6 * nb * 16, 0);
-        } else {
-            r.q = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + (1 + 2 * n) * nb * 16, 0);
-            r.sc = __builtin_amdgcn_raw_buffer_load_b32(rw, o.h, b * 16 + 4 * ((8 * n + 2 * ((e0 & 127) >> 5)) >> 2), 0);
-            r.d = __builtin_amdgcn_raw_buffer_load_b32(rw, o.d, b * 4, 0);
-        }
-    } else if constexpr (FMT == QP_Q5_K) {
-        // qs chunk 3 + 2*(j/2) + l/16, qh chunk 1 + l/16 (the same 8 bytes l of both)
-        const uint32_t j = e0 >> 5;
-        r.q = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + (3 + 2 * (j >> 1)) * nb * 16, 0);
-        r.qh = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + nb * 16, 0);
-        r.h = __builtin_amdgcn_raw_buffer_load_b128(rw, o.h, b * 16, 0);
-    } else {
-        const uint32_t h = e0 >> 7, qd = (e0 & 127) >> 5;
-        r.q = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + (h * 4 + (qd & 1) * 2) * nb * 16, 0);
-        r.qh = __builtin_amdgcn_raw_buffer_load_b64(rw, o.q, b * 16 + (8 + h * 2) * nb * 16, 0);
-        r.sc = __builtin_amdgcn_raw_buffer_load_b32(rw, o.h, b * 16 + 12 * nb * 16 + 4 * (h * 2 + (qd >> 1)), 0);
-        r.d = __builtin_amdgcn_raw_buffer_load_b16(rw, o.d, b * 2, 0);
-    }
-}
-
-template <int FMT>
-QP_DEV void mm8_load(MmW8& r, const MmOff& o, __amdgpu_buffer_rsrc_t rx, __amdgpu_buffer_rsrc_t rw, uint32_t xplane,
-                     uint32_t xrows, uint32_t nb, uint32_t k0) {
-    mm8_xload(r, o, rx, xplane, xrows, k0);
-    mm8_wload<FMT>(r, o, rw, nb, k0);
-}
-
-template <int FMT>
-QP_DEV void mm8_deq(const MmW8& r, uint32_t k0, uint32_t sub, float (&w)[8]) {
-    const uint32_t e0 = k0 & 255;
-    uint32_t v[2];
-    float f, c;
-    if constexpr (FMT == QP_Q3_K) {
-        // fma(fd, q', -4 fd) = fd * (q' - 4) exactly (one rounding of the same value), q' = q2 | hbit << 2
-        const uint32_t n = e0 >> 7, jj = (e0 & 127) >> 5, s = 8 * n + 2 * jj + (sub >> 1);
-        f = h2f(r.h.w & 0xffffu) * ((float)q3k_scale6(r.h.x, r.h.y, r.h.z, s) - 32.0f);
-        c = -4.0f * f;
-        v[0] = ((r.q.x >> (2 * jj)) & 0x03030303u) | (((r.qh.x >> (4 * n + jj)) & 0x01010101u) << 2);
-        v[1] = ((r.q.y >> (2 * jj)) & 0x03030303u) | (((r.qh.y >> (4 * n + jj)) & 0x01010101u) << 2);
-    } else if constexpr (FMT == QP_Q2_K) {
-        const uint32_t n = e0 >> 7, jj = (e0 & 127) >> 5, j = 8 * n + 2 * jj + (sub >> 1);
-        const uint32_t sc = (r.sc >> ((j & 3) * 8)) & 0xffu;
-        f = h2f(r.d & 0xffffu) * (float)(sc & 15u);
-        c = -(h2f(r.d >> 16) * (float)(sc >> 4));
-        v[0] = (r.q.x >> (2 * jj)) & 0x03030303u;
-        v[1] = (r.q.y >> (2 * jj)) & 0x03030303u;
-    } else if constexpr (FMT == QP_Q4_K || FMT == QP_Q5_K) {
-        // fd*q - fm; a Q4_K high nibble is masked in place (16*q) with the scale divided by 16 (exact); Q5_K
-        // shifts the nibble down and adds 16 * bit j of qh
-        const uint32_t j = e0 >> 5, jj = (j & 3) * 8;  // the scale/min unpack of q4k_sm, without a branch
-        const uint32_t sa = (r.h.y >> jj) & 0xffu, sb = (r.h.z >> jj) & 0xffu, s8 = (r.h.w >> jj) & 0xffu;
-        const uint32_t lo4 = 0u - (uint32_t)(j < 4);  // all ones for j < 4: a blend, not a branch
-        const uint32_t sc = ((sa & 63u) & lo4) | (((s8 & 15u) | ((sa >> 6) << 4)) & ~lo4);
-        const uint32_t mn = ((sb & 63u) & lo4) | (((s8 >> 4) | ((sb >> 6) << 4)) & ~lo4);
-        c = -(h2f(r.h.x >> 16) * (float)mn);
-        if constexpr (FMT == QP_Q4_K) {
-            const uint32_t mask = (j & 1) ? 0xf0f0f0f0u : 0x0f0f0f0fu;
-            f = h2f(r.h.x & 0xffffu) * (float)sc * ((j & 1) ? 0.0625f : 1.0f);
-            v[0] = r.q.x & mask;
-            v[1] = r.q.y & mask;
-        } else {
-            const uint32_t ns = (j & 1) * 4;
-            f = h2f(r.h.x & 0xffffu) * (float)sc;
-            v[0] = ((r.q.x >> ns) & 0x0f0f0f0fu) | (((r.qh.x >> j) & 0x01010101u) << 4);
-            v[1] = ((r.q.y >> ns) & 0x0f0f0f0fu) | (((r.qh.y >> j) & 0x01010101u) << 4);
-        }
-    } else {
-        // fd*(q - 32) = fma(fd, q, -32*fd) exactly (both are one rounding of the same product)
-        const uint32_t qd = (e0 & 127) >> 5, sb = ((qd & 1) * 2 + (sub >> 1)) * 8;
-        f = h2f(r.d & 0xffffu) * (float)(int8_t)((r.sc >> sb) & 0xffu);
-        c = -32.0f * f;
-        const uint32_t ls = (qd >> 1) * 4, hs = qd * 2;
-        v[0] = ((r.q.x >> ls) & 0x0f0f0f0fu) | (((r.qh.x >> hs) & 0x03030303u) << 4);
-        v[1] = ((r.q.y >> ls) & 0x0f0f0f0fu) | (((r.qh.y >> hs) & 0x03030303u) << 4);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i++) w[i] = __builtin_fmaf(f, (float)((v[i >> 2] >> (8 * (i & 3))) & 0xffu), c);
-}
-
-template <int FMT>
-QP_DEV void gemm_mfma256_body(const QpGemmArgs& g) {
-    constexpr int TM = 256, TN = 128, TK = 32, LDK = 40, BUF = (TM + TM + TN + TN) * LDK;  // bf16 per buffer
-    extern __shared__ float4 smem4[];
-    __bf16* lds = reinterpret_cast<__bf16*>(smem4);
-    const uint32_t T = g.tfix ? g.tfix : paso_T(g.paso);
-    const uint32_t N = g.n, K = g.k;
-    const uint32_t mt = (uint32_t)gridDim.y, ntl = (uint32_t)gridDim.x, nz = (uint32_t)gridDim.z;
-    const uint32_t total = mt * ntl * nz, id = (blockIdx.z * mt + blockIdx.y) * ntl + blockIdx.x;
-    const uint32_t base = total >> 3, rem = total & 7, xcd = id & 7, j = id >> 3;
-    const uint32_t L = xcd * base + (xcd < rem ? xcd : rem) + j;
-    const uint32_t m_tile = L % mt, rest = L / mt, zs = rest % nz, n_tile = rest / nz;
-    const uint32_t t0 = m_tile * TM, n0 = n_tile * TN;
-    if (t0 >= T) return;
-    const uint32_t kbeg = g.kchunk ? zs * g.kchunk : 0;
-    const uint32_t kend = g.kchunk ? min(K, kbeg + g.kchunk) : K;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t wm = wave >> 1, wn = wave & 1;
-    // loaders, so that each 16-lane phase of an LDS store covers 16 rows: input row lr, quarters xq and xq + 2 of
-    // the step's 32 inputs (a wavefront loads 64 consecutive rows of one quarter: 1 KB contiguous); weight row wq (8
-    // inputs at 8*sub).  Weight rows past N load row 0; input rows past T read rows of the planes that the split
-    // did not write (rows < g.rows, inside the buffer), whose outputs are not stored.
-    const uint32_t lr = tid & 255, xq = tid >> 8, wq = wave * 16 + (lane & 15), sub = lane >> 4;
-    const uint32_t wr = n0 + wq < N ? n0 + wq : 0;
-    const uint32_t nb = K >> 8, xplane = 2 * g.rows * K;
-    const __amdgpu_buffer_rsrc_t rx = kq_rsrc(g.xs, 2ull * xplane);
-    constexpr uint32_t RBW = KQ<FMT>::RB;  // bytes per weight row and 256 inputs (Q6_K: its d array follows)
-    const __amdgpu_buffer_rsrc_t rw = kq_rsrc(g.w, (uint64_t)N * nb * (FMT == QP_Q6_K ? 210 : FMT == QP_Q2_K ? 84 : RBW));
-    MmOff off;
-    off.x = (xq * g.rows + t0 + lr) * 16;
-    off.q = wr * nb * RBW + (sub >> 1) * nb * 16 + (sub & 1) * 8;
-    off.h = wr * nb * RBW;
-    off.d = FMT == QP_Q2_K ? N * nb * 80 + wr * nb * 4 : N * nb * 208 + wr * nb * 2;
-    const uint32_t nsteps = (kend - kbeg + TK - 1) / TK;
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[a][b][v] = 0.0f;
-    MmW8 r0, r1;
-    auto load = [&](MmW8& r, uint32_t st) __attribute__((always_inline)) {
-        // past the last step: reload it (unused)
-        mm8_load<FMT>(r, off, rx, rw, xplane, g.rows, nb, kbeg + min(st, nsteps - 1) * TK);
-    };
-    auto stage = [&](const MmW8& r, uint32_t st, __bf16* buf) __attribute__((always_inline)) {
-        __bf16* xh = buf;
-        __bf16* xl = xh + TM * LDK;
-        __bf16* wh = xl + TM * LDK;
-        __bf16* wl = wh + TN * LDK;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            *reinterpret_cast<u32x4*>(xh + lr * LDK + 8 * (xq + 2 * i)) = r.x[i];
-            *reinterpret_cast<u32x4*>(xl + lr * LDK + 8 * (xq + 2 * i)) = r.x[2 + i];
-        }
-        float w[8];
-        mm8_deq<FMT>(r, kbeg + min(st, nsteps - 1) * TK, sub, w);
-        split_store8_pk(w, wh + wq * LDK + 8 * sub, wl + wq * LDK + 8 * sub);
-    };
-    // step s: the loads of step s + 2 go into the registers step s came in (staged during step s - 1), the
-    // matrix instructions read LDS buffer s % 2, and step s + 1 is dequantized into the other buffer
-    auto step = [&](uint32_t s, MmW8& mine, MmW8& next) __attribute__((always_inline)) {
-        load(mine, s + 2);
-        const __bf16* xh = lds + (s & 1) * BUF;
-        const __bf16* xl = xh + TM * LDK;
-        const __bf16* wh = xl + TM * LDK;
-        const __bf16* wl = wh + TN * LDK;
-#pragma unroll
-        for (int ks = 0; ks < TK / 16; ks++) {
-            const uint32_t kk = ks * 16 + 8 * (lane >> 5);
-            bf16x8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-            for (int a = 0; a < 2; a++) {
-                const uint32_t tr = wm * 64 + a * 32 + (lane & 31);
-                ah[a] = *reinterpret_cast<const bf16x8*>(xh + tr * LDK + kk);
-                al[a] = *reinterpret_cast<const bf16x8*>(xl + tr * LDK + kk);
-                const uint32_t nr = wn * 64 + a * 32 + (lane & 31);
-                bh[a] = *reinterpret_cast<const bf16x8*>(wh + nr * LDK + kk);
-                bl[a] = *reinterpret_cast<const bf16x8*>(wl + nr * LDK + kk);
-            }
-#pragma unroll
-            for (int a = 0; a < 2; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++) {
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[a], bh[b], acc[a][b], 0, 0, 0);
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[a], bl[b], acc[a][b], 0, 0, 0);
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[a], bh[b], acc[a][b], 0, 0, 0);
-                }
-        }
-        stage(next, s + 1, lds + ((s + 1) & 1) * BUF);  // after the last step: a copy of it, never read
-        // issue order: the step's global loads, the first operand reads, then each matrix instruction followed by
-        // two vector operations of the next step's dequantization (so both pipes stay busy), the remaining operand
-        // reads spread between them, the LDS stores last
-        __builtin_amdgcn_sched_group_barrier(0x020, 16, 0);  // VMEM reads
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);   // DS reads (ks 0)
-#pragma unroll
-        for (int i = 0; i < 12; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read (ks 1)
-            __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);  // VALU
-        }
-#pragma unroll
-        for (int i = 0; i < 12; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-        }
-        __builtin_amdgcn_sched_group_barrier(0x200, 16, 0);  // DS writes
-        __syncthreads();
-    };
-    load(r0, 0);
-    load(r1, 1);
-    stage(r0, 0, lds);
-    __syncthreads();
-    for (uint32_t s = 0; s < nsteps; s += 2) {  // nsteps is even: every K range is whole 64-input steps
-        step(s, r0, r1);
-        step(s + 1, r1, r0);
-    }
-    float* Y = g.ws ? mptr<float>(g.ws) + (uint64_t)zs * g.rows * N : mptr<float>(g.y);
-    const bool add = g.acc && !g.ws;
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const uint32_t n = n0 + wn * 64 + b * 32 + (lane & 31);
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const uint32_t t = t0 + wm * 64 + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (t < T && n < N) {
-                    float* o = Y + (uint64_t)t * N + n;
-                    *o = add ? *o + acc[a][b][v] : acc[a][b][v];
-                }
-            }
-        }
-}
-
-// ---- 256-token x 256-row tiles (large K-quant matmuls): 8 wavefronts in 2 x 4, each 128 tokens x 64 rows (4 x 2
-// matrix blocks), so that every operand fragment read from LDS feeds more matrix instructions and each input step
-// loaded feeds twice the rows of the 256 x 128 tile.  Same K steps of 32, two LDS buffers of 80 KB (the whole
-// 160 KB), the loads of step s + 2 in flight during step s, one barrier per step.  Thread tid stages input row
-// tid % 256 (quarters tid / 256 and + 2) and the 8 weights at 8*sub of rows wq and wq + 128.
-// GLU (matmul_<fmt>_t_swiglu): the tile's rows 0..127 are rows n0.. of the gate tensor and rows 128..255 the same
-// rows of the up tensor (w2), so a tile covers 128 outputs; the up wavefronts hand their sums to the gate
-// wavefronts through LDS and y = silu(gate) * up is stored (the swiglu kernel's formula; no K split).
-template <int FMT, bool GLU = false>
-QP_DEV void gemm_mfma256w_body(const QpGemmArgs& g) {
-    constexpr int TM = 256, TN = 256, TK = 32, LDK = 40, BUF = (TM + TM + TN + TN) * LDK;  // bf16 per buffer
-    extern __shared__ float4 smem4[];
-    __bf16* lds = reinterpret_cast<__bf16*>(smem4);
-    const uint32_t T = g.tfix ? g.tfix : paso_T(g.paso);
-    const uint32_t N = g.n, K = g.k;
-    const bool split_tail = GLU && g.tail != 0;
-    const uint32_t mt = split_tail ? g.mtiles : (uint32_t)gridDim.y, ntl = split_tail ? g.ntiles : (uint32_t)gridDim.x;
-    const uint32_t nz = split_tail ? 1u : (uint32_t)gridDim.z;
-    uint32_t L, half = 0, stile = 0;  // stile: the split tile's index among the tail tiles
-    bool split = false;
-    if (split_tail) {
-        // per XCD x (item % 8): whole tiles x * F .. x * F + F - 1, then K halves of tail tiles full + x * H ..
-        const uint32_t full = mt * ntl - g.tail, F = full >> 3, H = g.tail >> 3;
-        const uint32_t xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-        if (j < F) {
-            L = xcd * F + j;
-        } else {
-            const uint32_t jj = j - F;
-            stile = xcd * H + (jj >> 1);
-            L = full + stile;
-            half = jj & 1;
-            split = true;
-        }
-    } else {
-        const uint32_t total = mt * ntl * nz, id = (blockIdx.z * mt + blockIdx.y) * ntl + blockIdx.x;
-        const uint32_t base = total >> 3, rem = total & 7, xcd = id & 7, j = id >> 3;
-        L = xcd * base + (xcd < rem ? xcd : rem) + j;
-    }
-    const uint32_t m_tile = L % mt, rest = L / mt, zs = rest % nz, n_tile = rest / nz;
-    const uint32_t t0 = m_tile * TM, n0 = n_tile * (GLU ? TN / 2 : TN);
-    if (t0 >= T) return;  // (both halves of a split tile: neither counts, nothing is stored)
-    const uint32_t kbeg = split ? half * (K >> 1) : g.kchunk ? zs * g.kchunk : 0;
-    const uint32_t kend = split ? kbeg + (K >> 1) : g.kchunk ? min(K, kbeg + g.kchunk) : K;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t wm = wave >> 2, wn = wave & 3;
-    const uint32_t lr = tid & 255, xq = tid >> 8, wq = wave * 16 + (lane & 15), sub = lane >> 4;
-    // weight rows past N load row 0 (finite values whose outputs are not stored)
-    const uint32_t wr0 = n0 + wq < N ? n0 + wq : 0;
-    const uint32_t wr1 = GLU ? wr0 : n0 + wq + 128 < N ? n0 + wq + 128 : 0;
-    const uint32_t nb = K >> 8, xplane = 2 * g.rows * K;
-    const __amdgpu_buffer_rsrc_t rx = kq_rsrc(g.xs, 2ull * xplane);
-    constexpr uint32_t RBW = KQ<FMT>::RB;
-    const uint64_t wbytes = (uint64_t)N * nb * (FMT == QP_Q6_K ? 210 : FMT == QP_Q2_K ? 84 : RBW);
-    const __amdgpu_buffer_rsrc_t rw = kq_rsrc(g.w, wbytes);
-    const __amdgpu_buffer_rsrc_t rw1 = GLU ? kq_rsrc(g.w2, wbytes) : rw;  // the tensor of row wq + 128
-    MmOff o0;
-    o0.x = (xq * g.rows + t0 + lr) * 16;
-    o0.q = wr0 * nb * RBW + (sub >> 1) * nb * 16 + (sub & 1) * 8;
-    o0.h = wr0 * nb * RBW;
-    o0.d = FMT == QP_Q2_K ? N * nb * 80 + wr0 * nb * 4 : N * nb * 208 + wr0 * nb * 2;
-    MmOff o1 = o0;  // row wq + 128 (GLU: row wq of the up tensor)
-    o1.q = wr1 * nb * RBW + (sub >> 1) * nb * 16 + (sub & 1) * 8;
-    o1.h = wr1 * nb * RBW;
-    o1.d = FMT == QP_Q2_K ? N * nb * 80 + wr1 * nb * 4 : N * nb * 208 + wr1 * nb * 2;
-    const uint32_t nsteps = (kend - kbeg + TK - 1) / TK;
-    f32x16 acc[4][2];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[a][b][v] = 0.0f;
-    struct R2 {
-        MmW8 a, b;  // a: the inputs and the weights of row wq; b: the weights of row wq + 128
-    };
-    R2 r0, r1;
-    auto load = [&](R2& r, uint32_t st) __attribute__((always_inline)) {
-        const uint32_t k0 = kbeg + min(st, nsteps - 1) * TK;  // past the last step: reload it (unused)
-        mm8_xload(r.a, o0, rx, xplane, g.rows, k0);
-        mm8_wload<FMT>(r.a, o0, rw, nb, k0);
-        mm8_wload<FMT>(r.b, o1, rw1, nb, k0);
-    };
-    auto stage = [&](const R2& r, uint32_t st, __bf16* buf) __attribute__((always_inline)) {
-        __bf16* xh = buf;
-        __bf16* xl = xh + TM * LDK;
-        __bf16* wh = xl + TM * LDK;
-        __bf16* wl = wh + TN * LDK;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            *reinterpret_cast<u32x4*>(xh + lr * LDK + 8 * (xq + 2 * i)) = r.a.x[i];
-            *reinterpret_cast<u32x4*>(xl + lr * LDK + 8 * (xq + 2 * i)) = r.a.x[2 + i];
-        }
-        const uint32_t k0 = kbeg + min(st, nsteps - 1) * TK;
-        float w[8];
-        mm8_deq<FMT>(r.a, k0, sub, w);
-        split_store8_pk(w, wh + wq * LDK + 8 * sub, wl + wq * LDK + 8 * sub);
-        mm8_deq<FMT>(r.b, k0, sub, w);
-        split_store8_pk(w, wh + (wq + 128) * LDK + 8 * sub, wl + (wq + 128) * LDK + 8 * sub);
-    };
-    auto step = [&](uint32_t s, R2& mine, R2& next) __attribute__((always_inline)) {
-        load(mine, s + 2);
-        const __bf16* xh = lds + (s & 1) * BUF;
-        const __bf16* xl = xh + TM * LDK;
-        const __bf16* wh = xl + TM * LDK;
-        const __bf16* wl = wh + TN * LDK;
-#pragma unroll
-        for (int ks = 0; ks < TK / 16; ks++) {
-            const uint32_t kk = ks * 16 + 8 * (lane >> 5);
-            // the weight fragments for all four token blocks; the token fragments one block at a time (registers)
-            bf16x8 bh[2], bl[2];
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const uint32_t nr = wn * 64 + b * 32 + (lane & 31);
-                bh[b] = *reinterpret_cast<const bf16x8*>(wh + nr * LDK + kk);
-                bl[b] = *reinterpret_cast<const bf16x8*>(wl + nr * LDK + kk);
-            }
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const uint32_t tr = wm * 128 + a * 32 + (lane & 31);
-                const bf16x8 ah = *reinterpret_cast<const bf16x8*>(xh + tr * LDK + kk);
-                const bf16x8 al = *reinterpret_cast<const bf16x8*>(xl + tr * LDK + kk);
-#pragma unroll
-                for (int b = 0; b < 2; b++) {
-                    f32x16& c = acc[a][b];
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[b], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[b], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[b], c, 0, 0, 0);
-                }
-            }
-        }
-        stage(next, s + 1, lds + ((s + 1) & 1) * BUF);  // after the last step: a copy of it, never read
-        __builtin_amdgcn_sched_group_barrier(0x020, 24, 0);  // VMEM reads
-        __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);  // DS reads (ks 0)
-#pragma unroll
-        for (int i = 0; i < 24; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-        }
-#pragma unroll
-        for (int i = 0; i < 12; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read (ks 1)
-            __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);  // VALU
-        }
-#pragma unroll
-        for (int i = 0; i < 24; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-        }
-        __builtin_amdgcn_sched_group_barrier(0x200, 16, 0);  // DS writes
-        __syncthreads();
-    };
-    load(r0, 0);
-    load(r1, 1);
-    stage(r0, 0, lds);
-    __syncthreads();
-    for (uint32_t s = 0; s < nsteps; s += 2) {  // nsteps is even: every K range is whole 64-input steps
-        step(s, r0, r1);
-        step(s + 1, r1, r0);
-    }
-    if constexpr (GLU) {
-        if (split) {
-            // this half's sums to its slot, [wave][a][b][v][lane]; drained, then one agent-scope arrival (its
-            // release writes the L2 back); the second arrival adds the other slot (the sum of the two halves does
-            // not depend on which arrives last) and goes on with the whole tile
-            float* mine = mptr<float>(g.part) + ((uint64_t)stile * 2 + half) * (512u * 128u);
-            const float* other = cptr<float>(g.part) + ((uint64_t)stile * 2 + (half ^ 1u)) * (512u * 128u);
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) mine[(((wave * 4 + a) * 2 + b) * 16 + v) * 64 + lane] = acc[a][b][v];
-            vm_drain();
-            uint32_t* second = reinterpret_cast<uint32_t*>(smem4);  // the K loop's LDS is free after this barrier
-            __syncthreads();
-            if (tid == 0) {
-                QP_GLOBAL uint32_t* c = reinterpret_cast<QP_GLOBAL uint32_t*>(g.cnt) + stile;
-                const uint32_t old = __hip_atomic_fetch_add(c, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-                *second = old == 1u;
-                if (old == 1u) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();
-            if (!*second) return;
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++)
-                        acc[a][b][v] = acc[a][b][v] + other[(((wave * 4 + a) * 2 + b) * 16 + v) * 64 + lane];
-        }
-        // the up sums (wavefronts wn = 2, 3) to LDS, read by the gate wavefronts wn - 2 at the same index
-        __syncthreads();  // every wavefront has read the last step's LDS buffer
-        float* ex = reinterpret_cast<float*>(smem4);  // [wm][2][4][2][16][64] floats: 128 KB
-        if (wn >= 2) {
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++)
-                        ex[((((wm * 2 + (wn - 2)) * 4 + a) * 2 + b) * 16 + v) * 64 + lane] = acc[a][b][v];
-        }
-        __syncthreads();
-        if (g.yplanes) {
-            // y as the next matmul's input planes (xs_off's layout, g.rows token rows, K = N): the gate wavefronts'
-            // outputs go to an LDS tile [256 tokens][128 outputs] (rows padded to 132 floats) once the up sums are
-            // read, then every thread splits eight consecutive outputs of one token with qp_split_bf16's formula
-            // (the same planes that kernel makes of the f32 outputs) and stores their 16-byte high and low parts;
-            // token rows past T are not written
-            if (wn < 2) {
-#pragma unroll
-                for (int a = 0; a < 4; a++)
-#pragma unroll
-                    for (int b = 0; b < 2; b++)
-#pragma unroll
-                        for (int v = 0; v < 16; v++) {
-                            const float gv = acc[a][b][v];
-                            const float uv = ex[((((wm * 2 + wn) * 4 + a) * 2 + b) * 16 + v) * 64 + lane];
-                            acc[a][b][v] = (gv / (1.0f + expf(-gv))) * uv;
-                        }
-            }
-            __syncthreads();
-            float* tile = reinterpret_cast<float*>(smem4);
-            if (wn < 2) {
-#pragma unroll
-                for (int a = 0; a < 4; a++)
-#pragma unroll
-                    for (int b = 0; b < 2; b++)
-#pragma unroll
-                        for (int v = 0; v < 16; v++) {
-                            const uint32_t t = wm * 128 + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                            tile[t * 132 + wn * 64 + b * 32 + (lane & 31)] = acc[a][b][v];
-                        }
-            }
-            __syncthreads();
-            const uint64_t plane = 2ull * g.rows * N;  // bytes of the high plane (N % 32 == 0)
-            for (uint32_t i = tid; i < 256 * 16; i += 512) {
-                const uint32_t t = i & 255, c8 = i >> 8, n = n0 + 8 * c8;
-                if (t0 + t >= T || n >= N) continue;
-                const float4 v0 = *reinterpret_cast<const float4*>(tile + t * 132 + 8 * c8);
-                const float4 v1 = *reinterpret_cast<const float4*>(tile + t * 132 + 8 * c8 + 4);
-                const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-                const uint64_t o = xs_off(t0 + t, n, g.rows);
-                split_store8(v, reinterpret_cast<__bf16*>(g.y + o), reinterpret_cast<__bf16*>(g.y + plane + o));
-            }
-            return;
-        }
-        if (wn >= 2) return;
-        float* Y = mptr<float>(g.y);
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const uint32_t n = n0 + wn * 64 + b * 32 + (lane & 31);
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const uint32_t t = t0 + wm * 128 + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                    const float gv = acc[a][b][v];
-                    const float uv = ex[((((wm * 2 + wn) * 4 + a) * 2 + b) * 16 + v) * 64 + lane];
-                    if (t < T && n < N) Y[(uint64_t)t * N + n] = (gv / (1.0f + expf(-gv))) * uv;
-                }
-            }
-        return;
-    }
-    float* Y = g.ws ? mptr<float>(g.ws) + (uint64_t)zs * g.rows * N : mptr<float>(g.y);
-    const bool add = g.acc && !g.ws;
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const uint32_t n = n0 + wn * 64 + b * 32 + (lane & 31);
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const uint32_t t = t0 + wm * 128 + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (t < T && n < N) {
-                    float* o = Y + (uint64_t)t * N + n;
-                    *o = add ? *o + acc[a][b][v] : acc[a][b][v];
-                }
-            }
-        }
-}
-
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256w_q4k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q4_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256w_q5k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q5_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256w_q6k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q6_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256w_q3k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q3_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256w_q2k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q2_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_glu_q4k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q4_K, true>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_glu_q5k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q5_K, true>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_glu_q6k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q6_K, true>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_glu_q3k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q3_K, true>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_glu_q2k(QpGemmArgs a) { gemm_mfma256w_body<QP_Q2_K, true>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256_q4k(QpGemmArgs a) { gemm_mfma256_body<QP_Q4_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256_q5k(QpGemmArgs a) { gemm_mfma256_body<QP_Q5_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256_q3k(QpGemmArgs a) { gemm_mfma256_body<QP_Q3_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256_q2k(QpGemmArgs a) { gemm_mfma256_body<QP_Q2_K>(a); }
-KERNEL __launch_bounds__(512) void qp_gemm_mfma256_q6k(QpGemmArgs a) { gemm_mfma256_body<QP_Q6_K>(a); }
 
 KERNEL __launch_bounds__(256) void qp_gemm_mfma_q4k(QpGemmArgs a) { gemm_mfma_body<QP_Q4_K>(a); }
 KERNEL __launch_bounds__(256) void qp_gemm_mfma_q6k(QpGemmArgs a) { gemm_mfma_body<QP_Q6_K>(a); }

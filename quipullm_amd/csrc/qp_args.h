@@ -120,16 +120,6 @@ typedef struct {
     // rows e * n .. of the stacked tensor.  xrows, yrows, nlst: rows of x, y and entries of lst that exist.
     uint64_t lst, off;
     uint32_t n_exp, tpe, tfijo, xrows, yrows, nlst;
-    uint64_t w2;  // matmul_<fmt>_t_swiglu: the up tensor (w is the gate tensor); y = silu(x w) * (x w2)
-    // matmul_<fmt>_t_swiglu with a split tail (tail != 0): a 1-D grid of items over mtiles x ntiles tiles; per XCD
-    // (item % 8), whole tiles first, then its share of the last `tail` tiles as K halves.  Each half stores its
-    // sums to part (two 256 KB slots per split tile) and counts its arrival in cnt[tile]; the second adds the
-    // other's sums and finishes the tile (and resets the word).
-    uint32_t tail, mtiles, ntiles;
-    // matmul_<fmt>_t_swiglu: 1 = y receives the outputs as the next matmul's input planes (the bf16 high and low
-    // planes of qp_split_bf16's layout for rows token rows and K = n), not as f32 rows
-    uint32_t yplanes;
-    uint64_t part, cnt;
 } QpGemmArgs;
 
 // qp_sk_<fmt>: matmul of few token rows on integer weights (qp_small.hip).  xs: X as operands (qp_split_f16) of `rows`
@@ -166,7 +156,7 @@ typedef struct {
 } QpMoeGroupArgs;
 // x [T][k] -> bf16 high / low planes (hi = bf16(v), lo = bf16(v - hi)) at xs and xs + 2*rows*k.  mul != 0: the
 // first min(T * mul, cap) rows of x instead of T, in row-major planes ([rows][k rounded up to 32]: the grouped
-// expert matmul, whose tiles gather rows), not the chunk-quarter layout of the 256-token tiles.
+// expert matmul, whose tiles gather rows), not the chunk-quarter layout of the dense matmuls.
 // qp_split_f16 (the integer-weight matmuls' operands) takes the same: mul as there; mode 0: X to 22 bits, 1: X as its bf16
 // high + low parts first, 2: x holds those parts (qp_split_bf16's planes of prows token rows).  tbase (mul = 0): the token
 // that x's first row is.

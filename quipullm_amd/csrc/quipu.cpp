@@ -522,7 +522,7 @@ int run_sk(int fmt, QpSkArgs& a, uint32_t nt, uint32_t tpe, uint32_t E, uint32_t
     return launch(sk_kid(fmt, nt, R), gx, tpe * E, 1, 256, lds, a);
 }
 
-// The dense matmuls that take this path (the others: the 128- and 256-token tiles of op_matmul_mt), by the tokens the
+// The dense matmuls that take this path (the others: the 128-token tiles of op_matmul_mt), by the tokens the
 // dispatch covers, measured with weights past the last-level cache, this path against the tiles in us:
 //   K-quants up to 64 tokens, and below 256 where the matrix is small (qp_tile.hip's tiles then run in K splits whose
 //     sums are added after): this path against those tiles at 65 / 128 / 129 / 192 tokens Q4_K 14336 x 4096 72 / 81 /
@@ -594,7 +594,7 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
     a.k = K;
     a.acc = acc;
     const uint32_t tmax = c.gz * tokens_per_z;
-    // P[4] = 2 (x holds input planes) is read by the 256-token tiles only (below: K-quants, 256 tokens or more)
+    // P[4] = 2: x holds input planes (K-quants, 256 tokens or more)
     const bool xplanes = c.U(4) == 2;
     if (xplanes && (!is_kq(fmt) || tmax < 256 || (g_capturing && !g_noalloc) || getenv_flag("QP_NO_MFMA")))
         return fail(QP_E_ARG, "%s: P[4] = 2 (x holds input planes) needs K-quant weights and a chunk of 256 tokens "
@@ -625,11 +625,11 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         return 0;
     }
     // K-quants of more tokens: integer weights in 128 x 128 tiles (qp_tile.hip).  Against the 256-token tiles of bf16 high and
-    // low parts that they replaced, at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 95 / 153 / 290 / 560 against 109
-    // / 186 / 326 / 650, 4096 x 14336 105 / 163 / 296 / 561 against 116 / 206 / 375 / 681; Q6_K 4096 x 14336 130 / 216 / 401 /
-    // 770 against 129 / 228 / 416 / 781, 5120 x 13824 195 / 335 / 636 / 1049 against 185 / 334 / 612 / 1134.  Q6_K, whose weights
-    // take three products here too, gains no time (whole 256s of tokens lose up to 7 %: 4096 x 11008 at 256 112 against 104), but
-    // the sums are 2.5e-6 from 64 bits, not 4.3e-6.
+    // low parts that they replaced, at 256 / 512 / 1024 / 2048 tokens in us: Q4_K 14336 x 4096 95 / 150 / 287 / 519 against 107
+    // / 182 / 320 / 629, 4096 x 14336 105 / 163 / 296 / 561 against 116 / 206 / 375 / 681; Q6_K 4096 x 14336 130 / 216 / 401 /
+    // 770 against 129 / 228 / 416 / 781, 14336 x 4096 134 / 215 / 396 / 734 against 125 / 201 / 373 / 743.  Q6_K, whose weights
+    // take three products here too, gains no time (whole 256s of tokens up to 1024 lose up to 7 %, others gain: 288 tokens 187
+    // against 199), but the sums are 2.5e-6 from 64 bits, not 4.3e-6.
     if (is_kq(fmt) && tmax > 64 && (!g_capturing || g_noalloc) && !getenv_flag("QP_NO_MFMA")) {
         if (!xplanes)
             if (int e = noalloc_room(name, rows16, K, tmax, tmax >= 256 || fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K ? 256 : 128))
@@ -669,39 +669,24 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
         return 0;
     }
     if (tmax >= 64 && !getenv_flag("QP_NO_MFMA")) {
-        // matrix cores: 128 x 128 tiles (the kernel reads T from paso; tiles past it exit)
+        // matrix cores: 128 x 128 tiles of bf16 high and low parts (the kernel reads T from paso; tiles past it exit):
+        // Q8_0 and IQ4_NL, and what a capture records
         const Kid k = fmt == QP_Q4_K ? K_gemm_mfma_q4k : fmt == QP_Q6_K ? K_gemm_mfma_q6k
                     : fmt == QP_Q8_0 ? K_gemm_mfma_q8 : fmt == QP_IQ4_NL ? K_gemm_mfma_iq4nl : K_gemm_mfma_f32;
-        uint32_t mt = cdiv(tmax, 128);
-        uint32_t nt = cdiv(N, 128);
+        const uint32_t mt = cdiv(tmax, 128), nt = cdiv(N, 128);
         if (!g_capturing || g_noalloc) {
             // x split into bf16 planes once (not in every weight tile's workgroup), and the K range split when the
-            // tiles alone cannot occupy the CUs (a 128-row router at 2048 tokens is 16 tiles); partials summed in
-            // order.  K-quants from 256 tokens on: 256-token tiles (one 512-thread workgroup per CU, K steps of 32
-            // double-buffered in LDS) dequantize each weight tile half as often.
-            // Q5_K, Q3_K and Q2_K have only the 256-token tiles
-            const bool big = is_kq(fmt) && (tmax >= 256 || fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K);
-            if (big) mt = cdiv(tmax, 256);
-            // 256 x 256 tiles when they alone occupy three quarters of the CUs, or half of them at K >= 8192 (where
-            // splitting K in two costs little); measured at 2048 tokens: 14336 x 4096 789 vs 886 us, 6144 x 4096 375
-            // vs 439, 4096 x 14336 917 vs 941, and 4096 x 2048 130 vs 121 against the 256 x 128 tiles.
-            // QP_GEMM_TILES=wide / narrow forces one kind, for tests and comparisons.
-            const char* tiles = getenv("QP_GEMM_TILES");
-            const uint32_t wt = mt * cdiv(N, 256);
-            const bool wide = big && (tiles && !strcmp(tiles, "wide") ? true
-                                      : tiles && !strcmp(tiles, "narrow") ? false
-                                      : 4 * wt >= 3 * (uint32_t)g_cus || (2 * wt >= (uint32_t)g_cus && K >= 8192));
-            if (wide) nt = cdiv(N, 256);
-            const uint32_t steps = K / 64, slots = (big ? 1 : 2) * (uint32_t)g_cus;
+            // tiles alone cannot occupy the CUs; partials summed in order.
+            const uint32_t steps = K / 64, slots = 2 * (uint32_t)g_cus;
             uint32_t ns2 = 1;  // K splits, a power of two
             while (mt * nt * ns2 * 2 <= slots && steps / (ns2 * 2) >= 4) ns2 *= 2;
-            a.rows = mt * (big ? 256 : 128);
+            a.rows = mt * 128;
             // the bf16 planes: 2 x 2 bytes per token row and input, K rounded up to whole 32-input chunks
             const uint64_t xs_bytes = 4ull * a.rows * ((K + 31) / 32 * 32);
             uint32_t ns;
             uint64_t ws_bytes;
             for (;;) {
-                a.kchunk = ns2 > 1 ? cdiv(steps, ns2) * 64 : 0;  // whole 64-input steps (the 256-token tiles take 32)
+                a.kchunk = ns2 > 1 ? cdiv(steps, ns2) * 64 : 0;  // whole 64-input steps
                 ns = ns2 > 1 ? cdiv(K, a.kchunk) : 1;
                 ws_bytes = ns > 1 ? 4ull * ns * a.rows * N : 0;
                 // the fixed scratch of qp_dispatch_noalloc: fewer K splits (down to none) until the partials fit
@@ -709,42 +694,18 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
                 ns2 /= 2;
             }
             uint64_t ws = 0;
-            const uint32_t xmode = c.U(4);
-            if (xmode == 2) {
-                // P[4] = 2: x holds the input planes already (matmul_<fmt>_t_swiglu with planes = 1 wrote them for
-                // the same T), sized for 256-token tiles (big holds: checked above)
-                if (K % 32) return fail(QP_E_ARG, "%s: input planes need K %% 32 == 0", name);
-                if (int e = need_room(a.x, xs_bytes, name, "the input planes' buffer")) return e;
-                if (ws_bytes)
-                    if (int e = workspace(ws_bytes, &ws)) return e;
-                a.xs = a.x;
-                a.ws = ns > 1 ? ws : 0;
-            } else {
-                if (int e = workspace(xs_bytes + ws_bytes, &ws)) return e;
-                a.xs = ws;
-                a.ws = ns > 1 ? ws + xs_bytes : 0;
-                // P[4] = 1: reuse the previous matmul's input planes (see split_input)
-                if (int e = split_input(a.x, a.xs, a.paso, K, a.rows, tmax, xmode == 1)) return e;
-            }
-            if (wide) {
-                static const Kid kw_of[5] = {K_gemm_mfma256w_q4k, K_gemm_mfma256w_q5k, K_gemm_mfma256w_q6k,
-                                             K_gemm_mfma256w_q3k, K_gemm_mfma256w_q2k};
-                if (int e = launch(kw_of[kq_index(fmt)], nt, mt, ns, 512, 2 * (256 + 256 + 256 + 256) * 40 * 2, a))
-                    return e;
-            } else if (big) {
-                static const Kid kb_of[5] = {K_gemm_mfma256_q4k, K_gemm_mfma256_q5k, K_gemm_mfma256_q6k,
-                                             K_gemm_mfma256_q3k, K_gemm_mfma256_q2k};
-                const Kid kb = kb_of[kq_index(fmt)];
-                if (int e = launch(kb, nt, mt, ns, 512, 2 * (256 + 256 + 128 + 128) * 40 * 2, a)) return e;
-            } else if (int e = launch(k, nt, mt, ns, 256, 0, a)) {
-                return e;
-            }
+            if (int e = workspace(xs_bytes + ws_bytes, &ws)) return e;
+            a.xs = ws;
+            a.ws = ns > 1 ? ws + xs_bytes : 0;
+            // P[4] = 1: reuse the previous matmul's input planes (see split_input)
+            if (int e = split_input(a.x, a.xs, a.paso, K, a.rows, tmax, c.U(4) == 1)) return e;
+            if (int e = launch(k, nt, mt, ns, 256, 0, a)) return e;
             if (ns == 1) return 0;
             QpReduceArgs ra = {a.ws, a.y, a.paso, N, a.rows, ns, acc, 0, 0};
             return launch(K_gemm_reduce, grid_cap((uint64_t)tmax * N), 1, 1, 256, 0, ra);
         }
         if (fmt == QP_Q5_K || fmt == QP_Q3_K || fmt == QP_Q2_K)
-            return launch(K_gemm_mt, cdiv(N, 64), cdiv(tmax, 64), 1, 256, 0, a);  // under capture
+            return launch(K_gemm_mt, cdiv(N, 64), cdiv(tmax, 64), 1, 256, 0, a);
         return launch(k, nt, mt, 1, 256, 0, a);
     }
     return launch(K_gemm_mt, cdiv(N, 64), cdiv(tmax ? tmax : 1, 64), 1, 256, 0, a);
@@ -753,16 +714,14 @@ int op_matmul_mt(const Ctx& c, int fmt, const char* name, uint32_t tokens_per_z)
 // matmul_<fmt>_t_swiglu: P{N, K, planes, xplanes}; [paso, w_gate, w_up, x, y]; y[t][n] = silu(x[t] . gate[n]) *
 // (x[t] . up[n]) for the T tokens of paso (K-quants).  No counterpart in the reference, whose prompt pass runs
 // matmul_<fmt>_t on the gate and up tensors and then swiglu (transformer.js:311-313): the same three results in one
-// matrix-core launch (256-token tiles of 128 gate and 128 up rows), for prompt chunks of at least 256 tokens.  Same
-// accumulation as matmul_<fmt>_t with 256 x 256 tiles.  Not while capturing a graph (the input planes may need a
-// larger workspace).  planes = 1 (the third word; absent: 0): y receives the outputs as the input planes of the
+// matrix-core launch (tiles of 128 tokens x 64 gate and 64 up rows, the sums of matmul_<fmt>_t's tiles without K splits),
+// for prompt chunks of at least 256 tokens.  Not while capturing a graph (the operands may need a larger workspace).
+// planes = 1 (the third word; absent: 0): y receives the outputs as the input planes of the
 // matmul that reads them next (matmul_<fmt>_t with P[4] = 2), the values qp_split_bf16 would make of the f32 rows,
 // for R = 256 * ceil(T / 256) token rows and K = N: 4 R N bytes.  P[3] = 1: x holds its input as such planes
 // (rmsnorm_planes), 4 R K bytes.
 uint64_t tensor_bytes(int fmt, uint64_t rows, uint32_t K);
 int need_room(uint64_t p, uint64_t bytes, const char* op, const char* what);
-constexpr uint32_t kGluCntWords = 1024;  // split tiles of one launch at most (one arrival word each)
-uint64_t g_glu_cnt = 0;                  // the arrival words, allocated on first use, kept until the process ends
 int op_matmul_glu(const Ctx& c, int fmt, const char* name) {
     if (int e = need_bufs(c, 5, name)) return e;
     const uint32_t N = c.U(0), K = c.U(1);
@@ -775,88 +734,40 @@ int op_matmul_glu(const Ctx& c, int fmt, const char* name) {
     const uint64_t tb = tensor_bytes(fmt, N, K);
     if (int e = need_room(c.B(1), tb, name, "the gate tensor's buffer")) return e;
     if (int e = need_room(c.B(2), tb, name, "the up tensor's buffer")) return e;
-    QpGemmArgs a = {};
-    a.w = c.B(1);
-    a.w2 = c.B(2);
-    a.x = c.B(3);
-    a.y = c.B(4);
-    a.paso = c.B(0);
-    a.fmt = fmt;
-    a.n = N;
-    a.k = K;
-    const uint32_t mt = cdiv(tmax, 256), nt = cdiv(N, 128);
-    a.rows = mt * 256;
-    a.yplanes = c.U(2);
-    if (a.yplanes > 1) return fail(QP_E_ARG, "%s: P[2] = %u (0: f32 rows, 1: input planes)", name, a.yplanes);
-    if (a.yplanes) {
+    QpTileArgs s = {};
+    s.w = c.B(1);
+    s.w2 = c.B(2);
+    s.y = c.B(4);
+    s.paso = c.B(0);
+    s.n = N;
+    s.k = K;
+    s.wrows = N;
+    s.kb = K / 256;
+    const uint64_t x = c.B(3);
+    const uint32_t rows16 = cdiv(tmax, 16) * 16, prows = cdiv(tmax, 256) * 256, planes = c.U(2);
+    if (planes > 1) return fail(QP_E_ARG, "%s: P[2] = %u (0: f32 rows, 1: input planes)", name, planes);
+    if (planes) {
         if (N % 32) return fail(QP_E_ARG, "%s: the input planes need N %% 32 == 0 (N = %u)", name, N);
-        if (int e = need_room(a.y, 4ull * a.rows * N, name, "the output planes' buffer")) return e;
+        if (int e = need_room(s.y, 4ull * prows * N, name, "the output planes' buffer")) return e;
+        s.yplanes = prows;
     }
-    const uint32_t rows16 = cdiv(tmax, 16) * 16;
-    // Integer weights in tiles of 128 tokens x (64 gate + 64 up) rows (qp_tile.hip): 14336 x 4096 of Q4_K at 2048 tokens 1208 us against 1320, of Q5_K at 333 334 against 357.
-    {
-        const bool xp = c.U(3) == 1;
-        if (xp) {
-            if (int e = need_room(a.x, 4ull * a.rows * K, name, "the input planes' buffer")) return e;
-        } else if (int e = noalloc_room(name, rows16, K, tmax, 256)) {
-            return e;
-        }
-        QpTileArgs s = {};
-        s.w = a.w;
-        s.w2 = a.w2;
-        s.y = a.y;
-        s.paso = a.paso;
-        s.n = N;
-        s.k = K;
-        s.wrows = N;
-        s.kb = K / 256;
-        s.yplanes = a.yplanes ? a.rows : 0;
-        const uint32_t step = pass_rows(rows16, K);
-        if (int e = workspace(sk_bytes(step, K), &s.xs)) return e;
-        for (s.tbase = 0; s.tbase < rows16; s.tbase += step, s.y += (s.yplanes ? 16ull : 4ull * N) * step) {
-            s.rows = rows16 - s.tbase < step ? rows16 - s.tbase : step;
-            s.mt = cdiv(s.rows, 128);
-            if (int e = tile_input(a.x, s.xs, a.paso, K, s.rows, tmax, false, xp, s.tbase)) return e;
-            if (int e = run_tile(fmt, s, true, 1)) return e;
-        }
-        return 0;
+    const bool xp = c.U(3) == 1;
+    if (xp) {
+        if (int e = need_room(x, 4ull * prows * K, name, "the input planes' buffer")) return e;
+    } else if (int e = noalloc_room(name, rows16, K, tmax, 256)) {
+        return e;
     }
-    // One workgroup per CU (the kernel takes the whole LDS), so the tiles run in rounds of g_cus.  When the last
-    // round would leave at least half the CUs idle, its tiles run as K halves instead (two items each, the second to
-    // finish adds the other's sums): 896 tiles of the 8B gate/up at 2048 tokens take 3.5 rounds' time, not 4.
-    // Needs every XCD to get the same numbers of whole and split tiles and K halves of whole 64-input steps; not
-    // under qp_dispatch_noalloc (the partials need workspace); QP_GLU_SPLIT=0 turns it off.
-    const uint32_t tiles = mt * nt, C = g_cus > 0 ? (uint32_t)g_cus : 1u, rem = tiles % C;
-    const char* sp = getenv("QP_GLU_SPLIT");
-    const bool split = !g_noalloc && !(sp && !strcmp(sp, "0")) && tiles > C && rem > 0 && 2 * rem <= C &&
-                       rem % 8 == 0 && (tiles - rem) % 8 == 0 && K % 128 == 0 && rem <= kGluCntWords;
-    // P[3] = 1: x holds the input planes already (rmsnorm_planes wrote them for the same T)
-    const bool xpl = c.U(3) == 1;
-    const uint64_t planes = xpl ? 0 : 4ull * a.rows * K, part = split ? (uint64_t)rem * 2 * 512 * 128 * 4 : 0;
-    if (xpl)
-        if (int e = need_room(a.x, 4ull * a.rows * K, name, "the input planes' buffer")) return e;
-    uint64_t ws = 0;
-    if (planes + part)
-        if (int e = workspace(planes + part, &ws)) return e;
-    a.xs = xpl ? a.x : ws;
-    if (!xpl)
-        if (int e = split_input(a.x, a.xs, a.paso, K, a.rows, tmax, false)) return e;
-    static const Kid kg_of[5] = {K_gemm_glu_q4k, K_gemm_glu_q5k, K_gemm_glu_q6k, K_gemm_glu_q3k, K_gemm_glu_q2k};
-    const uint32_t lds = 2 * (256 + 256 + 256 + 256) * 40 * 2;
-    if (!split) return launch(kg_of[kq_index(fmt)], nt, mt, 1, 512, lds, a);
-    if (!g_glu_cnt) {
-        // the arrival words: zero once, and every split tile's second arrival sets its word back to zero
-        void* p = nullptr;
-        HIPCHK(hipMalloc(&p, 4ull * kGluCntWords), "hipMalloc (split-tile counters)");
-        HIPCHK(hipMemsetAsync(p, 0, 4ull * kGluCntWords, g_stream), "hipMemsetAsync");
-        g_glu_cnt = (uint64_t)p;
+    // (against 256-token tiles of bf16 parts: 14336 x 4096 of Q4_K at 256 / 2048 tokens 176 / 1053 us against 283 / 1340, of
+    // Q6_K 239 / 1497 against 376 / 1525, at 512, the one of these sizes that lost, 418 against 402)
+    const uint32_t step = pass_rows(rows16, K);
+    if (int e = workspace(sk_bytes(step, K), &s.xs)) return e;
+    for (s.tbase = 0; s.tbase < rows16; s.tbase += step, s.y += (planes ? 16ull : 4ull * N) * step) {
+        s.rows = rows16 - s.tbase < step ? rows16 - s.tbase : step;
+        s.mt = cdiv(s.rows, 128);
+        if (int e = tile_input(x, s.xs, s.paso, K, s.rows, tmax, false, xp, s.tbase)) return e;
+        if (int e = run_tile(fmt, s, true, 1)) return e;
     }
-    a.tail = rem;
-    a.mtiles = mt;
-    a.ntiles = nt;
-    a.part = ws + planes;
-    a.cnt = g_glu_cnt;
-    return launch(kg_of[kq_index(fmt)], tiles + rem, 1, 1, 512, lds, a);
+    return 0;
 }
 
 // matmul_<fmt>_e (kquants.js:256-304, kds.js:110-186): P{N,K,acc,tfijo,E}; [paso, w, x, y, sel]

@@ -4,8 +4,8 @@ matrix-core kernel for T >= 64), with random packed weights and X ~ N(0, 1).
     python -m quipullm_amd.gemm_bench [--shape q4k:14336x4096] [--tokens 512] [--iters 20]
 
 Launches rotate through enough weight copies (>= --rotate-mb) that the last-level cache cannot hold them; HIP
-events on the backend's stream time the loop.  Algorithmic FLOPs are 2*T*N*K per launch (the kernel issues 3x as
-many matrix-core operations: the bf16 high/low products).  One JSON line per shape on stdout.
+events on the backend's stream time the loop.  Algorithmic FLOPs are 2*T*N*K per launch (the kernels issue 2x as many
+matrix-core operations for the high and low products, 3x for Q6_K and f32).  One JSON line per shape on stdout.
 """
 from __future__ import annotations
 

@@ -76,8 +76,8 @@ read_kv_f16 = refs.read_kv_f16
                                   "mini_qwen3moe_iq4nl_c", "mini_gemma3_q4km_c", "mini_llama_f16_c"])
 @pytest.mark.parametrize("plen", [150, 300])
 def test_long_prefill_on_matrix_cores_matches_oracle(oracle, models_dir, tmp_path, name, plen):
-    """A 150- or 300-token prompt in one chunk runs the prefill matmuls on MFMA (bf16 hi/lo products; from 256
-    tokens on the 256-token tiles and, for the dense K-quant models, gate, up and SwiGLU fused into one launch);
+    """A 150- or 300-token prompt in one chunk runs the prefill matmuls on MFMA (split products; from 256
+    tokens on, for the dense K-quant models, gate, up and SwiGLU fused into one launch);
     the logits of the prompt's last token and the greedy continuation must still match the oracle."""
     path = synth.ensure_model(name, models_dir)
     vocab = oracle.GGUF(path).tensors["token_embd.weight"]["dims"][1]

@@ -279,10 +279,10 @@ def test_matmul_multi_token(quipu, dev, oracle, fmt, T, op):
                                         (300, 500, 256, 1), (128, 1024, 5632, 1), (512, 4096, 1024, 0),
                                         (1000, 700, 4864, 1), (256, 130, 2048, 0)])
 def test_matmul_prefill_mfma(quipu, dev, oracle, fmt, T, N, K, acc):
-    """The matrix-core prefill path (T >= 64): bf16 hi/lo products stay within the float32 dot bound, with
-    partial token and row tiles, and tile counts that are not a multiple of the 8 XCDs (3 x 4 = 12 tiles).  For
-    K-quants the input is split into bf16 planes once and small tile grids split K (K = 5632: 15 splits, the last
-    one partial), partials summed in order; from T = 256 on they take the 256-token tiles."""
+    """The matrix-core prefill path (T >= 64): split products stay within the float32 dot bound, with partial token and
+    row tiles, and tile counts that are not a multiple of the 8 XCDs.  The input is split once, small tile grids split K
+    (K = 5632, 4864), partials summed in order; Q8_0 and IQ4_NL take 128 x 128 tiles of bf16 parts, f32 and the K-quants of
+    small matrices the wavefronts' own weights, the others 128 x 128 tiles of integer weights."""
     if fmt in PLANAR and K % 64:
         K += 32
     raw = raw_matrix(fmt, N, K, 61)
@@ -299,6 +299,37 @@ def test_matmul_prefill_mfma(quipu, dev, oracle, fmt, T, N, K, acc):
     want = (W.astype(np.float64) @ x.astype(np.float64).T).T + (y0 if acc else 0)
     bound = (np.abs(W.astype(np.float64)) @ np.abs(x.astype(np.float64)).T).T * 2e-5 + 2e-7 * np.abs(y0) + 1e-30
     assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("T,N,K", [(130, 200, 1024), (40, 70, 768)])
+def test_matmul_in_a_captured_graph(quipu, dev, oracle, fmt, T, N, K):
+    """matmul_<fmt>_t recorded by qp_dispatch during a capture, which has no workspace: the tiles that split their rows
+    themselves (64 tokens or more) and the vector-unit kernel.  Replayed with fresh inputs, eager calls between."""
+    raw = raw_matrix(fmt, N, K, 68)
+    W = (oracle.dequant(fmt, raw, N * K) if fmt != capi.F32 else raw.view(np.float32)).reshape(N, K)
+    w = dev.matrix(fmt, raw, N, K)
+    wb = [w, capi.scale_plane(fmt, w, N, K)] if fmt in PLANAR else [w]
+    xb, y, y2, p = dev.zeros(4 * T * K), dev.zeros(4 * T * N), dev.zeros(4 * T * N), dev.paso(T, 0)
+    args = ("matmul_%s_t" % capi.FMT_NAME[fmt], [("u", N), ("u", K), ("u", 0), ("u", 0)])
+    grid = ((N + 63) // 64, 1, (T + 31) // 32)
+    quipu.graph_begin()
+    try:
+        quipu.dispatch(*args, [p] + wb + [xb, y], grid)
+    finally:
+        g = quipu.graph_end()
+    try:
+        for r in range(3):
+            x = (np.random.default_rng(25 + r).standard_normal((T, K)) * 3).astype(np.float32)
+            quipu.upload(xb, x)
+            quipu.graph_launch(g)
+            quipu.dispatch(*args, [p] + wb + [xb, y2], grid)
+            want = x.astype(np.float64) @ W.astype(np.float64).T
+            bound = 2e-5 * (np.abs(x.astype(np.float64)) @ np.abs(W.astype(np.float64)).T) + 1e-30
+            for h in (y, y2):
+                assert np.all(np.abs(dev.get(h, (T, N)) - want) <= bound), r
+    finally:
+        quipu.graph_free(g)
 
 
 KQ_FMTS = [capi.Q2_K, capi.Q3_K, capi.Q4_K, capi.Q5_K, capi.Q6_K]
@@ -343,7 +374,7 @@ def test_matmul_prefill_tile_kinds(quipu, dev, oracle, fmt, x_as, T, N, K, acc):
 @pytest.mark.parametrize("fmt", KQ_FMTS)
 @pytest.mark.parametrize("T,N,K", [(256, 300, 2048), (300, 520, 1024), (513, 130, 4864)])
 def test_matmul_swiglu_fused(quipu, dev, oracle, fmt, T, N, K):
-    """matmul_<fmt>_t_swiglu: silu(x . gate) * (x . up) in one launch (tiles of 128 gate and 128 up rows), against
+    """matmul_<fmt>_t_swiglu: silu(x . gate) * (x . up) in one launch (tiles of 64 gate and 64 up rows), against
     float64: the gate and up sums within the float32 dot bound, propagated through silu and the product."""
     rg, ru = raw_matrix(fmt, N, K, 71), raw_matrix(fmt, N, K, 72)
     Wg = oracle.dequant(fmt, rg, N * K).reshape(N, K).astype(np.float64)
@@ -364,11 +395,9 @@ def test_matmul_swiglu_fused(quipu, dev, oracle, fmt, T, N, K):
 
 
 @pytest.mark.parametrize("fmt", [capi.Q4_K, capi.Q6_K])
-def test_matmul_swiglu_fused_equals_the_three_ops(quipu, dev, monkeypatch, fmt):
-    """At 2048 tokens x 4352 rows (136 tiles of 256 x 256: no K split) the fused op gives exactly what
-    matmul_<fmt>_t on gate and on up followed by swiglu give: the same sums in the same order."""
-    monkeypatch.setenv("QP_GEMM_TILES", "wide")
-    monkeypatch.setenv("QP_GLU_SPLIT", "0")  # 272 tiles: on 256 CUs the last 16 would run as K halves
+def test_matmul_swiglu_fused_equals_the_three_ops(quipu, dev, fmt):
+    """At 2048 tokens x 4352 rows (544 tiles of 128 x 128, more than half the places for them: no K split) the fused op gives
+    exactly what matmul_<fmt>_t on gate and on up followed by swiglu give: the same sums in the same order."""
     T, N, K = 2048, 4352, 1024
     rg, ru = raw_matrix(fmt, N, K, 73), raw_matrix(fmt, N, K, 74)
     wg, wu = dev.matrix(fmt, rg, N, K), dev.matrix(fmt, ru, N, K)
@@ -385,12 +414,10 @@ def test_matmul_swiglu_fused_equals_the_three_ops(quipu, dev, monkeypatch, fmt):
     assert np.array_equal(dev.get(y, (T, N)), dev.get(g, (T, N)))
 
 
-def test_matmul_swiglu_split_tail(quipu, dev, oracle, monkeypatch):
-    """matmul_q4k_t_swiglu at 256 tokens x 33792 rows (264 tiles): on 256 CUs the last 8 tiles run as K halves,
-    the second half to finish adding the first's sums.  Within the float64 bound; the same bits on a second call
-    (the arrival words are back at zero, and the sum of the two halves does not depend on their order); close to
-    the unsplit launch (QP_GLU_SPLIT=0), whose sums are accumulated in another order."""
-    fmt, T, N, K = capi.Q4_K, 256, 33792, 256
+def test_matmul_swiglu_many_row_tiles(quipu, dev, oracle):
+    """matmul_q4k_t_swiglu at 256 tokens x 33800 rows (2 x 529 tiles, which the 8 XCDs do not divide), one block of 256
+    inputs: within the float64 bound, and the same bits on a second call."""
+    fmt, T, N, K = capi.Q4_K, 256, 33800, 256
     rg, ru = raw_matrix(fmt, N, K, 75), raw_matrix(fmt, N, K, 76)
     Wg = oracle.dequant(fmt, rg, N * K).reshape(N, K).astype(np.float64)
     Wu = oracle.dequant(fmt, ru, N * K).reshape(N, K).astype(np.float64)
@@ -403,19 +430,16 @@ def test_matmul_swiglu_split_tail(quipu, dev, oracle, monkeypatch):
                        ((N + 63) // 64, 1, (T + 31) // 32))
         return dev.get(y, (T, N))
 
-    a, b = run(), run()
-    assert np.array_equal(a, b)
-    monkeypatch.setenv("QP_GLU_SPLIT", "0")
-    c = run()
+    got = run()
+    assert np.array_equal(got, run())
     x64 = x.astype(np.float64)
     g, u = x64 @ Wg.T, x64 @ Wu.T
     dg, du = 2e-5 * (np.abs(x64) @ np.abs(Wg).T), 2e-5 * (np.abs(x64) @ np.abs(Wu).T)
     sg = g / (1.0 + np.exp(np.minimum(-g, 700.0)))
     want = sg * u
     bound = 1.1 * dg * (np.abs(u) + du) + np.abs(sg) * du + 1e-6 * np.abs(want) + 1e-30
-    for got in (a, c):
-        got = got.astype(np.float64)
-        assert np.all(np.isfinite(got)) and np.all(np.abs(got - want) <= bound)
+    got = got.astype(np.float64)
+    assert np.all(np.isfinite(got)) and np.all(np.abs(got - want) <= bound)
 
 
 @pytest.mark.parametrize("fg,fd,T,F,D", [(capi.Q4_K, capi.Q6_K, 300, 512, 256), (capi.Q5_K, capi.Q4_K, 2048, 1536, 512),
@@ -425,7 +449,7 @@ def test_matmul_swiglu_planes_feed_down(quipu, dev, fg, fd, T, F, D, acc):
     """matmul_<fmt>_t_swiglu with P[2] = 1 writes the down matmul's input planes itself, and matmul_<fmt>_t with
     P[4] = 2 reads them: the down matmul's output equals, bit for bit, the f32 path (the fused op's f32 outputs
     split by the down matmul).  T = 300: token rows 300 .. 511 of the planes are not written; 2304 tokens x 15360
-    rows (1080 tiles): on 256 CUs the fused op's last 56 tiles run as K halves."""
+    rows: the largest K, four tile columns of the down matmul split along it."""
     rg, ru, rd = raw_matrix(fg, F, D, 91), raw_matrix(fg, F, D, 92), raw_matrix(fd, D, F, 93)
     wg, wu, wd = dev.matrix(fg, rg, F, D), dev.matrix(fg, ru, F, D), dev.matrix(fd, rd, D, F)
     x = dev.buf((np.random.default_rng(19).standard_normal((T, D)) * 0.5).astype(np.float32))
@@ -511,7 +535,7 @@ def test_atencion_output_planes_feed_wo(quipu, dev, hd, nh, nkv, T, pos0):
 
 
 def test_matmul_planes_rejections(quipu, dev):
-    """P[4] = 2 needs the 256-token tiles (under 256 tokens the matmul refuses it), and the planes' buffers must hold
+    """P[4] = 2 needs 256 tokens (under that the matmul refuses it), and the planes' buffers must hold
     4 * rows * K bytes (256-token rows)."""
     T, F, D = 300, 256, 256
     raw = raw_matrix(capi.Q4_K, F, D, 94)
@@ -581,7 +605,7 @@ def test_matmul_swiglu_fused_rejections(quipu, dev):
 
 @pytest.mark.parametrize("T,N,K", [(256, 300, 4096), (700, 130, 1024)])
 def test_matmul_q4k_prefill_row_magnitudes(quipu, dev, oracle, T, N, K):
-    """Q4_K prefill from 256 tokens on (the 256-token tiles, inputs as bf16 high + low planes): token rows of
+    """Q4_K prefill from 256 tokens on (inputs by way of their bf16 high + low parts): token rows of
     magnitude 1e-20 .. 1e20, an all-zero row and rows with one outlier 1e6 times the rest stay within the float32
     dot bound; the all-zero row gives exact zeros."""
     raw = raw_matrix(capi.Q4_K, N, K, 62)

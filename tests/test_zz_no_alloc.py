@@ -1,8 +1,8 @@
 """qp_dispatch_noalloc: the prefill matmul through the entry point that allocates nothing (its workspace is the
 library's fixed device scratch array) gives exactly qp_dispatch's results, on two calls in a row (the second with
-fewer tokens), with split-K and with the 256-token tiles; where qp_dispatch's split-K partials would not fit the
-scratch (the 8B model's 4096 x 14336 and 4096 x 4096 matmuls from 64 tokens on), it splits K fewer times and stays
-within the matmul's error bound of the float64 product (2e-5 sum |w x|); a call whose input planes alone would not
+fewer tokens), with split-K and in passes over the tokens; where qp_dispatch's split-K partials would not fit the
+scratch (the 8B model's 4096 x 14336 at 256 tokens), it splits K fewer times and stays
+within the matmul's error bound of the float64 product (2e-5 sum |w x|); a call whose rows as input planes would not
 fit fails with QP_E_ARG; and the calls can be captured in a HIP graph, whose replays (fresh inputs uploaded
 between them) match the eager calls: the plain matmul, the fused gate/up/SwiGLU matmul, and a matmul asked to
 reuse the previous call's input planes (P[4] = 1), which a capture must not take from eager state."""

@@ -27,8 +27,9 @@ extern "C" {
 #define QP_E_CAPTURE (-4)    /* call not allowed while a graph is being captured */
 
 /* ---------------------------------------------------------------- device (GPU.crear, gpu.js:1168-1193) */
-/* Opens `device`, creates the stream and loads the kernel code object (QP_KERNELS or quipu_kernels.hsaco
- * next to this library).  Replaces GPU.crear (web/js/gpu.js:1168-1182). */
+/* Opens `device`, creates the stream and loads the kernel code objects: quipu_kernels.hsaco next to this library or
+ * the file that QP_KERNELS names, and quipu_{small,attn,tile}.hsaco next to that file, or where it stands alone next to
+ * this library.  Replaces GPU.crear (web/js/gpu.js:1168-1182). */
 int qp_init(int device);
 /* JSON {"summary","arch","cus","hbm_bytes","max_buffer","bytes_used"} -- gpu.info (gpu.js:1186-1193). */
 int qp_info(char* json, size_t cap);

@@ -7,6 +7,7 @@
 #include "../../include/quipu.h"
 
 #include <dlfcn.h>
+#include <unistd.h>
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -1823,7 +1824,9 @@ int qp_init(int device) {
     const std::string dir = slash == std::string::npos ? std::string() : path.substr(0, slash + 1);
     hipModule_t mods[kObjects];
     for (int i = 0; i < kObjects; i++) {
-        const std::string p = i ? dir + kObjectNames[i] : path;
+        // the other objects beside the first where they are there (a whole other build), else beside this library
+        std::string p = i ? dir + kObjectNames[i] : path;
+        if (i && access(p.c_str(), R_OK)) p = self_dir() + "/" + kObjectNames[i];
         HIPCHK(hipModuleLoad(&mods[i], p.c_str()), ("hipModuleLoad " + p).c_str());
     }
     g_mod = mods[0];

@@ -7,6 +7,9 @@ rounding of a K-term sum in any order); the other float kernels to small relativ
 Every dispatch here uses buffers sized exactly as the kernel indexes them (shapes are checked by the op table
 on the host before any launch).
 """
+import os
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -70,6 +73,22 @@ def dev(quipu):
     d = Dev(quipu)
     yield d
     d.close()
+
+
+@pytest.mark.parametrize("others", [False, True])
+def test_kernels_from_another_file(tmp_path, others):
+    """QP_KERNELS names a lone quipu_kernels.hsaco (the other code objects then come from beside the library), or one with the
+    others beside it."""
+    import shutil
+    from conftest import ROOT, run
+    from quipullm_amd import build
+    for n in build.OBJECTS if others else build.OBJECTS[:1]:
+        shutil.copy(os.path.join(build.LIB, "quipu_%s.hsaco" % n), tmp_path)
+    code = "import numpy as np; from quipullm_amd import capi; q = capi.Quipu(0); h = q.buffer_from(np.zeros(4, np.uint32)); " \
+           "q.dispatch('fill_u32', [('u', 7), ('u', 4), ('u', 0)], [0, h]); q.sync(); print(q.download(h, (4,), np.uint32))"
+    rc, out, err = run([sys.executable, "-c", code],
+                       env={"QP_KERNELS": str(tmp_path / "quipu_kernels.hsaco"), "PYTHONPATH": ROOT})
+    assert rc == 0 and "[7 7 7 7]" in out, err
 
 
 def test_info(quipu):

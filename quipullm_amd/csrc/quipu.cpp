@@ -1290,7 +1290,8 @@ int op_matmul_eg(const Ctx& c, int fmt, const char* name) {
         q.k = K;
         q.acc = acc;
         q.rows = s.rows;
-        q.mt = s.nlst / 128 + E;  // the list's whole 128s and a tile more per expert
+        // the list's whole 128s (no more than an expert's tile for every token has) and a tile more per expert
+        q.mt = (s.nlst / 128 < E * a.tpe ? s.nlst / 128 : E * a.tpe) + E;
         q.nexp = E;
         q.kb = K / 256;
         q.tfijo = tfijo;

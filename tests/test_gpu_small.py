@@ -278,6 +278,42 @@ def test_grouped_matmul_in_large_buffers(quipu, dev, oracle, fmt, T, m):
         assert np.all(np.abs(got[j] - (xr.astype(np.float64) @ W[sel[j]].T)[0]) <= split_bound(W[sel[j]], xr)[0]), j
 
 
+def test_grouped_matmul_of_a_list_in_a_large_buffer(quipu, dev, oracle):
+    """A job list at the start of a 2 GiB buffer: the launch follows the jobs that the dispatch can have, not the room (20
+    million empty tiles took 5 ms; the call itself is below 0.1 ms)."""
+    import ctypes
+    fmt, E, N, K, k, T = capi.Q4_K, 3, 600, 256, 2, 100
+    rng = np.random.default_rng(94)
+    sel = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32).ravel()
+    raw = raw_matrix(fmt, E * N, K, 95)
+    W = weights(oracle, fmt, raw, E * N, K).reshape(E, N, K)
+    jobs = [np.flatnonzero(sel == e) for e in range(E)]
+    off = np.cumsum([0] + [len(j) for j in jobs]).astype(np.uint32)
+    lst = quipu.alloc(2 << 30)
+    dev.hs.append(lst)
+    quipu.upload(lst, np.concatenate(jobs).astype(np.uint32))
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    y = dev.zeros(4 * T * k * N)
+    b = [dev.paso(T, 0), dev.matrix(fmt, raw, E * N, K), dev.buf(x), y, lst, dev.buf(off)]
+    ev = [ctypes.c_uint64(), ctypes.c_uint64()]
+    for e in ev:
+        quipu.L.qp_event_create(ctypes.byref(e))
+    best = 1e9
+    for _ in range(3):
+        quipu.L.qp_event_record(ev[0])
+        quipu.dispatch("matmul_q4k_eg", [("u", N), ("u", K), ("u", 0), ("u", k), ("u", 1)], b, ((N + 63) // 64, E, (T + 31) // 32))
+        quipu.L.qp_event_record(ev[1])
+        ms = ctypes.c_float()
+        quipu.L.qp_event_elapsed(ev[0], ev[1], ctypes.byref(ms))
+        best = min(best, ms.value)
+    for e in ev:
+        quipu.L.qp_event_free(e)
+    got = dev.get(y, (T * k, N))
+    for j in range(T * k):
+        assert np.all(np.abs(got[j] - W[sel[j]] @ x[j // k].astype(np.float64)) <= bound(W[sel[j]], x[j // k][None])[0]), j
+    assert best < 2.0, best
+
+
 @pytest.mark.parametrize("f16", [0, 1])
 @pytest.mark.parametrize("hd,nh,nkv,T,pos0,swa,cap", [
     (128, 8, 8, 1, 0, 0, 0),          # one key

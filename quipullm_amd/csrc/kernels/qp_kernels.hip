@@ -4346,8 +4346,8 @@ QP_DEV uint2 topk_limit(const uint32_t (&o)[C], const uint32_t (&lo)[C], uint32_
 
 // Stage 1: workgroup g keeps the kp = k + 1 largest keys of logits [2048 g, 2048 g + 2048) (in no order, zeros after
 // them where there are fewer), plus a NaN flag.  part: kp keys per workgroup, then one u32 flag per workgroup.
-// Latency bound, like stage 2: the limit takes at most 16 counting steps of a barrier each where sorting the 2048 keys took 66
-// passes over LDS (128256 logits, k = 40: 7.2 us against 50.3, stage 2 11.9 against 38.5).
+// Latency bound, like stage 2: the limit takes at most 16 counting steps of a barrier each (17 more where equal values
+// straddle it) where sorting the 2048 keys took 66 passes over LDS (128256 logits, k = 40: 7.2 us against 50.3, stage 2 11.9 against 38.5).
 KERNEL __launch_bounds__(256) void qp_topk_part(QpCandArgs a) {
     __shared__ uint64_t cnt[33];
     __shared__ uint32_t fill;

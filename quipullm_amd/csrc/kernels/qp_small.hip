@@ -5,9 +5,16 @@
 // v_mfma_f32_16x16x32_f16 with the integers as f16 (exact) and X as f16 high + low parts of the row scaled by a power
 // of two per 256 inputs (22 bits): two matrix instructions per pair, and the block's scale multiplies the f32 sum of a
 // whole block.  K-quants with 6-bit (or smaller) sub-block scales take scale * quant as the integer (at most 1953, so
-// exact in f16) and one f32 scale per 256 inputs; Q6_K's int8 scale * quant reaches 4096, so its integers are a high
+// exact in f16) and one f32 scale per 256 inputs; Q6_K's int8 scale * quant reaches 8064, so its integers are a high
 // and a low f16 (three instructions); Q8_0 and IQ4_NL scale the sums of each 32 inputs; f32 rows are scaled by a power
-// of two per 32 inputs and split like X.
+// of two per 32 inputs and split like X (the product of the two low parts is left out).
+//
+// So X (and f32 weights) have 22 bits below the largest of their 256 (32) inputs, not f32's own: an input 2^11 and more
+// below that loses bits against the f32 multiply-adds that ran here before.  What an output is off by is mostly its sums'
+// rounding, and the matrix cores add in fewer steps: distance from 64 bits (2-norm, N(0, 1) inputs, 2 / 32 / 63 tokens, in
+// parentheses the kernels before: f32 multiply-adds below 64 dispatched tokens, then bf16 parts) f32 128 x 2048 1.6e-7 /
+// 1.4e-7 / 1.4e-7 (9e-7 / 8e-7 / 4.5e-6), Q4_K 512 x 4096 3.2e-7 (1.1e-6 / 1.2e-6 / 4.2e-6), Q6_K 3.6e-7 (1.2e-6 / 1.1e-6 /
+// 4.3e-6), Q8_0 512 x 1024 1.0e-7 (6e-7 / 6e-7 / 4.0e-6), IQ4_NL 1.0e-7 (5e-7 / 6e-7 / 4.3e-6).
 //
 // A wavefront takes 16 R weight rows and a slice of K and keeps them in registers, so nothing is staged in LDS: the
 // lanes of row n (n = lane % 16) load 16-byte chunks of four consecutive blocks (64 contiguous bytes), and a 4 x 4

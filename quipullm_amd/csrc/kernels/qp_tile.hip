@@ -8,10 +8,13 @@
 // sums are scaled by the block's f32 scale and the row's, less the minima times X's sums of 16 inputs (two instructions
 // per 32 x 32).  64 KB of LDS (80 KB for Q6_K): two workgroups per CU, whose barriers overlap.
 //
-// Bound by the matrix cores at their power limit: every weight takes two instructions' worth of products (X's two halves;
-// Q6_K three), and dense f16 products of random data reach about 1.2 PFLOP/s on this card in the library and 1.6 in a bare
-// loop.  Q4_K 14336 x 4096 at 2048 tokens: 597 us (0.81 PFLOP/s of f16 products; with bf16 planes of both sides, three
-// products, in 256 x 256 tiles 720 us), 524 us with the staging left out.  Instructions of 16 x 16 x 32: 640 us.
+// Bound by no unit alone: every weight takes two instructions' worth of products (X's two halves; Q6_K three), and in Q4_K
+// 14336 x 4096 at 2048 tokens the matrix cores are busy 49 % of the cycles and LDS 50 %, of which a quarter is bank conflicts,
+// at a clock that the load has brought to 1.9 GHz, and the wavefronts wait 26 % of theirs; Q6_K 4096 x 14336 50 / 44 / 29 % at
+// 1.7 GHz, at 256 tokens (7 blocks per K split, the inputs from farther away) 30 / 26 / 38 % at 2.2.
+// Measured in us, in parentheses 256-token tiles of bf16 planes of both sides (three products): Q4_K 14336 x 4096 at 2048 tokens
+// 519 with the input's split (629), 0.93 PFLOP/s of f16 products, where the library's dense f16 product reaches 1.15 to 1.2; Q6_K
+// 4096 x 14336 770 (781).  With the staging left out 0.88 of the time; with instructions of 16 x 16 x 32 1.07 of it.
 #include "qp_ints.h"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));

@@ -976,9 +976,10 @@ int op_atencion(const Ctx& c) {
         return launch((two ? km2 : km)[a.hd == 128][gi], a.nkv, cdiv(c.gy ? c.gy : 1, (two ? 1 : 4) * tpw), 1, 256, 0,
                       a);
     }
-    // f32 caches, windows and rings: matrix cores at f32 accuracy (qp_attn.hip), 16 or 32 (query, head) rows per
-    // workgroup, the keys shared out (grid z) while the rows alone give fewer than one workgroup per CU and every share
-    // keeps 128 keys.  A ring without a window, or a cache whose offsets pass 31 bits, stays with the general kernel.
+    // f32 caches, windows and rings: matrix cores (qp_attn.hip), 16 or 32 (query, head) rows per workgroup, the keys shared
+    // out (grid z) while the rows alone give fewer than one workgroup per CU and every share keeps 128 slots of the cache or
+    // window (the host does not know how many hold keys: early in a large cache the later shares have none).  A ring without a
+    // window, or a cache whose offsets pass 31 bits, stays with the general kernel.
     const uint32_t T = c.gy ? c.gy : 1, nrow = T * G, RG = nrow > 16 ? 2 : 1, yb = cdiv(nrow, 16 * RG);
     if ((!a.cap || a.swa) && 4ull * a.nkv * a.hd * ((a.rows + 31) / 32 * 32) < (1ull << 31) && !getenv_flag("QP_NO_MFMA")) {
         const uint32_t cus = g_cus > 0 ? (uint32_t)g_cus : 1u;

@@ -373,7 +373,7 @@ def test_attention_any_cache(quipu, dev, hd, nh, nkv, T, pos0, swa, cap, f16):
 @pytest.mark.parametrize("hd,nh,nkv,T,pos0,swa,cap", [(128, 8, 4, 24, 40, 0, 0),   # two blocks of 32 rows, f32 or window
                                                       (64, 4, 4, 9, 300, 40, 64),   # a block of 16 rows, a ring
                                                       (128, 6, 2, 1, 700, 600, 0)])  # one token, keys shared out
-@pytest.mark.parametrize("kind", ["k_infinite", "k_minus_infinite", "k_huge", "v_huge", "v_without_weight", "q_spread"])
+@pytest.mark.parametrize("kind", ["k_infinite", "k_minus_infinite", "k_huge", "v_huge", "v_without_weight", "q_spread", "blocks"])
 def test_attention_unlike_magnitudes(quipu, dev, hd, nh, nkv, T, pos0, swa, cap, f16, kind):
     """Keys and values far larger than the others, infinities among them: a row that does not see such a key, or gives it
     no weight, has the result that it would have without it.
@@ -402,6 +402,9 @@ def test_attention_unlike_magnitudes(quipu, dev, hd, nh, nkv, T, pos0, swa, cap,
         vf[pos0 - 3] = big
         kf[pos0 - 3] = 0
         kf[pos0 - 3, 0::hd] = -3000
+    elif kind == "blocks":  # magnitudes that change forth and back along the keys
+        kf[::37] *= np.float32(1e-6)
+        vf[n // 2:n // 2 + 200] *= np.float32(1e-4 if f16 else 1e-7)
     else:
         q[T // 2:, :, 3] *= np.float32(2.0 ** 30)
         kf[:, 3::hd] = 0
